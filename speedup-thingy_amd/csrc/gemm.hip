@@ -16,7 +16,8 @@
 // register r of lane l holds row 8*(r/4) + 4*(l/32) + (r%4), column l % 32.
 // Any consistent k permutation gives the same dot products, so only the output
 // mapping has to match the hardware; the GPU parity tests pin it.
-#include "gemm.hpp"
+#include "gemm_dev.hpp"
+#include "gemm_tile.hpp"
 
 #include <stdio.h>
 #include <stdlib.h>
@@ -30,24 +31,6 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kMaxSplits = 32;                      // split-K partials per output tile
 constexpr size_t kMaxSplitBytes = (size_t)64 << 20;  // split-K workspace ceiling
-
-__device__ __forceinline__ int64_t ilv_row(int64_t r, int32_t half) {
-  return ((r & 63) < 32 ? 0 : half) + (r >> 6) * 32 + (r & 31);
-}
-
-__device__ __forceinline__ int log2i(int v) { return 31 - __clz(v); }
-
-__device__ __forceinline__ int64_t row_off(const Operand& o, int64_t r) {
-  if (o.ilv) r = ilv_row(r, o.ilv);
-  if (o.rows) r = o.rows[r];
-  if (o.rdiv) return (r >> log2i(o.rdiv)) * o.rs_hi + (r & (o.rdiv - 1)) * o.ld;
-  return r * o.ld;
-}
-
-__device__ __forceinline__ int64_t col_off(const Operand& o, int c) {
-  if (o.cdiv) return (int64_t)(c >> log2i(o.cdiv)) * o.cs_hi + (c & (o.cdiv - 1));
-  return c;
-}
 
 // ------------------------------------------------------------------ loaders
 
@@ -191,75 +174,6 @@ struct Loader<R, BK, true> {
   __device__ __forceinline__ void store(bf16* lds, int tid) const { l.template store<S>(lds, tid); }
 };
 
-// ------------------------------------------------------------------ output chunks
-
-// Writes W consecutive outputs (row m of the tile space, columns n..n+W-1) applying
-// alpha, row_scale, output-row mapping, residual and beta.  vec: 16-byte path allowed.
-template <int W>
-__device__ __forceinline__ void store_chunk(const Epilogue& e, int g, int m, int n, int N, float* v, bool vec) {
-  const float rs = e.row_scale ? e.row_scale[m] : 1.0f;
-  int64_t orow = m + (int64_t)g * e.c_growstride;
-  if (e.c_ilv) orow = ilv_row(orow, e.c_ilv);
-  if (e.c_rows) orow = e.c_rows[orow];
-  const int nv = N - n < W ? N - n : W;
-#pragma unroll
-  for (int t = 0; t < W; ++t) v[t] *= e.alpha * rs;
-  if (e.resid) {
-    const float* rp = e.resid + orow * e.ld_resid + n;
-    if (vec && nv == W) {
-#pragma unroll
-      for (int t = 0; t < W; t += 4) {
-        const float4 x = *reinterpret_cast<const float4*>(rp + t);
-        v[t] += x.x; v[t + 1] += x.y; v[t + 2] += x.z; v[t + 3] += x.w;
-      }
-    } else {
-      for (int t = 0; t < nv; ++t) v[t] += rp[t];
-    }
-  }
-  // W-column chunks start at multiples of W and never cross a 32-column run of the interleave
-  const int64_t ocol = e.c_col_ilv ? ilv_row((int64_t)g * e.c_gstride + n, e.c_col_ilv) : (int64_t)g * e.c_gstride + n;
-  if (e.c_f32) {
-    float* cp = reinterpret_cast<float*>(e.c) + orow * e.ldc + ocol;
-    if (vec && nv == W) {
-#pragma unroll
-      for (int t = 0; t < W; t += 4) {
-        if (e.beta != 0.0f) {
-          const float4 o = *reinterpret_cast<const float4*>(cp + t);
-          v[t] += e.beta * o.x; v[t + 1] += e.beta * o.y; v[t + 2] += e.beta * o.z; v[t + 3] += e.beta * o.w;
-        }
-        *reinterpret_cast<float4*>(cp + t) = make_float4(v[t], v[t + 1], v[t + 2], v[t + 3]);
-      }
-    } else {
-      for (int t = 0; t < nv; ++t) cp[t] = v[t] + (e.beta != 0.0f ? e.beta * cp[t] : 0.0f);
-    }
-  } else {
-    bf16* cp = reinterpret_cast<bf16*>(e.c) + orow * e.ldc + ocol;
-    if (vec && nv == W && W == 8) {
-      if (e.beta != 0.0f) {
-        const uint4 o = *reinterpret_cast<const uint4*>(cp);
-        const uint32_t ow[4] = {o.x, o.y, o.z, o.w};
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          v[2 * t] += e.beta * __uint_as_float(ow[t] << 16);
-          v[2 * t + 1] += e.beta * __uint_as_float(ow[t] & 0xffff0000u);
-        }
-      }
-      uint4 o;
-      o.x = pack_bf2(v[0], v[1]);
-      o.y = pack_bf2(v[2], v[3]);
-      o.z = pack_bf2(v[4], v[5]);
-      o.w = pack_bf2(v[6], v[7]);
-      *reinterpret_cast<uint4*>(cp) = o;
-    } else {
-      for (int t = 0; t < nv; ++t) cp[t] = f2bf(v[t] + (e.beta != 0.0f ? e.beta * bf2f(cp[t]) : 0.0f));
-    }
-  }
-}
-
-struct EpiFlags {
-  int vec;  // 16-byte stores / residual loads are aligned
-};
-
 // ------------------------------------------------------------------ kernel
 
 // Tiles larger than 128x128 keep one workgroup per CU (their LDS and accumulators fill it).
@@ -280,48 +194,6 @@ constexpr int wg_per_cu() {
     return n < 1 ? 1 : (n > 4 ? 4 : n);
   }
   return BM * BN > 128 * 128 ? 1 : 2;
-}
-
-// Direct-to-LDS stage layout: a tile row holds BK k values = CPR chunks of 16 bytes, chunk c
-// stored at position c ^ swz(row), so that 32 lanes reading the same logical chunk of 32
-// consecutive rows (the MFMA operand reads) spread over all LDS banks.  Both swizzles were
-// chosen by measurement (SQ_LDS_BANK_CONFLICT of ds_read_b128 patterns on gfx950: zero
-// conflicts for these two, conflicts for the unswizzled rows and for (row & 7), (row >> 1) & 3).
-template <int CPR>
-__device__ __forceinline__ int dl_swz(int row) {
-  if constexpr (CPR == 8) return (row ^ (row >> 3)) & 7;  // 128-byte rows
-  else return (row >> 2) & 3;                             // 64-byte rows
-}
-
-// 16 bytes per lane from global memory straight into LDS at (LDS base + 16 * lane); the LDS
-// base must be wave-uniform.  The host pass of the compiler has no such builtin and never
-// runs kernel bodies, so it only sees the declaration.
-__device__ __forceinline__ void lds_dma16(const void* src, void* lds_base) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  __builtin_amdgcn_global_load_lds(src, lds_base, 16, 0, 0);
-#else
-  (void)src;
-  (void)lds_base;
-#endif
-}
-
-// Four bf16 of a k-major LDS tile, transposed across the 16 lanes of each lane group
-// (ds_read_b64_tr_b16, gfx950).  Measured lane layout: within a group of 16 lanes, lane i
-// receives element (i % 4) of the 8-byte rows that lanes 4j + i / 4 (j = 0..3) point at, in j
-// order.  So if lane s of the group points at k-row (kb + s / 4) and columns (cb + 4 (s % 4))..+3,
-// lane i gets column cb + i at k-rows kb..kb + 3: an MFMA operand fragment.
-typedef short short4_v __attribute__((ext_vector_type(4)));
-
-// 16 zero bytes in global memory: the source of direct loads past the end of a k range (a
-// layout-T tile's rows beyond the group of a grouped-K problem), so LDS gets exact zeros.
-__device__ __align__(16) unsigned int kDlZero[4] = {0u, 0u, 0u, 0u};  // never written
-__device__ __forceinline__ short4_v lds_read_tr4(const unsigned char* lds_byte_ptr) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_v*)lds_byte_ptr);
-#else
-  (void)lds_byte_ptr;
-  return short4_v{0, 0, 0, 0};
-#endif
 }
 
 // One operand of the direct-to-LDS main loop: R tile rows (the output index i) by BK k per
@@ -407,13 +279,6 @@ struct DlOperand {
     }
   }
 };
-
-// s_waitcnt with vmcnt <= n and the other counters unconstrained (gfx9 encoding).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
 
 template <int BM, int BN, int BK, int WM, int WN, bool AT, bool BT, int EPI, bool DUALA = false, int DLS = 0>
 __global__ void __launch_bounds__(256, (wg_per_cu<BM, BN, BK, DLS, WM>())) gemm_kernel(GemmArgs p, EpiFlags fl) {
@@ -1152,16 +1017,6 @@ int launch_layouts(const GemmArgs& p, hipStream_t stream, void* ws, size_t ws_by
 // next block's B fragments are loaded before the current block is stored.
 constexpr int kSkPitch = 36;  // floats per patch row (144 bytes: 16-byte aligned rows)
 
-__device__ __forceinline__ bf16x8_v ld_frag16(const bf16* p) {
-  return __builtin_bit_cast(bf16x8_v, *reinterpret_cast<const uint4*>(p));
-}
-
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 template <int KS>
 __global__ void __launch_bounds__(256) gemm_sk_kernel(GemmArgs p, EpiFlags fl, int nch, int cpt) {
   __shared__ __align__(16) float patch[4][32 * kSkPitch];
@@ -1284,35 +1139,16 @@ int launch_sk(const GemmArgs& p, hipStream_t stream, int vec) {
   return check_launch("gemm_short_k");
 }
 
-// Direct-to-LDS mainloop selection.  Default: K <= 1024 -> BK 32, 2 stages (four workgroups
-// per CU: short reductions are latency-bound, occupancy hides it best); longer K -> BK 64,
-// 2 stages (fewer barriers per MFMA).  RTE_GEMM_DL overrides it for diagnostics: 0 keeps the
-// register-staged loop everywhere; otherwise 128x128 tiles with (BK, stages) = 2: (64, 2),
-// 3: (64, 3), 5: (32, 4), 6: (32, 3), 7: (32, 2); 4 = 256x128 tiles, (64, 2).
-int dl_env() {
-  static int mode = [] {
-    const char* v = getenv("RTE_GEMM_DL");
-    if (!v || !*v) return -1;
-    const int m = atoi(v);
-    return (m == 0 || (m >= 2 && m <= 7)) ? m : -1;
-  }();
-  return mode;
-}
-
-int dl_mode(const GemmArgs& p) {
-  const int env = dl_env();
-  if (env >= 0) return env;
-  const int klen = p.splits > 1 ? p.k_chunk : p.K;
-  return klen <= 1024 ? 7 : 2;
-}
+// Direct-to-LDS mainloop selection: K <= 1024 -> BK 32, 2 stages (four workgroups per CU: short
+// reductions are latency-bound, occupancy hides it best); longer K -> BK 64, 2 stages (fewer
+// barriers per MFMA).
+int dl_bk(const GemmArgs& p) { return (p.splits > 1 ? p.k_chunk : p.K) <= 1024 ? 32 : 64; }
 
 bool dl_ok(const GemmArgs& p) {
-  const int mode = dl_mode(p);
-  if (mode == 0 || p.a_koff2 || p.K <= 0) return false;
-  const int bk = mode >= 5 ? 32 : 64;
+  if (p.a_koff2 || p.K <= 0) return false;
   // dense / grouped-M: whole stages over K; grouped-K (both operands layout T): any group sizes
   if (p.mode == MODE_GROUP_K) return p.a_t && p.b_t;
-  return p.K % bk == 0;
+  return p.K % dl_bk(p) == 0;
 }
 
 template <int BM, int BK, int DLS, int EPI>
@@ -1350,20 +1186,45 @@ int launch_dl_narrow(const GemmArgs& p, hipStream_t stream, void* ws, size_t ws_
 
 template <int EPI>
 int launch_dl(const GemmArgs& p, hipStream_t stream, void* ws, size_t ws_bytes, int vec) {
-  const bool nn = !p.a_t && !p.b_t;
-  switch (nn ? dl_mode(p) : (dl_mode(p) >= 5 ? 7 : 2)) {  // layout T: the two default shapes
-    case 3: return launch_cfg<128, 128, 64, 2, 2, false, false, EPI, false, 3>(p, stream, ws, ws_bytes, vec);
-    case 4: return launch_cfg<256, 128, 64, 2, 2, false, false, EPI, false, 2>(p, stream, ws, ws_bytes, vec);
-    case 5: return launch_cfg<128, 128, 32, 2, 2, false, false, EPI, false, 4>(p, stream, ws, ws_bytes, vec);
-    case 6: return launch_cfg<128, 128, 32, 2, 2, false, false, EPI, false, 3>(p, stream, ws, ws_bytes, vec);
-    case 7: return launch_dl_shape<32, 2, EPI>(p, stream, ws, ws_bytes, vec);
-    default: return launch_dl_shape<64, 2, EPI>(p, stream, ws, ws_bytes, vec);
-  }
+  return dl_bk(p) == 32 ? launch_dl_shape<32, 2, EPI>(p, stream, ws, ws_bytes, vec)
+                        : launch_dl_shape<64, 2, EPI>(p, stream, ws, ws_bytes, vec);
 }
 
 // The SwiGLU epilogue kernels' direct-load loop: whole 64-k stages of layout-N A.
 bool dl_whole64(const GemmArgs& p) {
-  return dl_mode(p) != 0 && !p.a_koff2 && !p.a_t && p.mode != MODE_GROUP_K && p.K > 0 && p.K % 64 == 0;
+  return !p.a_koff2 && !p.a_t && p.mode != MODE_GROUP_K && p.K > 0 && p.K % 64 == 0;
+}
+
+// Operands the tile kernels address: row offsets affine in k (the SwiGLU interleave is affine per
+// 64 k), unsplit columns, no gather, and 32-bit byte offsets.  rows x cols: memory rows and columns.
+// Returns the operand's extent in bytes, 0 if the kernels do not take it.
+uint32_t tile_operand(const Operand& o, int64_t rows, int64_t cols) {
+  if (o.cdiv || o.rows || o.rdiv || rows <= 0 || cols <= 0) return 0;
+  if (o.ilv && (rows % 64 != 0 || rows != 2 * (int64_t)o.ilv)) return 0;
+  const int64_t bytes = ((rows - 1) * o.ld + cols) * 2;
+  return bytes < ((int64_t)1 << 31) ? (uint32_t)bytes : 0;
+}
+
+bool tile_ok(GemmArgs& p, int epi_kind) {
+  if (p.mode != MODE_DENSE || p.a_koff2 || p.K < kTileMinK || (p.a_t && !p.b_t) || p.splits_forced) return false;
+  // narrow outputs and few rows over a long reduction: the narrow tiles below, split further
+  if (p.N <= 64 || (epi_kind == EPI_STORE && p.M <= 64 && (p.a_t || p.K > kTileRowK))) return false;
+  if (!(p.a_t && p.b_t) && p.K % 64 != 0) return false;
+  if (epi_kind == EPI_SWIGLU_BWD && p.epi.dw_row) return false;
+  p.a_bytes = p.a_t ? tile_operand(p.a, p.K, p.M) : tile_operand(p.a, p.M, p.K);
+  p.b_bytes = p.b_t ? tile_operand(p.b, p.K, p.N) : tile_operand(p.b, p.N, p.K);
+  return p.a_bytes && p.b_bytes;
+}
+
+// The tile kernels, and the sum of the partials where they split the reduction.
+int launch_tiles(const GemmArgs& p, int epi_kind, hipStream_t stream, int vec, void* ws, size_t ws_bytes) {
+  GemmArgs q = p;
+  RTE_TRY(gemm_tile_launch(q, epi_kind, stream, vec, ws, ws_bytes, &q.splits));
+  if (q.splits <= 1) return 0;
+  q.splitk_ws = static_cast<float*>(ws);
+  const int64_t n = (int64_t)p.M * ((p.N + 3) / 4);
+  hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, q, EpiFlags{vec});
+  return check_launch("gemm_splitk_reduce");
 }
 
 bool pow2_or_zero(int v) { return v == 0 || (v > 0 && (v & (v - 1)) == 0); }
@@ -1427,8 +1288,11 @@ int gemm_launch(const GemmArgs& p, int epi_kind, hipStream_t stream, void* ws, s
                 "gemm: QKV outputs must be 16-byte aligned with head_dim %% 8 == 0");
   }
 
+  GemmArgs q = p;
+  const bool tiles = tile_ok(q, epi_kind);
   switch (epi_kind) {
     case EPI_STORE: {
+      if (tiles) return launch_tiles(q, epi_kind, stream, vec, ws, ws_bytes);
       // short reductions over k-contiguous operands: output-bound, the barrier-free wave kernel
       if (p.K <= 32 && !p.a_t && !p.b_t && p.mode != MODE_GROUP_K)
         return launch_sk(p, stream, vec);
@@ -1458,6 +1322,7 @@ int gemm_launch(const GemmArgs& p, int epi_kind, hipStream_t stream, void* ws, s
         RTE_REQUIRE(p.mode == MODE_DENSE && p.N % 128 == 0, "gemm: dual-A SwiGLU needs dense mode and N %% 128 == 0");
         return launch_cfg<128, 128, 32, 2, 2, false, false, EPI_SWIGLU_FWD, true>(p, stream, ws, ws_bytes, 1);
       }
+      if (tiles) return launch_tiles(q, epi_kind, stream, 1, nullptr, 0);
       if (dl_whole64(p)) {
         if (p.N == 64)
           return launch_cfg<128, 64, 64, 4, 1, false, false, EPI_SWIGLU_FWD, false, 2>(p, stream, ws, ws_bytes, 1);
@@ -1470,6 +1335,7 @@ int gemm_launch(const GemmArgs& p, int epi_kind, hipStream_t stream, void* ws, s
       RTE_REQUIRE(p.epi.ug && p.epi.ug_in, "gemm: SwiGLU backward needs UG input and dUG output");
       RTE_REQUIRE(p.N % 32 == 0, "gemm: SwiGLU backward needs N %% 32 == 0");
       if (p.epi.dw_row) RTE_REQUIRE(p.N <= 128, "gemm: per-row reduction supports N <= 128");
+      if (tiles) return launch_tiles(q, epi_kind, stream, 1, nullptr, 0);
       if (dl_whole64(p)) {
         if (p.N <= 32)
           return p.b_t ? launch_cfg<128, 32, 64, 4, 1, false, true, EPI_SWIGLU_BWD, false, 2>(p, stream, ws, ws_bytes, 1)
@@ -1492,7 +1358,7 @@ int gemm_launch(const GemmArgs& p, int epi_kind, hipStream_t stream, void* ws, s
       RTE_REQUIRE(!p.a_t && !p.b_t, "gemm: QKV epilogue expects layout-N operands");
       RTE_REQUIRE(p.epi.q && p.epi.k && p.epi.v && p.epi.cos_t && p.epi.sin_t, "gemm: QKV outputs");
       RTE_REQUIRE(p.epi.hd % 2 == 0 && p.epi.dmodel * 3 == p.N, "gemm: QKV shape");
-      if (ws && p.mode == MODE_DENSE && p.K >= 256 && p.N % 4 == 0 &&
+      if (ws && p.mode == MODE_DENSE && p.K >= 256 && p.N % 4 == 0 && !(tiles && p.K <= kTileRowK) &&
           (int64_t)((p.M + 31) / 32) * ((p.N + 127) / 128) < 256 &&
           ws_bytes >= (size_t)2 * p.M * p.N * sizeof(float)) {
         // few output tiles (a short sequence batch): split the reduction, the split-K reduce
@@ -1503,6 +1369,7 @@ int gemm_launch(const GemmArgs& p, int epi_kind, hipStream_t stream, void* ws, s
         ps.splits_forced = 1;
         return gemm_launch(ps, EPI_STORE, stream, ws, ws_bytes);
       }
+      if (tiles) return launch_tiles(q, epi_kind, stream, 1, nullptr, 0);
       if (dl_ok(p)) return launch_dl<EPI_ROPE_QKV>(p, stream, ws, ws_bytes, 1);
       return launch_cfg<128, 128, 64, 2, 2, false, false, EPI_ROPE_QKV>(p, stream, ws, ws_bytes, 1);
     default:

@@ -99,6 +99,8 @@ struct GemmArgs {
   int gk_chunk = 0;
   const int32_t* gk_first = nullptr;  // [G + 1]
   float* gk_part = nullptr;
+  // bytes from each operand's first element past its last one (the tile kernels' buffer bounds)
+  uint32_t a_bytes = 0, b_bytes = 0;
   Epilogue epi;
 };
 

@@ -1,0 +1,503 @@
+// Dense bf16 MFMA GEMM with a register-pipelined main loop (gfx950), fp32 accumulation.
+//
+// One workgroup owns a BM x BN output tile; each of its WM x WN waves holds a (BM / WM) x
+// (BN / WN) block in v_mfma_f32_32x32x16_bf16 accumulators.  K advances in tiles of BK through ST
+// LDS stages filled by global_load_lds_dwordx4 (no registers), and the MFMA operands of the next
+// 16-k step are read from LDS while the current step's products run, across tile boundaries too:
+//
+//   step (kt, last): wait until tile kt + 1 has landed; barrier; refill tile kt's stage with tile
+//                    kt + ST; read the operands of (kt + 1, 0); products of (kt, last)
+//
+// so a barrier is passed with a whole step's products still to issue, and a load has ST - 1 tiles
+// of products to arrive.
+#include "gemm_dev.hpp"
+#include "gemm_tile.hpp"
+
+#include <type_traits>
+
+namespace rte {
+
+namespace {
+
+// One operand: R tile rows (the output index) by BK k per stage.  Layout N (k contiguous): LDS
+// rows are output rows of BK k, 16-byte chunk c at c ^ dl_swz(row).  Layout T (output index
+// contiguous): LDS rows are k rows of R elements, chunk c at c ^ 4 (k % 4), so the four k rows of
+// a ds_read_b64_tr_b16 sit in distinct 64-byte windows.
+template <int R, int NT, int BK, bool T>
+struct TileOperand {
+  static constexpr int ROWB = T ? R * 2 : BK * 2;
+  static constexpr int CPR = ROWB / 16;
+  static constexpr int BYTES = R * BK * 2;
+  static constexpr int INS = BYTES / 16 / NT;
+  static_assert(INS >= 1 && BYTES == INS * 16 * NT, "whole 16-byte loads per thread");
+  static_assert(!T || CPR >= 16, "layout-T tiles hold at least 128 columns");
+
+  uint32_t off[INS];  // byte offset of this thread's loads in the operand (under 2^31: host check)
+
+  __device__ __forceinline__ void init(const Operand& o, int i0, int ilim, int tid) {
+#pragma unroll
+    for (int u = 0; u < INS; ++u) {
+      const int q = u * NT + tid, row = q / CPR, pc = q % CPR;
+      if constexpr (!T) {
+        int i = i0 + row;
+        if (i >= ilim) i = ilim - 1;  // rows past the end re-read the last one; never stored
+        off[u] = (uint32_t)(row_off(o, i) + (pc ^ dl_swz<CPR>(row)) * 8) * 2;
+      } else {
+        int i = i0 + (pc ^ ((row & 3) * 4)) * 8;
+        if (i + 8 > ilim) i = ilim - 8;  // layout-T extents are multiples of 8
+        const int64_t krow = (o.ilv && row >= 32) ? (int64_t)(row - 32) + o.ilv : row;
+        off[u] = (uint32_t)(krow * o.ld + i) * 2;
+      }
+    }
+  }
+  // byte offset of the tile starting at k0 (a multiple of BK past a multiple of 64)
+  __device__ __forceinline__ static int advance(int ld, int ilv, int k0) {
+    if constexpr (!T) return k0 * 2;
+    return (ilv ? (k0 >> 6) * 32 + ((k0 >> 5) & 1) * ilv : k0) * ld * 2;
+  }
+  // LDS byte offset of this lane's part of 32-row block b at k-step ks
+  __device__ __forceinline__ static int frag_off(int rb, int lane, int b, int ks) {
+    if constexpr (!T) {
+      const int r = rb + 32 * b + (lane & 31);
+      return r * ROWB + (((ks * 2 + (lane >> 5)) ^ dl_swz<CPR>(r)) << 4);
+    } else {
+      const int g = lane >> 4, s = lane & 15;
+      const int kr = 8 * (g >> 1) + (s >> 2);
+      const int col = rb + 32 * b + 16 * (g & 1) + 4 * (s & 3);
+      return (kr + 16 * ks) * ROWB + (((col >> 3) ^ ((s >> 2) * 4)) << 4) + (col & 7) * 2;
+    }
+  }
+  __device__ __forceinline__ static bf16x8_v frag(const unsigned char* at) {
+    if constexpr (!T) {
+      return *reinterpret_cast<const bf16x8_v*>(at);
+    } else {
+      const short4_v lo = lds_read_tr4(at);
+      const short4_v hi = lds_read_tr4(at + 4 * ROWB);
+      typedef short short8_v __attribute__((ext_vector_type(8)));
+      return __builtin_bit_cast(bf16x8_v, (short8_v)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    }
+  }
+};
+
+constexpr int kBand = 4;  // tile rows walked together (4, 8 and 16 are within 2% but for long-k layout T: 413, 427, 504 us)
+constexpr int kPatchPitch = 68;  // floats per row of a wave's 32 x 64 output patch
+constexpr int kPatchBytes = 32 * kPatchPitch * 4;
+
+template <int BM, int BN, int WM, int WN, int BK, int ST>
+constexpr int tile_wgs() {
+  constexpr int by_lds = 163840 / (ST * (BM + BN) * BK * 2);
+  constexpr int by_regs = ((BM / WM) * (BN / WN) >= 128 * 128 ? 4 : (BM / WM) * (BN / WN) >= 128 * 64 ? 8 : 16) / (WM * WN);
+  return by_lds < by_regs ? by_lds : by_regs;
+}
+
+template <int BM, int BN, int WM, int WN, int BK, int ST, bool AT, bool BT, int EPI>
+__global__ void __launch_bounds__(WM* WN * 64, (tile_wgs<BM, BN, WM, WN, BK, ST>() * WM * WN / 4))
+    gemm_tile_kernel(GemmArgs p, int vec) {
+  constexpr int NT = WM * WN * 64;
+  constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32, KS = BK / 16;
+  static_assert(TN % 2 == 0, "output patches are 64 columns");
+  static_assert(ST >= 2 && ST <= 4 && KS % 2 == 0, "stages and k-steps");
+  using OpA = TileOperand<BM, NT, BK, AT>;
+  using OpB = TileOperand<BN, NT, BK, BT>;
+  constexpr int INS = OpA::INS + OpB::INS;
+  constexpr int A_BYTES = OpA::BYTES, STAGE = OpA::BYTES + OpB::BYTES;
+  constexpr int PPS = STAGE / kPatchBytes;  // output patches per stage
+  static_assert(PPS * ST >= WM * WN, "the stages hold every wave's output patch");
+
+  // One LDS array per stage, each addressed by name: the compiler then knows that the operand
+  // reads of one stage do not touch the stages being filled and waits for no load it need not
+  // (from one array, a ds_read_b64_tr_b16 waits for every load in flight).
+  __shared__ __align__(16) unsigned char st0[STAGE], st1[STAGE], st2[ST > 2 ? STAGE : 16], st3[ST > 3 ? STAGE : 16];
+  auto stage_of = [&](auto s) -> unsigned char* {
+    constexpr int S = decltype(s)::value % ST;
+    if constexpr (S == 0) return st0;
+    else if constexpr (S == 1) return st1;
+    else if constexpr (S == 2) return st2;
+    else return st3;
+  };
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+
+  // Tile order: dispatch id d runs on XCD d % 8, so each XCD takes a contiguous run of tiles, and
+  // a run walks kBand tile rows column by column: the tiles an XCD works on at one time share
+  // few A and B panels of its L2.
+  const int gx = (p.M + BM - 1) / BM, gy = (p.N + BN - 1) / BN, total = gx * gy;
+  int lin = blockIdx.x;
+  {
+    const int q = total >> 3, r = total & 7, xcd = lin & 7;
+    lin = xcd * q + (xcd < r ? xcd : r) + (lin >> 3);
+  }
+  const int bw = kBand * gy, bi = lin / bw;
+  const int rows = gx - bi * kBand < kBand ? gx - bi * kBand : kBand;
+  const int m0 = (bi * kBand + (lin - bi * bw) % rows) * BM, n0 = ((lin - bi * bw) / rows) * BN;
+  int kbeg = 0, kend = p.K;
+  float* partial = nullptr;
+  if (p.splits > 1) {
+    kbeg = blockIdx.y * p.k_chunk;
+    kend = kbeg + p.k_chunk < p.K ? kbeg + p.k_chunk : p.K;
+    partial = p.splitk_ws + (int64_t)blockIdx.y * p.M * p.N;
+  }
+
+  f32x16_v acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+  OpA la;
+  OpB lb;
+  la.init(p.a, m0, p.M, tid);
+  lb.init(p.b, n0, p.N, tid);
+  const int alda = (int)p.a.ld, blda = (int)p.b.ld, ailv = p.a.ilv, bilv = p.b.ilv;
+  const BufferRsrc ra = buffer_rsrc(p.a.ptr, p.a_bytes), rb = buffer_rsrc(p.b.ptr, p.b_bytes);
+
+  // A ragged reduction (both operands layout T) reads k rows past its end in its last tile: they lie
+  // past the operands' buffer bounds, which the hardware turns into zeros.
+  auto issue = [&](unsigned char* st, int kt) {
+    const int k0 = kbeg + kt * BK;
+    const int ao = OpA::advance(alda, ailv, k0), bo = OpB::advance(blda, bilv, k0);
+    unsigned char* dst = st + wave * 1024;
+#pragma unroll
+    for (int u = 0; u < OpA::INS; ++u) lds_dma16_buf(ra, dst + u * NT * 16, la.off[u], ao);
+#pragma unroll
+    for (int u = 0; u < OpB::INS; ++u) lds_dma16_buf(rb, dst + A_BYTES + u * NT * 16, lb.off[u], bo);
+  };
+
+  int aof[TM], bof[TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) aof[i] = OpA::frag_off(wm * WTM, lane, i, 0);
+#pragma unroll
+  for (int j = 0; j < TN; ++j) bof[j] = OpB::frag_off(wn * WTN, lane, j, 0);
+  // layout N: k-step ks of a row sits at chunk (2 ks + half) ^ swz, i.e. the offset XOR 32 ks;
+  // layout T: 16 k rows further
+  auto at_step = [&](int off, int ks, bool t, int rowb) { return t ? off + ks * 16 * rowb : off ^ (ks * 32); };
+
+  bf16x8_v af[2][TM], bfr[2][TN];
+  auto read = [&](auto set, const unsigned char* st, int ks) {
+    constexpr int S = decltype(set)::value;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) bfr[S][j] = OpB::frag(st + A_BYTES + at_step(bof[j], ks, BT, OpB::ROWB));
+#pragma unroll
+    for (int i = 0; i < TM; ++i) af[S][i] = OpA::frag(st + at_step(aof[i], ks, AT, OpA::ROWB));
+  };
+  auto mul = [&](auto set) {
+    constexpr int S = decltype(set)::value;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[S][i], bfr[S][j], acc[i][j], 0, 0, 0);
+  };
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, 1>;
+
+  // Tile kt sits in stage (kt + off) % ST, with off so that the last round ends at stage ST - 1:
+  // a first round of ST - off tiles, full rounds, and a last one that fetches nothing.  The host
+  // gives every k range at least ST tiles.
+  const int nk = (kend - kbeg + BK - 1) / BK;
+  const int rounds = (nk + ST - 1) / ST, off = rounds * ST - nk;
+
+  // One operand read after each product: the LDS and the matrix cores work at the same time.
+  auto interleave = [&] {
+    constexpr int READS = (AT ? 2 : 1) * TM + (BT ? 2 : 1) * TN, MULS = TM * TN;
+    constexpr int PER = (READS + MULS - 1) / MULS;
+#pragma unroll
+    for (int m = 0; m < MULS; ++m) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, PER, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // Products of the tile in stage S; then the next tile: wait for it (YOUNGER tiles' loads may
+  // still be in flight), refill this stage with tile `refill`, read its first operands.
+  auto step = [&](auto s, auto younger, auto more, int refill) {
+    constexpr int S = decltype(s)::value;
+    const unsigned char* st = stage_of(s);
+#pragma unroll
+    for (int ks = 0; ks < KS - 1; ++ks) {
+      if ((ks & 1) == 0) {
+        read(S1{}, st, ks + 1);
+        mul(S0{});
+      } else {
+        read(S0{}, st, ks + 1);
+        mul(S1{});
+      }
+      interleave();
+    }
+    if constexpr (decltype(younger)::value >= 0) {
+      wait_vmcnt_lgkm0<decltype(younger)::value * INS>();
+      wg_barrier();
+      if constexpr (decltype(more)::value) issue(stage_of(s), refill);
+      read(S0{}, stage_of(std::integral_constant<int, (S + 1) % ST>{}), 0);
+    }
+    mul(S1{});
+    interleave();
+  };
+  auto each_stage = [&](auto f) {
+    f(std::integral_constant<int, 0>{});
+    f(std::integral_constant<int, 1>{});
+    if constexpr (ST > 2) f(std::integral_constant<int, 2>{});
+    if constexpr (ST > 3) f(std::integral_constant<int, 3>{});
+  };
+  using Young = std::integral_constant<int, ST - 2>;
+
+  each_stage([&](auto s) {
+    const int t = decltype(s)::value - off;
+    issue(stage_of(s), t < 0 ? t + ST : t);
+  });
+  if (off == 0) wait_vmcnt_lgkm0<(ST - 1) * INS>();  // tile 0 came first
+  else wait_vmcnt_lgkm0<0>();
+  wg_barrier();
+  each_stage([&](auto s) {
+    if (decltype(s)::value == off) read(S0{}, stage_of(s), 0);
+  });
+  int kt = -off;  // the tile of stage 0 in the current round
+  if (off > 0) {
+    each_stage([&](auto s) {
+      if (decltype(s)::value >= off) step(s, Young{}, std::true_type{}, kt + decltype(s)::value + ST);
+    });
+    kt += ST;
+  }
+  for (; kt + ST < nk; kt += ST)
+    each_stage([&](auto s) { step(s, Young{}, std::true_type{}, kt + decltype(s)::value + ST); });
+  each_stage([&](auto s) {
+    step(s, std::integral_constant<int, ST - 2 - decltype(s)::value>{}, std::false_type{}, 0);
+  });
+  __syncthreads();  // the output patches reuse the stages
+
+  // ---------------------------------------------------------------- output: 32 x 64 wave patches
+  const Epilogue& e = p.epi;
+  unsigned char* pst = wave < PPS ? st0 : (wave < 2 * PPS ? st1 : (wave < 3 * PPS ? st2 : st3));
+  float* pt = reinterpret_cast<float*>(pst + (wave % PPS) * kPatchBytes);
+  const int half = lane >> 5, l32 = lane & 31;
+#pragma unroll
+  for (int jp = 0; jp < TN / 2; ++jp) {
+    const int nb = n0 + wn * WTN + jp * 64;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int mb = m0 + wm * WTM + i * 32;
+      wave_lds_fence();
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          pt[(8 * (r >> 2) + 4 * half + (r & 3)) * kPatchPitch + j * 32 + l32] = acc[i][jp * 2 + j][r];
+      wave_lds_fence();
+      if constexpr (EPI == EPI_STORE) {
+        if (partial || e.c_f32) {
+          const int cc = (lane & 15) * 4, n = nb + cc;
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            const int row = u * 4 + (lane >> 4), m = mb + row;
+            if (m >= p.M || n >= p.N) continue;
+            const float4 x = *reinterpret_cast<const float4*>(pt + row * kPatchPitch + cc);
+            if (partial) {
+              float* dst = partial + (int64_t)m * p.N + n;
+              if (vec && n + 4 <= p.N) {
+                *reinterpret_cast<float4*>(dst) = x;
+              } else {
+                const float v[4] = {x.x, x.y, x.z, x.w};
+                for (int t = 0; t < 4 && n + t < p.N; ++t) dst[t] = v[t];
+              }
+            } else {
+              float v[4] = {x.x, x.y, x.z, x.w};
+              store_chunk<4>(e, 0, m, n, p.N, v, vec);
+            }
+          }
+          continue;
+        }
+      }
+      const int cc = (lane & 7) * 8;
+      if constexpr (EPI == EPI_SWIGLU_FWD) {
+        // patch columns 0..31 are the up values, 32..63 the gates of the same neurons
+        const int c8 = (lane & 3) * 8;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int row = u * 16 + (lane >> 2), m = mb + row;
+          if (m >= p.M || nb >= p.N) continue;
+          const float* src = pt + row * kPatchPitch + c8;
+          const float rs = e.row_scale ? e.row_scale[m] : 1.0f;
+          uint32_t uw[4], gw[4], zw[4];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const float2 a = *reinterpret_cast<const float2*>(src + 2 * t);
+            const float2 b = *reinterpret_cast<const float2*>(src + 32 + 2 * t);
+            uw[t] = pack_bf2(a.x, a.y);
+            gw[t] = pack_bf2(b.x, b.y);
+            const float u0 = __uint_as_float(uw[t] << 16), u1 = __uint_as_float(uw[t] & 0xffff0000u);
+            const float g0 = __uint_as_float(gw[t] << 16), g1 = __uint_as_float(gw[t] & 0xffff0000u);
+            zw[t] = pack_bf2(u0 * g0 * sigmoidf_(g0) * rs, u1 * g1 * sigmoidf_(g1) * rs);
+          }
+          bf16* up = e.ug + (int64_t)m * e.ld_ug + nb + c8;
+          *reinterpret_cast<uint4*>(up) = make_uint4(uw[0], uw[1], uw[2], uw[3]);
+          *reinterpret_cast<uint4*>(up + 32) = make_uint4(gw[0], gw[1], gw[2], gw[3]);
+          *reinterpret_cast<uint4*>(e.z + (int64_t)m * e.ld_z + nb / 2 + c8) = make_uint4(zw[0], zw[1], zw[2], zw[3]);
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int row = u * 8 + (lane >> 3), m = mb + row, n = nb + cc;
+          if (m >= p.M || n >= p.N) continue;
+          const float4 x = *reinterpret_cast<const float4*>(pt + row * kPatchPitch + cc);
+          const float4 y = *reinterpret_cast<const float4*>(pt + row * kPatchPitch + cc + 4);
+          float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+          if constexpr (EPI == EPI_STORE) {
+            store_chunk<8>(e, 0, m, n, p.N, v, vec);
+          } else if constexpr (EPI == EPI_SWIGLU_BWD) {
+            // v = dZ of neurons n .. n + 7; their up / gate values sit 32 columns apart
+            const int64_t at = (int64_t)m * e.ld_ug + (int64_t)(n >> 5) * 64 + (n & 31);
+            const uint4 uq = *reinterpret_cast<const uint4*>(e.ug_in + at);
+            const uint4 gq = *reinterpret_cast<const uint4*>(e.ug_in + at + 32);
+            const uint32_t uw[4] = {uq.x, uq.y, uq.z, uq.w}, gw[4] = {gq.x, gq.y, gq.z, gq.w};
+            const float rs = e.row_scale ? e.row_scale[m] : 1.0f;
+            uint32_t du[4], dg[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              float a[2], b[2];
+#pragma unroll
+              for (int h = 0; h < 2; ++h) {
+                const float up = h ? __uint_as_float(uw[t] & 0xffff0000u) : __uint_as_float(uw[t] << 16);
+                const float gt = h ? __uint_as_float(gw[t] & 0xffff0000u) : __uint_as_float(gw[t] << 16);
+                const float s = sigmoidf_(gt), dz = v[2 * t + h] * rs;
+                a[h] = dz * (gt * s);
+                b[h] = dz * up * s * (1.0f + gt * (1.0f - s));
+              }
+              du[t] = pack_bf2(a[0], a[1]);
+              dg[t] = pack_bf2(b[0], b[1]);
+            }
+            *reinterpret_cast<uint4*>(e.ug + at) = make_uint4(du[0], du[1], du[2], du[3]);
+            *reinterpret_cast<uint4*>(e.ug + at + 32) = make_uint4(dg[0], dg[1], dg[2], dg[3]);
+          } else {  // EPI_ROPE_QKV: 8 columns of one head; RoPE pairs (2i, 2i + 1)
+            const int part = n / e.dmodel, within = n - part * e.dmodel;
+            const int hh = within / e.hd, dim = within - hh * e.hd;
+            const int b = m / e.S, s = m - b * e.S;
+            if (part < 2) {
+              const float* cp = e.cos_t + (int64_t)s * e.hd + dim;
+              const float* sp = e.sin_t + (int64_t)s * e.hd + dim;
+#pragma unroll
+              for (int t = 0; t < 4; ++t) {
+                const float2 c = *reinterpret_cast<const float2*>(cp + 2 * t);
+                const float2 sn = *reinterpret_cast<const float2*>(sp + 2 * t);
+                const float xe = v[2 * t], xo = v[2 * t + 1];
+                v[2 * t] = xe * c.x - xo * sn.x;
+                v[2 * t + 1] = xo * c.y + xe * sn.y;
+              }
+            }
+            bf16* dst = part == 0 ? e.q : (part == 1 ? e.k : e.v);
+            *reinterpret_cast<uint4*>(dst + (((int64_t)b * e.H + hh) * e.S + s) * e.hd + dim) =
+                make_uint4(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]), pack_bf2(v[4], v[5]), pack_bf2(v[6], v[7]));
+          }
+        }
+      }
+    }
+  }
+}
+
+template <int BM, int BN, int WM, int WN, int BK, int ST, bool AT, bool BT, int EPI>
+int launch(const GemmArgs& p, hipStream_t stream, int vec) {
+  auto fn = gemm_tile_kernel<BM, BN, WM, WN, BK, ST, AT, BT, EPI>;
+  const int64_t tiles = (int64_t)((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
+  hipLaunchKernelGGL(fn, dim3((unsigned)tiles, (unsigned)(p.splits > 1 ? p.splits : 1)), dim3(WM * WN * 64), 0, stream,
+                     p, vec);
+  return check_launch("gemm_tile");
+}
+
+template <int BM, int BN, int WM, int WN, int BK, int ST, int EPI>
+int layouts(const GemmArgs& p, hipStream_t stream, int vec) {
+  if (!p.a_t && !p.b_t) return launch<BM, BN, WM, WN, BK, ST, false, false, EPI>(p, stream, vec);
+  if constexpr (EPI == EPI_STORE || EPI == EPI_SWIGLU_BWD) {
+    if (!p.a_t) return launch<BM, BN, WM, WN, BK, ST, false, true, EPI>(p, stream, vec);
+  }
+  if constexpr (EPI == EPI_STORE) {
+    if (p.b_t) return launch<BM, BN, WM, WN, BK, ST, true, true, EPI>(p, stream, vec);
+  }
+  set_error("gemm_tile: operand layouts not taken by this epilogue");
+  return -1;
+}
+
+
+// Tile and split choice: the estimated time of each (tile, splits) pair, in us.  Measured on the
+// card (M x N x K from 128 x 512 x 512 to 16384 x 8192 x 16384, all layouts): a 256x256 tile alone
+// on its CU takes 0.0268 us per k (1.25 PFLOP/s over the chip); a 128x128 tile 0.0155 with two on
+// its CU, 0.0104 alone and 0.0085 with most of the chip idle; a round of workgroups costs about 4.5
+// us besides (first loads, output).  Split partials are written and read once at about 5 TB/s, and
+// the reduce launch costs about 6 us.  The estimate is mostly within 15% of the measured times, so
+// it picks the large tile where the grid fills the chip (16384 x 3072 x 1024: 104 us against 118),
+// the small one where it does not (8192 x 512 x 4096: 46 against 81), and splits long reductions
+// into one chip's worth of workgroups (3072 x 1024 x 16384: 111 us at 4 splits; the same product
+// unsplit on 128x128 tiles: 263).
+struct TilePick {
+  int tile, splits;
+  double us;
+};
+
+TilePick pick_tile(int M, int N, int K, int lo, int hi, size_t max_split_bytes) {
+  TilePick best{128, 1, 1e30};
+  for (int tile : {256, 128}) {
+    const int64_t tiles = (int64_t)((M + tile - 1) / tile) * ((N + tile - 1) / tile);
+    const int64_t slots = tile == 256 ? 256 : 512;
+    for (int s = lo; s <= hi; ++s) {
+      const int kc = ((K + s - 1) / s + 63) / 64 * 64;
+      if (s > 1 && (kc < 256 || (K + kc - 1) / kc != s || K - (s - 1) * kc < kTileMinK)) continue;
+      if (tiles * s > 2 * slots && s > lo) break;  // two rounds of splits never pay
+      const double part = 4.0 * M * N * s;
+      if (s > 1 && part > (double)max_split_bytes) break;
+      const int64_t wgs = tiles * s, rounds = (wgs + slots - 1) / slots;
+      const double per_k = tile == 256 ? 0.0268 : (wgs <= 64 ? 0.0085 : (wgs <= 256 ? 0.0104 : 0.0155));
+      const double us = rounds * (per_k * (s > 1 ? kc : K) + 4.5) + (s > 1 ? 2.0 * part / 5e6 + 6.0 : 0.0);
+      if (us < best.us) best = {tile, s, us};
+    }
+  }
+  return best;
+}
+
+template <int EPI>
+int launch_tile(const GemmArgs& p, hipStream_t stream, int vec, int tile) {
+  if (tile == 256) return layouts<256, 256, 2, 4, 64, 2, EPI>(p, stream, vec);
+  // both operands layout T: rows are long whatever BK is, four short stages hide more latency
+  // (512 x 2048 x 8192 in 4 splits: 31 us against 33); layout N wants whole 128-byte lines per row
+  // (8192 x 2048 x 8192: 258 us against 316)
+  if constexpr (EPI == EPI_STORE) {
+    if (p.a_t) return launch<128, 128, 2, 2, 32, 4, true, true, EPI>(p, stream, vec);
+  }
+  return layouts<128, 128, 2, 2, 64, 2, EPI>(p, stream, vec);
+}
+
+}  // namespace
+
+int gemm_tile_launch(const GemmArgs& p0, int epi_kind, hipStream_t stream, int vec, void* ws, size_t ws_bytes,
+                     int* splits) {
+  GemmArgs p = p0;
+  const bool may_split = epi_kind == EPI_STORE && ws;
+  int lo = 1, hi = 1;
+  if (may_split && p.a_t) {
+    hi = kTileMaxSplits;
+  } else if (may_split && p.K > kTileRowK) {
+    // Rows of activations: the number of splits sets the order of an element's sum, so it is
+    // chosen for the nearest power of two of M: a sample's rows give the same bits whether a few
+    // other rows share their call or not.
+    int m2 = 64;
+    while ((double)p.M > 1.4142 * m2) m2 *= 2;
+    lo = hi = pick_tile(m2, p.N, p.K, 1, kTileMaxSplits, ws_bytes / 2).splits;
+  }
+  const TilePick pick = pick_tile(p.M, p.N, p.K, lo, hi, ws_bytes);
+  p.splits = pick.splits;
+  if (p.splits > 1) {
+    p.k_chunk = ((p.K + p.splits - 1) / p.splits + 63) / 64 * 64;
+    p.splitk_ws = static_cast<float*>(ws);
+  }
+  *splits = p.splits;
+  switch (epi_kind) {
+    case EPI_STORE: return launch_tile<EPI_STORE>(p, stream, vec, pick.tile);
+    case EPI_SWIGLU_FWD: return launch_tile<EPI_SWIGLU_FWD>(p, stream, vec, pick.tile);
+    case EPI_SWIGLU_BWD: return launch_tile<EPI_SWIGLU_BWD>(p, stream, vec, pick.tile);
+    default: return launch_tile<EPI_ROPE_QKV>(p, stream, vec, pick.tile);
+  }
+}
+
+}  // namespace rte

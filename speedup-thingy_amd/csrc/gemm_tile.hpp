@@ -1,0 +1,21 @@
+// Dense GEMM on the register-pipelined tile kernels (gemm_tile.hip).
+#pragma once
+
+#include "gemm.hpp"
+
+namespace rte {
+
+constexpr int kTileMinK = 128;      // shortest k range of a workgroup: one tile per LDS stage
+constexpr int kTileMaxSplits = 32;
+// Products over rows of activations (layout-N A) up to this k are never split, whatever M: a
+// 1024 x 512 x 512 product takes 8.8 us in one launch, 12.8 in four splits and their sum; 128 x 512
+// x 512 8.7 and 8.6.
+constexpr int kTileRowK = 512;
+
+// Launches p (MODE_DENSE, operands in plain layouts with a_bytes / b_bytes set) on the tile the
+// estimate picks.  EPI_STORE with a workspace may split the reduction: *splits > 1 then says how
+// many fp32 [M, N] partials the launch leaves in ws for the caller to sum in order.
+int gemm_tile_launch(const GemmArgs& p, int epi_kind, hipStream_t stream, int vec, void* ws, size_t ws_bytes,
+                     int* splits);
+
+}  // namespace rte

@@ -1,0 +1,107 @@
+"""The register-pipelined tile GEMM (csrc/gemm_tile.hip) at the sizes where it can go wrong: tile
+edges, odd numbers of k tiles, ragged layout-T reductions (rows past the end come back as zeros),
+split reductions, and its epilogues (residual / beta / alpha, bf16 and fp32 output, SwiGLU forward
+and backward), against float64 on the CPU.
+
+Tolerances: bf16 operands are exact in float64; an fp32 sum of K products is off by at most about
+sqrt(K) 2^-24 of the row norms (Frobenius, factor 8 for the worst draw), a bf16 output by 2^-9."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _hip():
+    from rte_amd import _lib
+
+    if not _lib.device_ready():
+        pytest.fail("HIP backend not ready on this GPU box (library or gfx950 device missing)")
+    yield
+
+
+def _rel(got, ref):
+    return float((got.double().cpu() - ref).norm() / ref.norm())
+
+
+def _mat(rows, cols, g):
+    return torch.randn(rows, cols, generator=g).to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("lay,M,N,K", [
+    ("nn", 65, 72, 128),        # one k tile per stage, ragged tile edges
+    ("nn", 7, 520, 512),        # few rows, short reduction: unsplit
+    ("nn", 129, 136, 192),      # three k tiles in two stages
+    ("nn", 300, 200, 576),
+    ("nn", 4096, 4160, 320),    # 256 x 256 tiles with ragged columns, odd tile count
+    ("nt", 257, 264, 448),
+    ("nt", 1000, 512, 4096),    # split reduction over activation rows
+    ("tt", 136, 128, 129),      # ragged reductions: one row past, most of a tile missing, long
+    ("tt", 72, 264, 200),
+    ("tt", 512, 520, 8191),     # split, the last chunk ragged
+    ("tt", 4096, 4352, 1000),   # 256 x 256 tiles, ragged reduction
+    ("tt", 96, 96, 127),        # below the kernel's shortest reduction: the general kernel
+])
+@pytest.mark.parametrize("f32", [True, False])
+def test_layouts(lay, M, N, K, f32):
+    from rte_amd.kernels import hip_ops as H
+
+    g = torch.Generator().manual_seed(M * 31 + N * 7 + K)
+    a = _mat(K, M, g) if lay[0] == "t" else _mat(M, K, g)
+    b = _mat(K, N, g) if lay[1] == "t" else _mat(N, K, g)
+    ref = (a.double().t() if lay[0] == "t" else a.double()) @ (b.double() if lay[1] == "t" else b.double().t())
+    got = H.gemm(a.to(DEV), b.to(DEV), a_t=lay[0] == "t", b_t=lay[1] == "t", out_f32=f32)
+    tol = 8 * K**0.5 * 2**-24 if f32 else 2**-9
+    assert _rel(got, ref) <= tol
+    again = H.gemm(a.to(DEV), b.to(DEV), a_t=lay[0] == "t", b_t=lay[1] == "t", out_f32=f32)
+    assert torch.equal(got, again)
+
+
+@pytest.mark.parametrize("M,K", [(200, 256), (1000, 4096)])  # unsplit, split
+def test_epilogue_terms(M, K):
+    from rte_amd.kernels import hip_ops as H
+
+    g = torch.Generator().manual_seed(3)
+    N = 136
+    a, b = _mat(M, K, g), _mat(N, K, g)
+    r, c = torch.randn(M, N, generator=g), torch.randn(M, N, generator=g)
+    ref = 0.5 * (a.double() @ b.double().t()) + r.double() - 2.0 * c.double()
+    got = H.gemm(a.to(DEV), b.to(DEV), alpha=0.5, resid=r.to(DEV), out=c.to(DEV), beta=-2.0, out_f32=True)
+    assert _rel(got, ref) <= 8 * K**0.5 * 2**-24
+
+
+def test_rows_do_not_depend_on_their_company():
+    """An activation row's product has the same bits alone, in a small call and in a larger one
+    (unsplit k, and a split k within one power of two of rows)."""
+    from rte_amd.kernels import hip_ops as H
+
+    g = torch.Generator().manual_seed(5)
+    for K, sizes in ((512, (64, 1088, 8192)), (2048, (1024, 1088))):
+        a, b = _mat(max(sizes), K, g).to(DEV), _mat(520, K, g).to(DEV)
+        outs = [H.gemm(a[:m].contiguous(), b, out_f32=True)[:64] for m in sizes]
+        for o in outs[1:]:
+            assert torch.equal(o, outs[0])
+
+
+@pytest.mark.parametrize("T,d,F", [(5, 128, 32), (70, 192, 96), (300, 256, 1056), (2048, 512, 2048)])
+def test_dense_swiglu(T, d, F):
+    from rte_amd.kernels import hip_ops as H
+
+    g = torch.Generator().manual_seed(T)
+    x, dy = _mat(T, d, g), _mat(T, d, g)
+    wug, wd = (torch.randn(2 * F, d, generator=g) * d**-0.5), (torch.randn(d, F, generator=g) * F**-0.5)
+    args = [t.to(DEV).requires_grad_() for t in (x, wug, wd)]
+    y = H.dense_swiglu(*args)
+    grads = torch.autograd.grad(y, args, dy.float().to(DEV))
+    ref_args = [t.to(torch.bfloat16).double().requires_grad_() for t in (x, wug, wd)]
+    up, gate = (ref_args[0] @ ref_args[1].t()).chunk(2, dim=-1)
+    ref = (up * torch.nn.functional.silu(gate)) @ ref_args[2].t()
+    ref_grads = torch.autograd.grad(ref, ref_args, dy.double())
+    # up, gate, z, dz, dug are each kept in bf16 (2^-9 relative at most, 2^-10 rms): a few of them meet
+    for got, want in zip((y, *grads), (ref, *ref_grads)):
+        assert _rel(got, want.detach()) <= 4 * 2**-9
