@@ -724,6 +724,15 @@ int rte_gemm_f32(const float* A, int64_t lda, int a_t, const int32_t* a_rows, co
                  int64_t ldb, int b_t, const int32_t* b_rows, const float* b_scale, float* C, int64_t ldc,
                  const int32_t* c_rows, int M, int N, int K, float alpha, float beta, int Z1, int Z2, int64_t sA1,
                  int64_t sA2, int64_t sB1, int64_t sB2, int64_t sC1, int64_t sC2, void* stream);
+/* The same with a workspace of at least rte_gemm_f32_workspace_bytes(M, N, K): a long reduction with
+ * A transposed (a weight gradient) and one batch is cut into k ranges over more workgroups, their
+ * fp32 partials added in order by a second launch. */
+size_t rte_gemm_f32_workspace_bytes(int M, int N, int K);
+int rte_gemm_f32_ws(const float* A, int64_t lda, int a_t, const int32_t* a_rows, const float* a_scale, const float* B,
+                    int64_t ldb, int b_t, const int32_t* b_rows, const float* b_scale, float* C, int64_t ldc,
+                    const int32_t* c_rows, int M, int N, int K, float alpha, float beta, int Z1, int Z2, int64_t sA1,
+                    int64_t sA2, int64_t sB1, int64_t sB2, int64_t sC1, int64_t sC2, void* ws, size_t ws_bytes,
+                    void* stream);
 /* Grouped form over device offsets goff[G+1] (int32).  mode 1 (rows): group g computes output rows
  * [goff[g], goff[g+1]) of the M total with B at b_goff[g] (int64, optional) or g*b_gstride and
  * b_rows shifted by g*b_rows_gstride: the routed / banked pools' per-cluster products and the macro
@@ -738,6 +747,15 @@ int rte_gemm_f32_grouped(int mode, const int32_t* goff, int G, const float* A, i
                          int64_t b_rows_gstride, float* C, int64_t ldc, const int32_t* c_rows, const int64_t* c_goff,
                          int64_t c_gstride, int64_t c_rows_gstride, int M, int N, int K, float alpha, float beta,
                          void* stream);
+/* The same with a workspace of at least rte_gemm_f32_grouped_workspace_bytes: mode 2 cuts each
+ * group's reduction into chunks (partials added in order by a second launch). */
+size_t rte_gemm_f32_grouped_workspace_bytes(int mode, int M, int N, int K, int G);
+int rte_gemm_f32_grouped_ws(int mode, const int32_t* goff, int G, const float* A, int64_t lda, int a_t,
+                            const int32_t* a_rows, const float* a_scale, const float* B, int64_t ldb, int b_t,
+                            const int32_t* b_rows, const float* b_scale, const int64_t* b_goff, int64_t b_gstride,
+                            int64_t b_rows_gstride, float* C, int64_t ldc, const int32_t* c_rows,
+                            const int64_t* c_goff, int64_t c_gstride, int64_t c_rows_gstride, int M, int N, int K,
+                            float alpha, float beta, void* ws, size_t ws_bytes, void* stream);
 /* Causal softmax of score rows s [Z, S, S] (F.scaled_dot_product_attention(is_causal=True)'s
  * softmax, rte/kernels/optimized.py:75-91): p = softmax(scale s) over keys <= query, y = oscale[z] p
  * (oscale optional: the banked recipe's head mask, rte/layers.py:702-728).  rows = Z*S. */

@@ -14,9 +14,14 @@
 //  * pair combine (out[t] = resid[t] + sum_j w[t, j] rows[slot(t, j)]) and the pair row dots of its
 //    weight gradient
 //
-// Tile: 64 x 64 outputs per 256-thread workgroup (four waves of 32 x 32), k steps of 16 staged
-// through LDS k-major (each MFMA operand a contiguous 32-float LDS row segment), the next k tile's
-// global loads issued before the current tile's MFMAs.
+// Tile: 64 x 64 outputs per 256-thread workgroup (four waves of 32 x 32), k steps of 32 staged
+// through two LDS buffers k-major (each MFMA operand a contiguous 32-float LDS row segment): while
+// step s multiplies, step s + 1 is written to the other buffer and step s + 2 is on its way from
+// memory, with one barrier per step.  These products are bound by the latency of their k steps and
+// by too few workgroups, not by the matrix cores, so long reductions are cut into k ranges whose
+// fp32 partials a second kernel adds in order: a 32 x 256 x 8192 weight gradient took 4 workgroups
+// 512 serial steps before.  fp32 routed pool layer (T 8192, d 256, 32 x 32, top-4) forward +
+// backward: 1333 -> 540 us (kernel time 1361 -> 327).
 #include "common.hpp"
 
 namespace rte {
@@ -24,8 +29,8 @@ namespace {
 
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
 
-constexpr int kBM = 64, kBN = 64, kBK = 16, kThreads = 256;
-constexpr int kPad = 4;
+constexpr int kBM = 64, kBN = 64, kBK = 32, kThreads = 256;
+constexpr int kPitch = kBM + 4;
 
 struct GemmF32 {
   const float* A;
@@ -54,132 +59,209 @@ struct GemmF32 {
   int64_t b_gstride, b_rows_gstride;
   const int64_t* c_goff;  // GROUP_K: C element offset of group g (else g * c_gstride)
   int64_t c_gstride, c_rows_gstride;
+  // split reductions: dense (mode 0, one batch) split blockIdx.z covers k [z chunk, (z + 1) chunk);
+  // GROUP_K work item blockIdx.z is a chunk of its group (an empty group has one item, a group of
+  // one chunk stores directly).  part holds fp32 [item][M][N].
+  int chunk;
+  float* part;
 };
 
-// One 64 x 16 operand tile into registers: element e of thread t.  Non-transposed operands are
-// contiguous along k (thread: one row, four k), transposed ones along the row index (thread: one
-// k, four rows).  Rows outside [r0, r_end) and k outside [k0, k_end) read as 0.
-__device__ __forceinline__ void load_tile(const float* X, int64_t ld, int x_t, const int32_t* rows,
-                                          const float* scale, int r0, int r_end, int k0, int k_end, float v[4]) {
-  const int t = threadIdx.x;
-  if (!x_t) {
-    const int r = r0 + (t >> 2);
-    const int kq = k0 + (t & 3) * 4;
-    if (r < r_end) {
-      const int64_t row = rows ? (int64_t)rows[r] : (int64_t)r;
-      const float sc = scale ? scale[r] : 1.0f;
-      const float* p = X + row * ld;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = (kq + i < k_end) ? p[kq + i] * sc : 0.0f;
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = 0.0f;
-    }
-  } else {
-    const int k = k0 + (t >> 4);
-    const int rq = r0 + (t & 15) * 4;
+// One 64 x 32 operand tile through registers, eight elements per thread.  Non-transposed operands
+// are contiguous along k (thread: one row, eight k), transposed ones along the row index (thread:
+// one k, eight rows).  Rows outside [r0, r_end) and k outside [k_lo, k_end) read as 0.
+template <bool T>
+struct TileF32 {
+  const float* base;
+  const float* row_ptr;  // layout N: this thread's row, nullptr past the end
+  float row_scale;
+  int next_row;  // layout T: the memory row of the next step's k (gathers are looked up a step ahead)
+  float next_scale;
+  float v[8];
+
+  __device__ __forceinline__ static int sub() { return T ? threadIdx.x >> 3 : threadIdx.x >> 2; }
+  __device__ __forceinline__ static int at() { return T ? (threadIdx.x & 7) * 8 : (threadIdx.x & 3) * 8; }
+
+  __device__ __forceinline__ void look(const int32_t* rows, const float* scale, int k0, int k_end) {
+    const int k = k0 + sub();
+    next_row = k;
+    next_scale = 1.0f;
     if (k < k_end) {
-      const int64_t row = rows ? (int64_t)rows[k] : (int64_t)k;
-      const float sc = scale ? scale[k] : 1.0f;
-      const float* p = X + row * ld;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = (rq + i < r_end) ? p[rq + i] * sc : 0.0f;
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = 0.0f;
+      if (rows) next_row = rows[k];
+      if (scale) next_scale = scale[k];
     }
   }
-}
-
-__device__ __forceinline__ void store_tile(float (*S)[kBM + kPad], int x_t, const float v[4]) {
-  const int t = threadIdx.x;
-  if (!x_t) {
-    const int r = t >> 2, kq = (t & 3) * 4;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) S[kq + i][r] = v[i];
-  } else {
-    const int k = t >> 4, rq = (t & 15) * 4;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) S[k][rq + i] = v[i];
+  __device__ __forceinline__ void init(const float* X, int64_t ld, const int32_t* rows, const float* scale, int r0,
+                                       int r_end, int k_lo, int k_end) {
+    base = X;
+    if constexpr (T) {
+      look(rows, scale, k_lo, k_end);
+    } else {
+      const int r = r0 + sub();
+      row_ptr = r < r_end ? X + (int64_t)(rows ? rows[r] : r) * ld : nullptr;
+      row_scale = (scale && r < r_end) ? scale[r] : 1.0f;
+    }
   }
+  // the tile starting at k0; vec: 16-byte loads are aligned
+  __device__ __forceinline__ void load(int64_t ld, const int32_t* rows, const float* scale, int r0, int r_end, int k0,
+                                       int k_end, bool vec) {
+    const float* p;
+    float sc;
+    int n;  // valid elements from p on
+    if constexpr (T) {
+      p = base + (int64_t)next_row * ld + r0 + at();
+      sc = next_scale;
+      n = k0 + sub() < k_end ? r_end - r0 - at() : 0;
+      look(rows, scale, k0 + kBK, k_end);
+    } else {
+      p = row_ptr + k0 + at();
+      sc = row_scale;
+      n = row_ptr ? k_end - k0 - at() : 0;
+    }
+    if (n >= 8 && vec) {
+      const float4 x = *reinterpret_cast<const float4*>(p), y = *reinterpret_cast<const float4*>(p + 4);
+      v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+      v[4] = y.x; v[5] = y.y; v[6] = y.z; v[7] = y.w;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = i < n ? p[i] : 0.0f;
+    }
+    if (scale) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] *= sc;
+    }
+  }
+  __device__ __forceinline__ void store(float (*S)[kPitch]) const {
+    if constexpr (T) {
+      float* d = &S[sub()][at()];
+      *reinterpret_cast<float4*>(d) = make_float4(v[0], v[1], v[2], v[3]);
+      *reinterpret_cast<float4*>(d + 4) = make_float4(v[4], v[5], v[6], v[7]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) S[at() + i][sub()] = v[i];
+    }
+  }
+};
+
+// Group and position of element x of the sequence that lists, group by group, ceil(count / per)
+// entries (at least `least`): 64 groups at a time by one wave.  Returns {group or -1, index within
+// the group, entries of the group}.
+__device__ __forceinline__ int3 find_group(const int32_t* goff, int G, int per, int least, int x, int lane) {
+  int base = 0;
+  for (int c0 = 0; c0 < G; c0 += 64) {
+    const int g = c0 + lane;
+    int cnt = 0;
+    if (g < G) {
+      cnt = (goff[g + 1] - goff[g] + per - 1) / per;
+      if (cnt < least) cnt = least;
+    }
+    int incl = cnt;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int y = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += y;
+    }
+    const unsigned long long hit = __ballot(cnt > 0 && x >= base + incl - cnt && x < base + incl);
+    if (hit) {
+      const int l = __ffsll((long long)hit) - 1;
+      const int n = __shfl(cnt, l, 64);
+      return make_int3(c0 + l, x - base - __shfl(incl, l, 64) + n, n);
+    }
+    base += __shfl(incl, 63, 64);
+  }
+  return make_int3(-1, 0, 0);
 }
 
+template <bool AT, bool BT>
 __global__ void __launch_bounds__(kThreads) gemm_f32_kernel(GemmF32 p) {
-  __shared__ float As[kBK][kBM + kPad];
-  __shared__ float Bs[kBK][kBN + kPad];
-  __shared__ int s_info[3];
+  __shared__ __align__(16) float As[2][kBK][kPitch];
+  __shared__ __align__(16) float Bs[2][kBK][kPitch];
   const float* A = p.A;
   const float* B = p.B;
   float* C = p.C;
   const int32_t* b_rows = p.b_rows;
   const int32_t* c_rows = p.c_rows;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int m0, m_end = p.M, k_lo = 0, k_hi = p.K;
   const int n0 = blockIdx.y * kBN;
+  float* part = nullptr;
   if (p.mode == 1) {
-    // GROUP_M: the x index enumerates each group's row tiles in group order (one thread walks the
-    // offsets; tile counts are ceil(rows / 64) per group)
-    if (threadIdx.x == 0) {
-      int tile = blockIdx.x, g = 0, found = -1, start = 0;
-      for (; g < p.G; ++g) {
-        const int lo = p.goff[g], hi = p.goff[g + 1];
-        const int nt = (hi - lo + kBM - 1) / kBM;
-        if (tile < nt) {
-          found = g;
-          start = lo + tile * kBM;
-          break;
-        }
-        tile -= nt;
-      }
-      s_info[0] = found;
-      s_info[1] = start;
-      s_info[2] = found >= 0 ? p.goff[found + 1] : 0;
-    }
-    __syncthreads();
-    const int g = s_info[0];
+    // GROUP_M: the x index enumerates each group's row tiles in group order
+    const int3 f = find_group(p.goff, p.G, kBM, 0, blockIdx.x, lane);
+    const int g = f.x;
     if (g < 0) return;
-    m0 = s_info[1];
-    m_end = s_info[2];
+    m0 = p.goff[g] + f.y * kBM;
+    m_end = p.goff[g + 1];
     B += p.b_goff ? p.b_goff[g] : (int64_t)g * p.b_gstride;
     if (b_rows) b_rows += (int64_t)g * p.b_rows_gstride;
   } else if (p.mode == 2) {
-    const int g = blockIdx.z;
+    int g = blockIdx.z;
     m0 = blockIdx.x * kBM;
-    k_lo = p.goff[g];
-    k_hi = p.goff[g + 1];
+    if (p.part) {
+      const int3 f = find_group(p.goff, p.G, p.chunk, 1, blockIdx.z, lane);
+      g = f.x;
+      if (g < 0) return;
+      k_lo = p.goff[g] + f.y * p.chunk;
+      k_hi = k_lo + p.chunk < p.goff[g + 1] ? k_lo + p.chunk : p.goff[g + 1];
+      if (f.z > 1) part = p.part + (int64_t)blockIdx.z * p.M * p.N;
+    } else {
+      k_lo = p.goff[g];
+      k_hi = p.goff[g + 1];
+    }
     C += p.c_goff ? p.c_goff[g] : (int64_t)g * p.c_gstride;
     if (c_rows) c_rows += (int64_t)g * p.c_rows_gstride;
   } else {
     m0 = blockIdx.x * kBM;
-    const int z = blockIdx.z, z1 = z / p.Z2, z2 = z - z1 * p.Z2;
-    A += z1 * p.sA1 + z2 * p.sA2;
-    B += z1 * p.sB1 + z2 * p.sB2;
-    C += z1 * p.sC1 + z2 * p.sC2;
+    if (p.part) {
+      k_lo = blockIdx.z * p.chunk;
+      k_hi = k_lo + p.chunk < p.K ? k_lo + p.chunk : p.K;
+      part = p.part + (int64_t)blockIdx.z * p.M * p.N;
+    } else {
+      const int z = blockIdx.z, z1 = z / p.Z2, z2 = z - z1 * p.Z2;
+      A += z1 * p.sA1 + z2 * p.sA2;
+      B += z1 * p.sB1 + z2 * p.sB2;
+      C += z1 * p.sC1 + z2 * p.sC2;
+    }
   }
   if (m0 >= m_end || n0 >= p.N) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   f32x16 acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-  float va[4], vb[4];
   // a_t: A's memory rows run over k; else over m (rows gathered / scaled by the logical index)
-  load_tile(A, p.lda, p.a_t, p.a_rows, p.a_scale, m0, m_end, k_lo, k_hi, va);
-  load_tile(B, p.ldb, p.b_t, b_rows, p.b_scale, n0, p.N, k_lo, k_hi, vb);
-  for (int k0 = k_lo; k0 < k_hi; k0 += kBK) {
-    store_tile(As, p.a_t, va);
-    store_tile(Bs, p.b_t, vb);
+  const bool avec = (((uintptr_t)A | ((uintptr_t)p.lda << 2)) & 15) == 0 && (AT || (k_lo & 3) == 0);
+  const bool bvec = (((uintptr_t)B | ((uintptr_t)p.ldb << 2)) & 15) == 0 && (BT || (k_lo & 3) == 0);
+  TileF32<AT> ta;
+  TileF32<BT> tb;
+  auto load = [&](int k0) {
+    ta.load(p.lda, p.a_rows, p.a_scale, m0, m_end, k0, k_hi, avec);
+    tb.load(p.ldb, b_rows, p.b_scale, n0, p.N, k0, k_hi, bvec);
+  };
+  auto store = [&](int b) {
+    ta.store(As[b]);
+    tb.store(Bs[b]);
+  };
+  if (k_lo < k_hi) {
+    ta.init(A, p.lda, p.a_rows, p.a_scale, m0, m_end, k_lo, k_hi);
+    tb.init(B, p.ldb, b_rows, p.b_scale, n0, p.N, k_lo, k_hi);
+    load(k_lo);
+    store(0);
+    if (k_lo + kBK < k_hi) load(k_lo + kBK);
     __syncthreads();
-    if (k0 + kBK < k_hi) {
-      load_tile(A, p.lda, p.a_t, p.a_rows, p.a_scale, m0, m_end, k0 + kBK, k_hi, va);
-      load_tile(B, p.ldb, p.b_t, b_rows, p.b_scale, n0, p.N, k0 + kBK, k_hi, vb);
-    }
+    int buf = 0;
+    for (int k0 = k_lo; k0 < k_hi; k0 += kBK) {
+      if (k0 + kBK < k_hi) {
+        store(buf ^ 1);
+        if (k0 + 2 * kBK < k_hi) load(k0 + 2 * kBK);
+      }
 #pragma unroll
-    for (int kk = 0; kk < kBK; kk += 2) {
-      const float a = As[kk + (lane >> 5)][wm * 32 + (lane & 31)];
-      const float b = Bs[kk + (lane >> 5)][wn * 32 + (lane & 31)];
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
+      for (int kk = 0; kk < kBK; kk += 2) {
+        const float a = As[buf][kk + (lane >> 5)][wm * 32 + (lane & 31)];
+        const float b = Bs[buf][kk + (lane >> 5)][wn * 32 + (lane & 31)];
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
+      }
+      __syncthreads();
+      buf ^= 1;
     }
-    __syncthreads();
   }
   const int col = n0 + wn * 32 + (lane & 31);
   if (col >= p.N) return;
@@ -187,12 +269,107 @@ __global__ void __launch_bounds__(kThreads) gemm_f32_kernel(GemmF32 p) {
   for (int r = 0; r < 16; ++r) {
     const int m = m0 + wm * 32 + (lane >> 5) * 4 + (r >> 2) * 8 + (r & 3);
     if (m < m_end) {
+      if (part) {
+        part[(int64_t)m * p.N + col] = acc[r];
+        continue;
+      }
       const int64_t row = c_rows ? (int64_t)c_rows[m] : (int64_t)m;
       float* c = C + row * p.ldc + col;
       const float v = p.alpha * acc[r];
       *c = p.beta != 0.0f ? v + p.beta * *c : v;
     }
   }
+}
+
+// The partials of a split reduction, added in k order.  Grid (elements / 256, groups or 1).
+__global__ void __launch_bounds__(256) gemm_f32_reduce_kernel(GemmF32 p, int items) {
+  const int g = blockIdx.y;
+  int q0 = 0, n = items;
+  float* C = p.C;
+  const int32_t* c_rows = p.c_rows;
+  if (p.mode == 2) {
+    // the group's items: entries of the groups before it, and its own
+    __shared__ int s_q[2];
+    if (threadIdx.x < 64) {
+      int before = 0, own = 0;
+      for (int h = threadIdx.x; h <= g; h += 64) {
+        int cnt = (p.goff[h + 1] - p.goff[h] + p.chunk - 1) / p.chunk;
+        if (cnt < 1) cnt = 1;
+        if (h < g) before += cnt;
+        else own = cnt;
+      }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        before += __shfl_xor(before, o, 64);
+        own += __shfl_xor(own, o, 64);
+      }
+      if (threadIdx.x == 0) {
+        s_q[0] = before;
+        s_q[1] = own;
+      }
+    }
+    __syncthreads();
+    q0 = s_q[0];
+    n = s_q[1];
+    if (n == 1) return;  // stored by the product itself
+    C += p.c_goff ? p.c_goff[g] : (int64_t)g * p.c_gstride;
+    if (c_rows) c_rows += (int64_t)g * p.c_rows_gstride;
+  }
+  const int64_t plane = (int64_t)p.M * p.N;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= plane) return;
+  const float* src = p.part + q0 * plane + i;
+  float v = 0.0f;
+  int q = 0;
+  for (; q + 8 <= n; q += 8) {  // eight partials in flight
+    float x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = src[(q + u) * plane];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v += x[u];
+  }
+  for (; q < n; ++q) v += src[q * plane];
+  const int m = (int)(i / p.N), col = (int)(i - (int64_t)m * p.N);
+  float* c = C + (int64_t)(c_rows ? c_rows[m] : m) * p.ldc + col;
+  v *= p.alpha;
+  *c = p.beta != 0.0f ? v + p.beta * *c : v;
+}
+
+// k range of one workgroup of a split dense product (0: not split): about 512 workgroups of at least
+// 256 k.  Only for weight gradients (A transposed: the reduction runs over tokens), so a row of
+// activations keeps its one sum whatever shares its call.
+int dense_chunk(int M, int N, int K) {
+  const int64_t tiles = (int64_t)((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN);
+  if (tiles >= 256 || K < 512) return 0;
+  int64_t s = (512 + tiles - 1) / tiles;
+  if (s > K / 256) s = K / 256;
+  if (s > 64) s = 64;
+  const int64_t kc = ((K + s - 1) / s + kBK - 1) / kBK * kBK;
+  return kc < K ? (int)kc : 0;
+}
+
+// k chunk of a grouped reduction: 256 (8192 slots of 32 groups, 64 x 256 outputs: 512 workgroups of 8
+// steps), longer where the partials would pass 256 MiB.
+constexpr size_t kGroupPartBytes = (size_t)256 << 20;
+int group_chunk(int M, int N, int K, int G) {
+  int64_t c = 256;
+  while (c < K && ((size_t)(K / c) + 1 + G) * M * N * 4 > kGroupPartBytes) c *= 2;
+  return (int)c;
+}
+
+size_t group_bytes(int M, int N, int K, int G) {
+  const int64_t c = group_chunk(M, N, K, G);
+  if (c >= K) return 0;
+  const size_t b = ((size_t)((K + c - 1) / c) + G) * M * N * 4;
+  return b <= kGroupPartBytes + (size_t)M * N * 4 ? b : 0;
+}
+
+int launch_f32(const GemmF32& p, dim3 grid, hipStream_t stream) {
+  if (!p.a_t && !p.b_t) hipLaunchKernelGGL((gemm_f32_kernel<false, false>), grid, dim3(kThreads), 0, stream, p);
+  else if (!p.a_t) hipLaunchKernelGGL((gemm_f32_kernel<false, true>), grid, dim3(kThreads), 0, stream, p);
+  else if (!p.b_t) hipLaunchKernelGGL((gemm_f32_kernel<true, false>), grid, dim3(kThreads), 0, stream, p);
+  else hipLaunchKernelGGL((gemm_f32_kernel<true, true>), grid, dim3(kThreads), 0, stream, p);
+  return check_launch("gemm_f32");
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -316,48 +493,94 @@ using namespace rte;
 
 extern "C" {
 
-int rte_gemm_f32(const float* A, int64_t lda, int a_t, const int32_t* a_rows, const float* a_scale, const float* B,
-                 int64_t ldb, int b_t, const int32_t* b_rows, const float* b_scale, float* C, int64_t ldc,
-                 const int32_t* c_rows, int M, int N, int K, float alpha, float beta, int Z1, int Z2, int64_t sA1,
-                 int64_t sA2, int64_t sB1, int64_t sB2, int64_t sC1, int64_t sC2, void* stream) {
+size_t rte_gemm_f32_workspace_bytes(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  const int kc = dense_chunk(M, N, K);
+  return kc ? (size_t)((K + kc - 1) / kc) * M * N * 4 : 0;
+}
+
+int rte_gemm_f32_ws(const float* A, int64_t lda, int a_t, const int32_t* a_rows, const float* a_scale, const float* B,
+                    int64_t ldb, int b_t, const int32_t* b_rows, const float* b_scale, float* C, int64_t ldc,
+                    const int32_t* c_rows, int M, int N, int K, float alpha, float beta, int Z1, int Z2, int64_t sA1,
+                    int64_t sA2, int64_t sB1, int64_t sB2, int64_t sC1, int64_t sC2, void* ws, size_t ws_bytes,
+                    void* stream) {
   RTE_REQUIRE(M >= 0 && N >= 0 && K >= 0 && Z1 >= 1 && Z2 >= 1, "gemm_f32: bad sizes");
   RTE_REQUIRE(A && B && C, "gemm_f32: null operand");
   RTE_REQUIRE((int64_t)Z1 * Z2 <= 65535, "gemm_f32: at most 65535 batches");
   if (M == 0 || N == 0) return 0;
   GemmF32 p{A, lda, a_t, a_rows, a_scale, B, ldb, b_t, b_rows, b_scale, C, ldc, c_rows, M, N, K, alpha, beta,
-            Z2, sA1, sA2, sB1, sB2, sC1, sC2, 0, nullptr, 0, nullptr, 0, 0, nullptr, 0, 0};
+            Z2, sA1, sA2, sB1, sB2, sC1, sC2, 0, nullptr, 0, nullptr, 0, 0, nullptr, 0, 0, 0, nullptr};
   dim3 grid((M + kBM - 1) / kBM, (N + kBN - 1) / kBN, Z1 * Z2);
   RTE_REQUIRE(grid.y <= 65535, "gemm_f32: N too large");
-  hipLaunchKernelGGL(gemm_f32_kernel, grid, dim3(kThreads), 0, static_cast<hipStream_t>(stream), p);
-  return check_launch("gemm_f32");
+  const size_t need = a_t && Z1 * Z2 == 1 ? rte_gemm_f32_workspace_bytes(M, N, K) : 0;
+  if (!need || !ws || ws_bytes < need) return launch_f32(p, grid, static_cast<hipStream_t>(stream));
+  p.chunk = dense_chunk(M, N, K);
+  p.part = static_cast<float*>(ws);
+  grid.z = (K + p.chunk - 1) / p.chunk;
+  RTE_TRY(launch_f32(p, grid, static_cast<hipStream_t>(stream)));
+  hipLaunchKernelGGL(gemm_f32_reduce_kernel, dim3((unsigned)(((int64_t)M * N + 255) / 256)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), p, (int)grid.z);
+  return check_launch("gemm_f32_reduce");
+}
+
+int rte_gemm_f32(const float* A, int64_t lda, int a_t, const int32_t* a_rows, const float* a_scale, const float* B,
+                 int64_t ldb, int b_t, const int32_t* b_rows, const float* b_scale, float* C, int64_t ldc,
+                 const int32_t* c_rows, int M, int N, int K, float alpha, float beta, int Z1, int Z2, int64_t sA1,
+                 int64_t sA2, int64_t sB1, int64_t sB2, int64_t sC1, int64_t sC2, void* stream) {
+  return rte_gemm_f32_ws(A, lda, a_t, a_rows, a_scale, B, ldb, b_t, b_rows, b_scale, C, ldc, c_rows, M, N, K, alpha,
+                         beta, Z1, Z2, sA1, sA2, sB1, sB2, sC1, sC2, nullptr, 0, stream);
+}
+
+size_t rte_gemm_f32_grouped_workspace_bytes(int mode, int M, int N, int K, int G) {
+  if (mode != 2 || M <= 0 || N <= 0 || K <= 0 || G <= 0) return 0;
+  return group_bytes(M, N, K, G);
 }
 
 // Grouped products.  mode 1 (GROUP_M): group g owns rows [goff[g], goff[g+1]) of the M total and
 // reads B at b_goff[g] (or g * b_gstride) with b_rows shifted by g * b_rows_gstride.  mode 2
 // (GROUP_K): group g reduces over k in [goff[g], goff[g+1]) and writes C at c_goff[g] (or
-// g * c_gstride) with c_rows shifted by g * c_rows_gstride.
-int rte_gemm_f32_grouped(int mode, const int32_t* goff, int G, const float* A, int64_t lda, int a_t,
-                         const int32_t* a_rows, const float* a_scale, const float* B, int64_t ldb, int b_t,
-                         const int32_t* b_rows, const float* b_scale, const int64_t* b_goff, int64_t b_gstride,
-                         int64_t b_rows_gstride, float* C, int64_t ldc, const int32_t* c_rows, const int64_t* c_goff,
-                         int64_t c_gstride, int64_t c_rows_gstride, int M, int N, int K, float alpha, float beta,
-                         void* stream) {
+// g * c_gstride) with c_rows shifted by g * c_rows_gstride; with a workspace, in chunks.
+int rte_gemm_f32_grouped_ws(int mode, const int32_t* goff, int G, const float* A, int64_t lda, int a_t,
+                            const int32_t* a_rows, const float* a_scale, const float* B, int64_t ldb, int b_t,
+                            const int32_t* b_rows, const float* b_scale, const int64_t* b_goff, int64_t b_gstride,
+                            int64_t b_rows_gstride, float* C, int64_t ldc, const int32_t* c_rows,
+                            const int64_t* c_goff, int64_t c_gstride, int64_t c_rows_gstride, int M, int N, int K,
+                            float alpha, float beta, void* ws, size_t ws_bytes, void* stream) {
   RTE_REQUIRE(mode == 1 || mode == 2, "gemm_f32_grouped: mode must be 1 (rows) or 2 (reduction)");
   RTE_REQUIRE(G >= 0 && M >= 0 && N >= 0 && K >= 0, "gemm_f32_grouped: bad sizes");
   RTE_REQUIRE(goff && A && B && C, "gemm_f32_grouped: null argument");
   if (G == 0 || N == 0 || (mode == 1 && M == 0) || (mode == 2 && M == 0)) return 0;
   GemmF32 p{A, lda, a_t, a_rows, a_scale, B, ldb, b_t, b_rows, b_scale, C, ldc, c_rows, M, N, K, alpha, beta,
             1, 0, 0, 0, 0, 0, 0, mode, goff, G, b_goff, b_gstride, b_rows_gstride, c_goff, c_gstride,
-            c_rows_gstride};
-  dim3 grid;
+            c_rows_gstride, 0, nullptr};
+  const hipStream_t st = static_cast<hipStream_t>(stream);
   if (mode == 1) {
-    grid = dim3((M + kBM - 1) / kBM + G, (N + kBN - 1) / kBN, 1);  // a bound on the groups' row tiles
-  } else {
-    RTE_REQUIRE(G <= 65535, "gemm_f32_grouped: at most 65535 reduction groups");
-    grid = dim3((M + kBM - 1) / kBM, (N + kBN - 1) / kBN, G);
+    // a bound on the groups' row tiles
+    return launch_f32(p, dim3((M + kBM - 1) / kBM + G, (N + kBN - 1) / kBN, 1), st);
   }
-  hipLaunchKernelGGL(gemm_f32_kernel, grid, dim3(kThreads), 0, static_cast<hipStream_t>(stream), p);
-  return check_launch("gemm_f32_grouped");
+  RTE_REQUIRE(G <= 65535, "gemm_f32_grouped: at most 65535 reduction groups");
+  dim3 grid((M + kBM - 1) / kBM, (N + kBN - 1) / kBN, G);
+  const size_t need = group_bytes(M, N, K, G);
+  const int64_t chunk = group_chunk(M, N, K, G), items = ((int64_t)K + chunk - 1) / chunk + G;
+  if (!need || !ws || ws_bytes < need || items > 65535) return launch_f32(p, grid, st);
+  p.chunk = (int)chunk;
+  p.part = static_cast<float*>(ws);
+  grid.z = (unsigned)items;
+  RTE_TRY(launch_f32(p, grid, st));
+  hipLaunchKernelGGL(gemm_f32_reduce_kernel, dim3((unsigned)(((int64_t)M * N + 255) / 256), (unsigned)G), dim3(256), 0,
+                     st, p, 0);
+  return check_launch("gemm_f32_reduce");
+}
+
+int rte_gemm_f32_grouped(int mode, const int32_t* goff, int G, const float* A, int64_t lda, int a_t,
+                         const int32_t* a_rows, const float* a_scale, const float* B, int64_t ldb, int b_t,
+                         const int32_t* b_rows, const float* b_scale, const int64_t* b_goff, int64_t b_gstride,
+                         int64_t b_rows_gstride, float* C, int64_t ldc, const int32_t* c_rows, const int64_t* c_goff,
+                         int64_t c_gstride, int64_t c_rows_gstride, int M, int N, int K, float alpha, float beta,
+                         void* stream) {
+  return rte_gemm_f32_grouped_ws(mode, goff, G, A, lda, a_t, a_rows, a_scale, B, ldb, b_t, b_rows, b_scale, b_goff,
+                                 b_gstride, b_rows_gstride, C, ldc, c_rows, c_goff, c_gstride, c_rows_gstride, M, N, K,
+                                 alpha, beta, nullptr, 0, stream);
 }
 
 int rte_softmax_causal_f32_fwd(const float* s, int64_t rows, int S, float scale, const float* oscale, float* p,

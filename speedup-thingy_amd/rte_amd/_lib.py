@@ -146,8 +146,14 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "rte_replay_param_reduce": (_I, [_I] * 4 + [_P] * 7),
     "rte_gemm_f32": (_I, [_P, _I64, _I, _P, _P, _P, _I64, _I, _P, _P, _P, _I64, _P, _I, _I, _I, _F, _F, _I, _I,
                           _I64, _I64, _I64, _I64, _I64, _I64, _P]),
+    "rte_gemm_f32_workspace_bytes": (_SZ, [_I, _I, _I]),
+    "rte_gemm_f32_ws": (_I, [_P, _I64, _I, _P, _P, _P, _I64, _I, _P, _P, _P, _I64, _P, _I, _I, _I, _F, _F, _I, _I,
+                             _I64, _I64, _I64, _I64, _I64, _I64, _P, _SZ, _P]),
     "rte_gemm_f32_grouped": (_I, [_I, _P, _I, _P, _I64, _I, _P, _P, _P, _I64, _I, _P, _P, _P, _I64, _I64, _P, _I64,
                                   _P, _P, _I64, _I64, _I, _I, _I, _F, _F, _P]),
+    "rte_gemm_f32_grouped_workspace_bytes": (_SZ, [_I, _I, _I, _I, _I]),
+    "rte_gemm_f32_grouped_ws": (_I, [_I, _P, _I, _P, _I64, _I, _P, _P, _P, _I64, _I, _P, _P, _P, _I64, _I64, _P,
+                                     _I64, _P, _P, _I64, _I64, _I, _I, _I, _F, _F, _P, _SZ, _P]),
     "rte_softmax_causal_f32_fwd": (_I, [_P, _I64, _I, _F, _P, _P, _P, _P]),
     "rte_softmax_causal_f32_bwd": (_I, [_P, _P, _I64, _I, _F, _P, _P, _P]),
     "rte_swiglu_f32_fwd": (_I, [_P, _I64, _I, _I64, _P, _P]),

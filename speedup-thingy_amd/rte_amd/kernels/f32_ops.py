@@ -38,19 +38,24 @@ def _c32(t: torch.Tensor) -> torch.Tensor:
 def gemm(A, lda, a_t, B, ldb, b_t, C, ldc, M, N, K, *, alpha=1.0, beta=0.0, a_rows=None, a_scale=None, b_rows=None,
          b_scale=None, c_rows=None, batch=(1, 1), sA=(0, 0), sB=(0, 0), sC=(0, 0)):
     """C(m, n) = alpha sum_k A(m, k) B(n, k) + beta C(m, n) on raw fp32 buffers (see rte_gemm_f32)."""
-    call("rte_gemm_f32", ptr(A), int(lda), int(a_t), ptr(a_rows), ptr(a_scale), ptr(B), int(ldb), int(b_t), ptr(b_rows),
-         ptr(b_scale), ptr(C), int(ldc), ptr(c_rows), int(M), int(N), int(K), float(alpha), float(beta), int(batch[0]),
-         int(batch[1]), int(sA[0]), int(sA[1]), int(sB[0]), int(sB[1]), int(sC[0]), int(sC[1]), _s())
+    nb = _lib.load().rte_gemm_f32_workspace_bytes(int(M), int(N), int(K)) if a_t and batch == (1, 1) else 0
+    ws, nb = H.workspace(nb, A.device)  # a weight gradient's long reduction is split
+    call("rte_gemm_f32_ws", ptr(A), int(lda), int(a_t), ptr(a_rows), ptr(a_scale), ptr(B), int(ldb), int(b_t),
+         ptr(b_rows), ptr(b_scale), ptr(C), int(ldc), ptr(c_rows), int(M), int(N), int(K), float(alpha), float(beta),
+         int(batch[0]), int(batch[1]), int(sA[0]), int(sA[1]), int(sB[0]), int(sB[1]), int(sC[0]), int(sC[1]), ws, nb,
+         _s())
 
 
 def gemm_grouped(mode, goff, G, A, lda, a_t, B, ldb, b_t, C, ldc, M, N, K, *, alpha=1.0, beta=0.0, a_rows=None,
                  a_scale=None, b_rows=None, b_scale=None, b_goff=None, b_gstride=0, b_rows_gstride=0, c_rows=None,
                  c_goff=None, c_gstride=0, c_rows_gstride=0):
     """mode 1: group g owns rows [goff[g], goff[g+1]); mode 2: group g reduces over that k range."""
-    call("rte_gemm_f32_grouped", int(mode), ptr(goff), int(G), ptr(A), int(lda), int(a_t), ptr(a_rows), ptr(a_scale),
-         ptr(B), int(ldb), int(b_t), ptr(b_rows), ptr(b_scale), ptr(b_goff), int(b_gstride), int(b_rows_gstride),
-         ptr(C), int(ldc), ptr(c_rows), ptr(c_goff), int(c_gstride), int(c_rows_gstride), int(M), int(N), int(K),
-         float(alpha), float(beta), _s())
+    ws, nb = H.workspace(_lib.load().rte_gemm_f32_grouped_workspace_bytes(int(mode), int(M), int(N), int(K), int(G)),
+                         A.device)
+    call("rte_gemm_f32_grouped_ws", int(mode), ptr(goff), int(G), ptr(A), int(lda), int(a_t), ptr(a_rows),
+         ptr(a_scale), ptr(B), int(ldb), int(b_t), ptr(b_rows), ptr(b_scale), ptr(b_goff), int(b_gstride),
+         int(b_rows_gstride), ptr(C), int(ldc), ptr(c_rows), ptr(c_goff), int(c_gstride), int(c_rows_gstride), int(M),
+         int(N), int(K), float(alpha), float(beta), ws, nb, _s())
 
 
 def _wlayout(w: torch.Tensor):
