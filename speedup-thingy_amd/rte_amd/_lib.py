@@ -215,14 +215,23 @@ def loaded() -> bool:
         return False
 
 
+_READY = False
+
+
 def device_ready() -> bool:
-    """Library loads and a gfx950 ROCm device is visible."""
+    """Library loads and a gfx950 ROCm device is visible.  Every operator asks before it launches; a
+    process whose device was there once keeps it, so only the first yes queries the runtime (about
+    5 us a time)."""
+    global _READY
+    if _READY:
+        return True
     if not loaded() or not torch.cuda.is_available() or torch.version.hip is None:
         return False
     try:
-        return "gfx950" in torch.cuda.get_device_properties(0).gcnArchName
+        _READY = "gfx950" in torch.cuda.get_device_properties(0).gcnArchName
     except Exception:  # pragma: no cover
         return False
+    return _READY
 
 
 def last_error() -> str:
@@ -237,8 +246,17 @@ def call(name: str, *args) -> int:
     return rc
 
 
-def stream_ptr(device: torch.device | None = None) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
+def stream_ptr(device: torch.device | int | None = None) -> int:
+    """The current stream's handle on `device` (None: the current device).  Each launch asks for it:
+    the handle itself, without the Stream object torch.cuda.current_stream builds (4 us a call)."""
+    if _raw_stream is None or _raw_device is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream(device).cuda_stream
+    idx = device if isinstance(device, int) or device is None else device.index
+    return _raw_stream(_raw_device() if idx is None else idx)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

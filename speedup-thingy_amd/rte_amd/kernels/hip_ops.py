@@ -68,7 +68,7 @@ def workspace(nbytes: int, device: torch.device) -> tuple[int, int]:
     if nbytes <= 0:
         return 0, 0
     idx = device.index if device.index is not None else torch.cuda.current_device()
-    key = (idx, torch.cuda.current_stream(idx).cuda_stream)
+    key = (idx, _lib.stream_ptr(idx))
     buf = _WS.get(key)
     if buf is None or buf.numel() < nbytes:
         buf = torch.empty(((nbytes + 255) // 256) * 256, dtype=torch.uint8, device=device)
