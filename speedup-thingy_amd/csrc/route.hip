@@ -26,96 +26,24 @@ __device__ __forceinline__ bool better(float a, int ia, float b, int ib) {
   return ia < ib;
 }
 
-constexpr int kMaxPerLane = 16;  // C <= 1024
+constexpr int kMaxC = 1024;
 
-__global__ void __launch_bounds__(256) route_topk_kernel(const float* __restrict__ logits, int T, int C,
-                                                         int k, int32_t* __restrict__ ids,
-                                                         float* __restrict__ weights) {
-  const int lane = threadIdx.x & 63;
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t >= T) return;
-  const float* row = logits + (int64_t)t * C;
-  float v[kMaxPerLane];
-  bool used[kMaxPerLane];
-  const int per = (C + 63) / 64;
-#pragma unroll
-  for (int i = 0; i < kMaxPerLane; ++i) {
-    const int c = lane + 64 * i;
-    used[i] = !(i < per && c < C);
-    v[i] = used[i] ? 0.0f : row[c];
+// Small pools (C <= 64): the rank of element c is the number of elements better than it, counted
+// against every logit of the row broadcast with readlane (no LDS round trips on the critical path);
+// the k best land in LDS at their rank, then lanes j < k take the softmax over them (xor tree).
+template <bool kNaN>
+__device__ __forceinline__ int rank_row(float v, int lane, int C) {
+  int rank = 0;
+  for (int l = 0; l < C; ++l) {
+    const float vj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+    if (kNaN)
+      rank += better(vj, l, v, lane) ? 1 : 0;
+    else
+      rank += (vj > v || (vj == v && l < lane)) ? 1 : 0;
   }
-  float my_v = 0.0f;
-  int my_i = 0;
-  for (int r = 0; r < k; ++r) {
-    // lane-local best among unused
-    float bv = 0.0f;
-    int bi = 0x7fffffff;
-#pragma unroll
-    for (int i = 0; i < kMaxPerLane; ++i) {
-      if (used[i]) continue;
-      const int c = lane + 64 * i;
-      if (bi == 0x7fffffff || better(v[i], c, bv, bi)) {
-        bv = v[i];
-        bi = c;
-      }
-    }
-    // wave arg-max (butterfly: every lane ends with the winner); empty lanes carry INT_MAX
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-      const float ov = __shfl_xor(bv, off, 64);
-      const int oi = __shfl_xor(bi, off, 64);
-      if (oi != 0x7fffffff && (bi == 0x7fffffff || better(ov, oi, bv, bi))) {
-        bv = ov;
-        bi = oi;
-      }
-    }
-    if (bi != 0x7fffffff && (bi & 63) == lane) {
-#pragma unroll
-      for (int i = 0; i < kMaxPerLane; ++i)
-        if (i == (bi >> 6)) used[i] = true;
-    }
-    if (lane == r) {
-      my_v = bv;
-      my_i = bi;
-    }
-  }
-  // lane j < k holds the j-th selection; softmax over the selected logits
-  const float mx = __shfl(my_v, 0, 64);
-  const float ex = lane < k ? expf(my_v - mx) : 0.0f;
-  float denom = ex;
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) denom += __shfl_xor(denom, off, 64);
-  if (lane < k) {
-    ids[(int64_t)t * k + lane] = my_i;
-    weights[(int64_t)t * k + lane] = ex / denom;
-  }
+  return rank;
 }
 
-// Small pools (C <= 64 * PER): the rank of element c is the number of elements better
-// than it, counted against every logit of the row broadcast with readlane (no LDS round
-// trips on the critical path); the k best land in LDS at their rank, then lanes j < k
-// finish exactly like route_topk_kernel (same selection values, same softmax order).
-template <int PER, bool kNaN>
-__device__ __forceinline__ void rank_row(const float (&v)[PER], int lane, int C, int (&rank)[PER]) {
-#pragma unroll
-  for (int q = 0; q < PER; ++q) {
-    const int nq = C - 64 * q < 64 ? C - 64 * q : 64;
-    for (int l = 0; l < nq; ++l) {
-      const float vj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[q]), l));
-      const int j = 64 * q + l;
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int c = lane + 64 * i;
-        if (kNaN)
-          rank[i] += better(vj, j, v[i], c) ? 1 : 0;
-        else
-          rank[i] += (vj > v[i] || (vj == v[i] && j < c)) ? 1 : 0;
-      }
-    }
-  }
-}
-
-template <int PER>
 __global__ void __launch_bounds__(256) route_topk_rank_kernel(const float* __restrict__ logits, int T, int C, int k,
                                                               int32_t* __restrict__ ids,
                                                               float* __restrict__ weights) {
@@ -125,27 +53,11 @@ __global__ void __launch_bounds__(256) route_topk_rank_kernel(const float* __res
   const int t = blockIdx.x * 4 + wave;
   const bool live = t < T;  // no early exit: every wave reaches the barrier below
   const float* row = logits + (int64_t)(live ? t : 0) * C;
-  float v[PER];
-  int rank[PER];
-  bool nan_here = false;
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int c = lane + 64 * i;
-    v[i] = (live && c < C) ? row[c] : 0.0f;
-    rank[i] = 0;
-    nan_here |= v[i] != v[i];
-  }
-  if (__ballot(nan_here) != 0)
-    rank_row<PER, true>(v, lane, C, rank);
-  else
-    rank_row<PER, false>(v, lane, C, rank);
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int c = lane + 64 * i;
-    if (c < C && rank[i] < k) {
-      sel_v[wave][rank[i]] = v[i];
-      sel_i[wave][rank[i]] = c;
-    }
+  const float v = (live && lane < C) ? row[lane] : 0.0f;
+  const int rank = __ballot(v != v) != 0 ? rank_row<true>(v, lane, C) : rank_row<false>(v, lane, C);
+  if (lane < C && rank < k) {
+    sel_v[wave][rank] = v;
+    sel_i[wave][rank] = lane;
   }
   __syncthreads();
   if (!live) return;
@@ -296,38 +208,12 @@ __global__ void __launch_bounds__(256) pack_scatter_kernel(const int32_t* __rest
   }
 }
 
-// One lane per token: the wave's 64 rows are staged in LDS (row pitch C + 1: lanes reading
-// the same column hit distinct banks), each lane inserts its row's logits in index order into
-// a sorted top-K list (the element carried down by an insertion is compared with the full order,
-// index ascending on equal values), then the softmax over the k selected logits is summed with the xor tree the
-// wave-per-token kernel's butterfly forms, so both kernels give identical results.
-template <int K, bool kNaN>
-__device__ __forceinline__ void insert_row(const float* rowl, int C, float (&tv)[K], int (&ti)[K]) {
-  for (int c = 0; c < C; ++c) {
-    float v = rowl[c];
-    int i = c;
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-      bool take;
-      if (kNaN)
-        take = ti[j] < 0 || better(v, i, tv[j], ti[j]);
-      else  // a carried (displaced) element meets later equal values: index ascending
-        take = ti[j] < 0 || v > tv[j] || (v == tv[j] && i < ti[j]);
-      const float ov = tv[j];
-      const int oi = ti[j];
-      tv[j] = take ? v : ov;
-      ti[j] = take ? i : oi;
-      v = take ? ov : v;
-      i = take ? oi : i;
-    }
-  }
-}
-
 // softmax over the k selected logits (sorted, tv[0] the largest) summed with the xor tree the
-// wave-per-token kernel's butterfly forms, then the k ids and weights stored
+// wave-per-token kernel's butterfly forms, then the k ids and weights stored (with lanes > 1, by
+// `lanes` lanes that all hold the list: lane `me` stores j = me, me + lanes, ...)
 template <int K>
 __device__ __forceinline__ void topk_softmax_store(const float (&tv)[K], const int (&ti)[K], int k, int32_t* ids,
-                                                   float* weights) {
+                                                   float* weights, int me = 0, int lanes = 1) {
   float ex[K], sm[K];
 #pragma unroll
   for (int j = 0; j < K; ++j) {
@@ -344,56 +230,10 @@ __device__ __forceinline__ void topk_softmax_store(const float (&tv)[K], const i
   }
 #pragma unroll
   for (int j = 0; j < K; ++j)
-    if (j < k) {
+    if (j < k && (j & (lanes - 1)) == me) {
       ids[j] = ti[j];
       weights[j] = ex[j] / sm[0];
     }
-}
-
-template <int K>
-__global__ void __launch_bounds__(64) route_topk_lanes_kernel(const float* __restrict__ logits, int T, int C, int k,
-                                                              int32_t* __restrict__ ids,
-                                                              float* __restrict__ weights) {
-  extern __shared__ float rows[];  // [64][C + 1]
-  const int lane = threadIdx.x;
-  const int t0 = blockIdx.x * 64;
-  const int nt = T - t0 < 64 ? T - t0 : 64;
-  const int P = C + 1;
-  const float* src = logits + (int64_t)t0 * C;
-  bool nan_here = false;
-  if ((C & 3) == 0) {  // 16-byte loads: consecutive lanes, consecutive logits
-    for (int e = 4 * lane; e < nt * C; e += 256) {
-      const float4 x = *reinterpret_cast<const float4*>(src + e);
-      nan_here |= x.x != x.x || x.y != x.y || x.z != x.z || x.w != x.w;
-      const int r = e / C, c = e - r * C;  // C % 4 == 0: the four stay in one row
-      float* d = rows + r * P + c;
-      d[0] = x.x;
-      d[1] = x.y;
-      d[2] = x.z;
-      d[3] = x.w;
-    }
-  } else {
-    for (int e = lane; e < nt * C; e += 64) {
-      const float x = src[e];
-      nan_here |= x != x;
-      const int r = e / C, c = e - r * C;
-      rows[r * P + c] = x;
-    }
-  }
-  __syncthreads();
-  if (lane >= nt) return;
-  float tv[K];
-  int ti[K];
-#pragma unroll
-  for (int j = 0; j < K; ++j) {
-    tv[j] = 0.0f;
-    ti[j] = -1;  // empty: below every logit
-  }
-  if (__ballot(nan_here) != 0)
-    insert_row<K, true>(rows + lane * P, C, tv, ti);
-  else
-    insert_row<K, false>(rows + lane * P, C, tv, ti);
-  topk_softmax_store<K>(tv, ti, k, ids + (int64_t)(t0 + lane) * k, weights + (int64_t)(t0 + lane) * k);
 }
 
 // ---- pack of per-sample route lists (the banked FFN: every token of sample b visits the
@@ -637,64 +477,62 @@ __global__ void __launch_bounds__(256) combine_kernel(const bf16* __restrict__ r
   store8<OutT>(out + (int64_t)t * d + c, acc);
 }
 
+constexpr int kRouteBwdCols = 1024;  // columns of a row held in LDS at a time
+
 // Routing-weight gradient: weights are softmax over the k selected logits, so
 // dlogit_j = w_j * (dw_j - sum_i w_i dw_i); everything else in the row is 0.
-// One thread per logit (t, c): the per-token sum s = sum_j w_j dw_j in j order, then the
-// gradient of the j that selected c (the last one, if an id repeats), zero elsewhere.  Rows
-// are written whole and coalesced.
+// One wave per token row: lane j holds selection j, the sum runs in j order, and the row leaves
+// whole through LDS (the last j that selected a cluster writes it).  Bound by the row writes; with a
+// thread per logit, each rereading the token's k selections, T 16384, C 256, k 16 took 42 us.
 __global__ void __launch_bounds__(256) route_bwd_kernel(const int32_t* __restrict__ ids,
                                                         const float* __restrict__ w,
                                                         const float* __restrict__ dw_slot,
                                                         const int32_t* __restrict__ slot_of_pair, int T,
                                                         int C, int k, bf16* __restrict__ dlogits,
                                                         float* __restrict__ dlogits_f32) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (int64_t)T * C) return;
-  const int64_t t = e / C;
-  const int c = (int)(e - t * C);
-  const int32_t* it = ids + t * k;
-  const float* wt = w + t * k;
-  const int32_t* st = slot_of_pair + t * k;
-  float s = 0.0f, wsel = 0.0f, dsel = 0.0f;
-  bool hit = false;
-  if (k <= 16) {
-    // the row's slots, weights and ids first, then the slot gradients: two memory latencies
-    int sl[16], id[16];
-    float wv[16], dv[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      sl[j] = j < k ? st[j] : -1;
-      wv[j] = j < k ? wt[j] : 0.0f;
-      id[j] = j < k ? it[j] : -1;
-    }
-#pragma unroll
-    for (int j = 0; j < 16; ++j) dv[j] = sl[j] >= 0 ? dw_slot[sl[j]] : 0.0f;
-#pragma unroll
-    for (int j = 0; j < 16; ++j)
-      if (j < k) {
-        s += wv[j] * dv[j];
-        if (id[j] == c) {
-          hit = true;
-          wsel = wv[j];
-          dsel = dv[j];
-        }
-      }
-  } else {
-    for (int j = 0; j < k; ++j) {
-      const int slot = st[j];
-      const float dw = slot >= 0 ? dw_slot[slot] : 0.0f;
-      const float wj = wt[j];
-      s += wj * dw;
-      if (it[j] == c) {
-        hit = true;
-        wsel = wj;
-        dsel = dw;
-      }
-    }
+  __shared__ __align__(16) float row_lds[4][kRouteBwdCols];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t t = (int64_t)blockIdx.x * 4 + wave;
+  float* row = row_lds[wave];
+  if (t >= T) return;  // rows are private to their wave: no workgroup barrier below
+  int id = -1;
+  float wv = 0.0f, dv = 0.0f;
+  if (lane < k) {
+    const int slot = slot_of_pair[t * k + lane];
+    id = ids[t * k + lane];
+    wv = w[t * k + lane];
+    dv = slot >= 0 ? dw_slot[slot] : 0.0f;
   }
-  const float g = hit ? wsel * (dsel - s) : 0.0f;
-  if (dlogits) dlogits[e] = f2bf(g);
-  if (dlogits_f32) dlogits_f32[e] = g;
+  float s = 0.0f;
+  bool last = lane < k;
+  for (int j = 0; j < k; ++j) {
+    s += __shfl(wv, j, 64) * __shfl(dv, j, 64);
+    if (__shfl(id, j, 64) == id && j > lane) last = false;
+  }
+  auto fence = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  for (int c0 = 0; c0 < C; c0 += kRouteBwdCols) {
+    const int n = C - c0 < kRouteBwdCols ? C - c0 : kRouteBwdCols;
+    fence();  // the previous columns have left
+    for (int c = lane; c < n; c += 64) row[c] = 0.0f;
+    fence();
+    if (last && id >= c0 && id < c0 + n) row[id - c0] = wv * (dv - s);
+    fence();
+    if (dlogits) {
+      bf16* d = dlogits + t * C + c0;
+      if ((C & 1) == 0 && ((uintptr_t)dlogits & 3) == 0) {
+        for (int c = 2 * lane; c < n; c += 128)
+          *reinterpret_cast<uint32_t*>(d + c) = pack_bf2(row[c], row[c + 1]);
+      } else {
+        for (int c = lane; c < n; c += 64) d[c] = f2bf(row[c]);
+      }
+    }
+    if (dlogits_f32)
+      for (int c = lane; c < n; c += 64) dlogits_f32[t * C + c0 + c] = row[c];
+  }
 }
 
 // ---- router GEMM + top-k + pack in two launches (C % 32 == 0, C <= 128, d % 64 == 0) ----
@@ -752,6 +590,81 @@ __device__ __forceinline__ void rt_sort(uint64_t (&key)[N]) {
           key[j] = sw ? x : y;
         }
       }
+}
+
+// Merges the sorted list b into a: the K largest keys of both, sorted descending.
+template <int K>
+__device__ __forceinline__ void rt_merge(uint64_t (&a)[K], const uint64_t (&b)[K]) {
+#pragma unroll
+  for (int i = 0; i < K; ++i)
+    if (b[K - 1 - i] > a[i]) a[i] = b[K - 1 - i];  // a bitonic sequence of the K largest
+#pragma unroll
+  for (int stride = K / 2; stride > 0; stride >>= 1)
+#pragma unroll
+    for (int i = 0; i < K; ++i)
+      if (!(i & stride)) {
+        const uint64_t x = a[i], y = a[i + stride];
+        a[i] = y > x ? y : x;
+        a[i + stride] = y > x ? x : y;
+      }
+}
+
+// Eight lanes per token: each sorts its share of the row (K keys at a time, merged into a running
+// list of K), then the eight lists merge over xor partners, so every lane ends with the row's K best
+// in order.  Bound by its compare-exchanges, which need no LDS and no rounds over the wave: C 256,
+// k 16, T 16384 took 157 us as 16 rounds of a wave arg-max.  The softmax sums with the xor tree of
+// topk_softmax_store.
+template <int K>
+__global__ void __launch_bounds__(256) route_topk_oct_kernel(const float* __restrict__ logits, int T, int C, int k,
+                                                             int32_t* __restrict__ ids,
+                                                             float* __restrict__ weights) {
+  const int o = threadIdx.x & 7;
+  const int64_t t = (int64_t)blockIdx.x * 32 + (threadIdx.x >> 3);
+  const float* row = logits + (t < T ? t : T - 1) * (int64_t)C;
+  const int quads = (C + 31) / 32;  // groups of four logits per lane
+  const bool vec = (C & 3) == 0 && ((uintptr_t)logits & 15) == 0;
+  uint64_t best[K];
+  for (int q0 = 0; q0 < quads; q0 += K / 4) {
+    uint64_t key[K];
+#pragma unroll
+    for (int q = 0; q < K / 4; ++q) {
+      const int c = ((q0 + q) * 8 + o) * 4;
+      float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (vec && c < C) {
+        const float4 x = *reinterpret_cast<const float4*>(row + c);
+        v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (c + j < C) v[j] = row[c + j];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) key[4 * q + j] = c + j < C ? rt_key(v[j], c + j) : 0;
+    }
+    rt_sort<K>(key);
+    if (q0 == 0) {
+#pragma unroll
+      for (int i = 0; i < K; ++i) best[i] = key[i];
+    } else {
+      rt_merge<K>(best, key);
+    }
+  }
+#pragma unroll
+  for (int off = 1; off <= 4; off <<= 1) {
+    uint64_t other[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) other[i] = rt_shfl_xor(best[i], off);
+    rt_merge<K>(best, other);
+  }
+  if (t >= T) return;
+  float tv[K];
+  int ti[K];
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    tv[j] = rt_key_val(best[j]);
+    ti[j] = rt_key_idx(best[j]);
+  }
+  topk_softmax_store<K>(tv, ti, k, ids + t * k, weights + t * k, o, 8);
 }
 
 template <int CB, int K>
@@ -991,26 +904,23 @@ __global__ void __launch_bounds__(256) pack_place_kernel(const int32_t* __restri
 }  // namespace
 
 int route_topk(const float* logits, int T, int C, int k, int32_t* ids, float* weights, hipStream_t s) {
-  RTE_REQUIRE(T >= 0 && C >= 1 && C <= 64 * kMaxPerLane, "route_topk: C must be in [1, 1024]");
+  RTE_REQUIRE(T >= 0 && C >= 1 && C <= kMaxC, "route_topk: C must be in [1, 1024]");
   RTE_REQUIRE(k >= 1 && k <= 16 && k <= C, "route_topk: k must be in [1, min(16, C)]");
   if (T == 0) return 0;
-  if (T >= 16384 && C <= 128) {
-    const size_t lds = (size_t)64 * (C + 1) * sizeof(float);
-    if (k <= 8)
-      hipLaunchKernelGGL(route_topk_lanes_kernel<8>, dim3((T + 63) / 64), dim3(64), lds, s, logits, T, C, k, ids,
-                         weights);
-    else
-      hipLaunchKernelGGL(route_topk_lanes_kernel<16>, dim3((T + 63) / 64), dim3(64), lds, s, logits, T, C, k, ids,
-                         weights);
+  // Few short rows: one wave per row counts ranks with less latency (C 64, k 16: T 1024 5.3 us
+  // against 11.2, T 8192 10.0 against 11.6, T 16384 20 against 13.5; k 8: T 1024 5.4 against 6.1, T
+  // 8192 10.0 against 6.3); everything else in octets (C 256, k 16, T 16384: 17.9 us).
+  if (C <= 64 && T <= (k > 8 ? 8192 : 2048)) {
+    hipLaunchKernelGGL(route_topk_rank_kernel, dim3((T + 3) / 4), dim3(256), 0, s, logits, T, C, k, ids, weights);
     return check_launch("route_topk");
   }
-  const dim3 grid((T + 3) / 4);
-  if (C <= 64)
-    hipLaunchKernelGGL(route_topk_rank_kernel<1>, grid, dim3(256), 0, s, logits, T, C, k, ids, weights);
-  else if (C <= 128)
-    hipLaunchKernelGGL(route_topk_rank_kernel<2>, grid, dim3(256), 0, s, logits, T, C, k, ids, weights);
+  const dim3 grid((unsigned)((T + 31) / 32));
+  if (k <= 4)
+    hipLaunchKernelGGL(route_topk_oct_kernel<4>, grid, dim3(256), 0, s, logits, T, C, k, ids, weights);
+  else if (k <= 8)
+    hipLaunchKernelGGL(route_topk_oct_kernel<8>, grid, dim3(256), 0, s, logits, T, C, k, ids, weights);
   else
-    hipLaunchKernelGGL(route_topk_kernel, grid, dim3(256), 0, s, logits, T, C, k, ids, weights);
+    hipLaunchKernelGGL(route_topk_oct_kernel<16>, grid, dim3(256), 0, s, logits, T, C, k, ids, weights);
   return check_launch("route_topk");
 }
 
@@ -1122,9 +1032,8 @@ int route_bwd(const int32_t* ids, const float* w, const float* dw_slot, const in
               int C, int k, bf16* dlogits, float* dlogits_f32, hipStream_t s) {
   RTE_REQUIRE(k >= 1 && k <= 16, "route_bwd: k must be in [1, 16]");
   if (T == 0) return 0;
-  const int64_t n = (int64_t)T * C;
-  hipLaunchKernelGGL(route_bwd_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ids, w, dw_slot,
-                     slot_of_pair, T, C, k, dlogits, dlogits_f32);
+  hipLaunchKernelGGL(route_bwd_kernel, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, s, ids, w, dw_slot, slot_of_pair,
+                     T, C, k, dlogits, dlogits_f32);
   return check_launch("route_bwd");
 }
 
