@@ -890,16 +890,15 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(GemmArgs p, EpiFlags
   store_chunk<4>(p.epi, 0, m, n, p.N, v, fl.vec);
 }
 
-// Chunk of a GROUP_K group: about half the mean group size, at least 256 rows, so a long
-// reduction is shared by a few workgroups (the fp32 partials cost less than the serial k
-// steps: measured on the cfg3 cluster-pool weight gradients) and a dominant group by many.
-int groupk_chunk(int K, int G) {
-  static const int env = [] {  // RTE_GK_CHUNK: fixed chunk for diagnostics
-    const char* v = getenv("RTE_GK_CHUNK");
-    return v && *v ? atoi(v) : 0;
-  }();
-  if (env >= 64) return (env + 63) / 64 * 64;
-  int64_t c = ((int64_t)K + G - 1) / (G > 0 ? G : 1) / 2;
+// Chunk of a GROUP_K group.  Few output tiles over all groups (fewer than 4 workgroups per CU): about
+// half the mean group size, at least 256 rows, so a long reduction is shared by a few workgroups (the
+// fp32 partials cost less than the serial k steps: 64 groups of 1024 rows, 64 x 512 outputs).  With
+// enough tiles the partials only cost: chunks of four mean groups still cut a dominant group (256
+// groups of 1024 rows, 128 x 1024 outputs: the partials' sum alone took 102 us).
+int groupk_chunk(int M, int N, int K, int G) {
+  const int64_t mean = ((int64_t)K + G - 1) / (G > 0 ? G : 1);
+  const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * G;
+  int64_t c = tiles >= 1024 ? 4 * mean : mean / 2;
   if (c < 256) c = 256;
   return (int)((c + 63) / 64 * 64);
 }
@@ -945,7 +944,7 @@ int launch_cfg(const GemmArgs& p0, hipStream_t stream, void* ws, size_t ws_bytes
     if (EPI == EPI_STORE && ws && p.N % 4 == 0 && p.G >= 1) {
       const size_t need = gemm_groupk_bytes(p.M, p.N, p.K, p.G);
       if (need > 0 && ws_bytes >= need) {
-        const int chunk = groupk_chunk(p.K, p.G);
+        const int chunk = groupk_chunk(p.M, p.N, p.K, p.G);
         p.gk_chunk = chunk;
         p.gk_first = static_cast<int32_t*>(ws);
         p.gk_part = reinterpret_cast<float*>(static_cast<char*>(ws) + groupk_first_bytes(p.G));
@@ -1235,7 +1234,7 @@ bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15) == 0; }
 
 size_t gemm_groupk_bytes(int M, int N, int K, int G) {
   if (M <= 0 || N <= 0 || K <= 0 || G <= 0) return 0;
-  const int chunk = groupk_chunk(K, G);
+  const int chunk = groupk_chunk(M, N, K, G);
   const size_t items = (size_t)((K + chunk - 1) / chunk) + (size_t)G;
   return groupk_first_bytes(G) + items * (size_t)M * N * sizeof(float);
 }
