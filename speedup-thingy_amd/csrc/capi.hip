@@ -168,10 +168,15 @@ Operand from_layout(const void* p, const int64_t* L) {
 
 // Weight gradients of the grouped SwiGLU (grouped-K reductions over each cluster's slots): dWug from
 // x[tok] and dUG, dWd from zw and dout[tok], in the parameters' layout (w_t = 0) or transposed.
-int pool_wgrad(const void* dout, const void* x, int d, const int32_t* offsets, int G, int n, int P,
+int pool_wgrad(const void* dout, const void* x, int T, int d, const int32_t* offsets, int G, int n, int P,
                const int32_t* tok_of_slot, int64_t ld_wd, const void* zw, const void* dug, float* dwug, float* dwd,
                int w_t, float beta, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   const int dff = G * n;
+  // rows of x / dout gathered by token, rows of dug / zw one per slot
+  auto set_extents = [&](GemmArgs& p) {
+    p.a.extent = (p.a.rows ? (int64_t)T : (int64_t)P) * p.a.ld * 2;
+    p.b.extent = (p.b.rows ? (int64_t)T : (int64_t)P) * p.b.ld * 2;
+  };
   if (w_t) {
     // dWug^T[:, ilv(g*2n + c)] = sum_slot x[tok(slot), :] dUG[slot, c]   ([d, 2F]: columns [up F | gate F])
     GemmArgs p;
@@ -192,6 +197,7 @@ int pool_wgrad(const void* dout, const void* x, int d, const int32_t* offsets, i
     p.epi.c_gstride = 2 * n;
     p.epi.c_col_ilv = dff;
     p.epi.beta = beta;
+    set_extents(p);
     RTE_TRY(gemm_launch(p, EPI_STORE, stream, workspace, workspace_bytes));
   } else {
     // dWug_g[c, :] = sum_slot dUG[slot, c] x[tok(slot), :]
@@ -213,6 +219,7 @@ int pool_wgrad(const void* dout, const void* x, int d, const int32_t* offsets, i
     p.epi.c_growstride = 2 * n;
     p.epi.c_ilv = dff;
     p.epi.beta = beta;
+    set_extents(p);
     RTE_TRY(gemm_launch(p, EPI_STORE, stream, workspace, workspace_bytes));
   }
   if (w_t) {
@@ -234,6 +241,7 @@ int pool_wgrad(const void* dout, const void* x, int d, const int32_t* offsets, i
     p.epi.c_f32 = 1;
     p.epi.c_growstride = n;
     p.epi.beta = beta;
+    set_extents(p);
     RTE_TRY(gemm_launch(p, EPI_STORE, stream, workspace, workspace_bytes));
   } else {
     // dWd[:, g*n + j] = sum_slot dout[tok(slot), :] zw[slot, j]
@@ -254,6 +262,7 @@ int pool_wgrad(const void* dout, const void* x, int d, const int32_t* offsets, i
     p.epi.c_f32 = 1;
     p.epi.c_gstride = n;
     p.epi.beta = beta;
+    set_extents(p);
     RTE_TRY(gemm_launch(p, EPI_STORE, stream, workspace, workspace_bytes));
   }
   return 0;
@@ -401,6 +410,8 @@ int rte_grouped_swiglu_fwd(const void* x, int T, int d, const int32_t* offsets, 
     p.epi.z = B16(zw);
     p.epi.ld_z = n;
     p.epi.row_scale = w_of_slot;
+    p.a.extent = (int64_t)T * d * 2;
+    p.b.extent = (int64_t)2 * dff * d * 2;
     RTE_TRY(gemm_launch(p, EPI_SWIGLU_FWD, S(stream)));
   }
   // stage 2: y_pairs[pair] = zw @ W_down_g    (B(n=dcol, k=j) = wd[dcol*ld_wd + g*n + j])
@@ -455,6 +466,8 @@ int rte_grouped_swiglu_bwd(const void* dout, const void* x, int T, int d, const 
     p.epi.ld_ug = 2 * n;
     p.epi.row_scale = w_of_slot;
     p.epi.dw_row = dw_slot;
+    p.a.extent = (int64_t)T * d * 2;
+    p.b.extent = ((int64_t)(d - 1) * ld_wd + dff) * 2;
     RTE_TRY(gemm_launch(p, EPI_SWIGLU_BWD, S(stream)));
   }
   if (P > 0) {
@@ -477,7 +490,7 @@ int rte_grouped_swiglu_bwd(const void* dout, const void* x, int T, int d, const 
     p.epi.c_rows = pair_of_slot;
     RTE_TRY(gemm_launch(p, EPI_STORE, S(stream)));
   }
-  RTE_TRY(pool_wgrad(dout, x, d, offsets, G, n, P, tok_of_slot, ld_wd, zw, dug, dwug, dwd, w_t, beta, workspace,
+  RTE_TRY(pool_wgrad(dout, x, T, d, offsets, G, n, P, tok_of_slot, ld_wd, zw, dug, dwug, dwd, w_t, beta, workspace,
                      workspace_bytes, S(stream)));
   (void)T;
   (void)pair_of_slot;
@@ -510,7 +523,7 @@ int rte_grouped_swiglu_fused_bwd(const void* dout, const void* x, int T, int d, 
   (void)T;
   RTE_TRY(pool_fused_bwd(B16(dout), d, offsets, G, n, P, tok_of_slot, pair_of_slot, w_of_slot, B16(wug), B16(wd),
                          ld_wd, B16(ug), B16(dug), dw_slot, B16(dx_pairs), S(stream)));
-  return pool_wgrad(dout, x, d, offsets, G, n, P, tok_of_slot, ld_wd, zw, dug, dwug, dwd, w_t, beta, workspace,
+  return pool_wgrad(dout, x, T, d, offsets, G, n, P, tok_of_slot, ld_wd, zw, dug, dwug, dwd, w_t, beta, workspace,
                     workspace_bytes, S(stream));
 }
 

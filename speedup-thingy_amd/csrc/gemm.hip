@@ -893,12 +893,16 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(GemmArgs p, EpiFlags
 // Chunk of a GROUP_K group.  Few output tiles over all groups (fewer than 4 workgroups per CU): about
 // half the mean group size, at least 256 rows, so a long reduction is shared by a few workgroups (the
 // fp32 partials cost less than the serial k steps: 64 groups of 1024 rows, 64 x 512 outputs).  With
-// enough tiles the partials only cost: chunks of four mean groups still cut a dominant group (256
+// enough tiles the partials only cost: chunks of two to four mean groups still cut a dominant group (256
 // groups of 1024 rows, 128 x 1024 outputs: the partials' sum alone took 102 us).
 int groupk_chunk(int M, int N, int K, int G) {
   const int64_t mean = ((int64_t)K + G - 1) / (G > 0 ? G : 1);
   const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * G;
-  int64_t c = tiles >= 1024 ? 4 * mean : mean / 2;
+  int64_t c = mean / 2;
+  if (tiles >= 1024) {
+    c = 4 * mean < kTileGroupChunk ? 4 * mean : kTileGroupChunk;
+    if (c < 2 * mean) c = 4 * mean;
+  }
   if (c < 256) c = 256;
   return (int)((c + 63) / 64 * 64);
 }
@@ -1215,6 +1219,40 @@ bool tile_ok(GemmArgs& p, int epi_kind) {
   return p.a_bytes && p.b_bytes;
 }
 
+// Grouped products on the tile kernels: whole 64-k stages of known extent (GROUP_M), or reductions
+// over layout-T rows with at most one gathered operand, in chunks (GROUP_K).
+bool tile_group_ok(GemmArgs& p, int epi_kind, void* ws, size_t ws_bytes) {
+  const int64_t lim = (int64_t)1 << 31;
+  for (const Operand* o : {&p.a, &p.b})
+    if (o->cdiv || o->rdiv || o->extent <= 0 || o->extent >= lim) return false;
+  p.a_bytes = (uint32_t)p.a.extent;
+  p.b_bytes = (uint32_t)p.b.extent;
+  if (p.mode == MODE_GROUP_M) {
+    if (p.K % 64 != 0 || p.K < kTileMinK || p.a_t || p.a.ilv || p.b.rows || p.a_koff2) return false;
+    if (epi_kind == EPI_SWIGLU_FWD) return !p.b_t;
+    return epi_kind == EPI_SWIGLU_BWD && p.b_t && p.N > 32 && p.N <= 64 && !p.b.ilv && !p.b.growstride;
+  }
+  if (p.mode != MODE_GROUP_K || epi_kind != EPI_STORE || !p.a_t || !p.b_t || p.K <= 0) return false;
+  if (p.a.ilv || p.b.ilv || p.a.gstride || p.b.gstride || p.a.growstride || p.b.growstride) return false;
+  if ((p.a.rows && p.b.rows) || p.M < 64 || p.N < 64 || p.N % 4 != 0 || !ws) return false;
+  const int chunk = groupk_chunk(p.M, p.N, p.K, p.G);
+  if (chunk > kTileGroupChunk || ws_bytes < gemm_groupk_bytes(p.M, p.N, p.K, p.G)) return false;
+  p.gk_chunk = chunk;
+  p.gk_first = static_cast<int32_t*>(ws);
+  p.gk_part = reinterpret_cast<float*>(static_cast<char*>(ws) + groupk_first_bytes(p.G));
+  return true;
+}
+
+int launch_group_tiles(const GemmArgs& p, int epi_kind, hipStream_t stream, int vec) {
+  RTE_TRY(gemm_tile_group_launch(p, epi_kind, stream, vec));
+  if (p.mode != MODE_GROUP_K) return 0;
+  const int64_t n = (int64_t)p.M * (p.N / 4);
+  RTE_REQUIRE(n < ((int64_t)1 << 31) && p.G <= 65535, "gemm: grouped-K output too large");
+  hipLaunchKernelGGL(groupk_reduce_kernel, dim3((unsigned)((n + 255) / 256), (unsigned)p.G), dim3(256), 0, stream, p,
+                     EpiFlags{vec});
+  return check_launch("gemm_groupk_reduce");
+}
+
 // The tile kernels, and the sum of the partials where they split the reduction.
 int launch_tiles(const GemmArgs& p, int epi_kind, hipStream_t stream, int vec, void* ws, size_t ws_bytes) {
   GemmArgs q = p;
@@ -1288,6 +1326,7 @@ int gemm_launch(const GemmArgs& p, int epi_kind, hipStream_t stream, void* ws, s
   }
 
   GemmArgs q = p;
+  if (tile_group_ok(q, epi_kind, ws, ws_bytes)) return launch_group_tiles(q, epi_kind, stream, vec);
   const bool tiles = tile_ok(q, epi_kind);
   switch (epi_kind) {
     case EPI_STORE: {

@@ -31,6 +31,7 @@ struct Operand {
   int32_t ilv = 0;                // >0: SwiGLU interleave, row r -> (r%64<32 ? 0 : ilv) + (r/64)*32 + r%32
   int32_t rdiv = 0;               // 0: plain rows, else (power of 2) row r -> (r/rdiv)*rs_hi + (r%rdiv)*ld
   int64_t rs_hi = 0;
+  int64_t extent = 0;             // bytes from ptr to the last element's end (0: not known)
   int32_t cdiv = 0;               // 0: plain cols, else (power of 2) col c -> (c/cdiv)*cs_hi + c%cdiv
   int64_t cs_hi = 0;
 };

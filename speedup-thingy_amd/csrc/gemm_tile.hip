@@ -21,8 +21,8 @@ namespace {
 
 // One operand: R tile rows (the output index) by BK k per stage.  Layout N (k contiguous): LDS
 // rows are output rows of BK k, 16-byte chunk c at c ^ dl_swz(row).  Layout T (output index
-// contiguous): LDS rows are k rows of R elements, chunk c at c ^ 4 (k % 4), so the four k rows of
-// a ds_read_b64_tr_b16 sit in distinct 64-byte windows.
+// contiguous): LDS rows are k rows of R elements, chunk c at c ^ tswz(k), so the four k rows of a
+// ds_read_b64_tr_b16 sit in distinct 64-byte windows of the 256 bytes the banks cover.
 template <int R, int NT, int BK, bool T>
 struct TileOperand {
   static constexpr int ROWB = T ? R * 2 : BK * 2;
@@ -30,23 +30,28 @@ struct TileOperand {
   static constexpr int BYTES = R * BK * 2;
   static constexpr int INS = BYTES / 16 / NT;
   static_assert(INS >= 1 && BYTES == INS * 16 * NT, "whole 16-byte loads per thread");
-  static_assert(!T || CPR >= 16, "layout-T tiles hold at least 128 columns");
+  static_assert(!T || CPR >= 8, "layout-T tiles hold at least 64 columns");
 
   uint32_t off[INS];  // byte offset of this thread's loads in the operand (under 2^31: host check)
 
-  __device__ __forceinline__ void init(const Operand& o, int i0, int ilim, int tid) {
+  __device__ __forceinline__ static int tswz(int krow) { return CPR >= 16 ? (krow & 3) * 4 : ((krow >> 1) & 1) * 4; }
+  __device__ __forceinline__ static int krow(int u, int tid) { return (u * NT + tid) / CPR; }
+
+  // group: the operand's group (row and element shifts); rows_later: layout T, leave the k row out
+  __device__ __forceinline__ void init(const Operand& o, int group, int i0, int ilim, int tid, bool rows_later) {
+    const int64_t shift = (int64_t)group * o.growstride, base = (int64_t)group * o.gstride;
 #pragma unroll
     for (int u = 0; u < INS; ++u) {
       const int q = u * NT + tid, row = q / CPR, pc = q % CPR;
       if constexpr (!T) {
         int i = i0 + row;
         if (i >= ilim) i = ilim - 1;  // rows past the end re-read the last one; never stored
-        off[u] = (uint32_t)(row_off(o, i) + (pc ^ dl_swz<CPR>(row)) * 8) * 2;
+        off[u] = (uint32_t)(base + row_off(o, i + shift) + (pc ^ dl_swz<CPR>(row)) * 8) * 2;
       } else {
-        int i = i0 + (pc ^ ((row & 3) * 4)) * 8;
+        int i = i0 + (pc ^ tswz(row)) * 8;
         if (i + 8 > ilim) i = ilim - 8;  // layout-T extents are multiples of 8
         const int64_t krow = (o.ilv && row >= 32) ? (int64_t)(row - 32) + o.ilv : row;
-        off[u] = (uint32_t)(krow * o.ld + i) * 2;
+        off[u] = (uint32_t)(base + (rows_later ? 0 : krow * o.ld) + i) * 2;
       }
     }
   }
@@ -64,7 +69,7 @@ struct TileOperand {
       const int g = lane >> 4, s = lane & 15;
       const int kr = 8 * (g >> 1) + (s >> 2);
       const int col = rb + 32 * b + 16 * (g & 1) + 4 * (s & 3);
-      return (kr + 16 * ks) * ROWB + (((col >> 3) ^ ((s >> 2) * 4)) << 4) + (col & 7) * 2;
+      return (kr + 16 * ks) * ROWB + (((col >> 3) ^ tswz(kr)) << 4) + (col & 7) * 2;
     }
   }
   __device__ __forceinline__ static bf16x8_v frag(const unsigned char* at) {
@@ -83,15 +88,78 @@ constexpr int kBand = 4;  // tile rows walked together (4, 8 and 16 are within 2
 constexpr int kPatchPitch = 68;  // floats per row of a wave's 32 x 64 output patch
 constexpr int kPatchBytes = 32 * kPatchPitch * 4;
 
-template <int BM, int BN, int WM, int WN, int BK, int ST>
+constexpr int kIdxRows = kTileGroupChunk;  // gathered rows of a grouped reduction held in LDS
+
+template <int BM, int BN, int WM, int WN, int BK, int ST, int MODE>
 constexpr int tile_wgs() {
-  constexpr int by_lds = 163840 / (ST * (BM + BN) * BK * 2);
+  constexpr int by_lds = 163840 / (ST * (BM + BN) * BK * 2 + (MODE == MODE_GROUP_K ? kIdxRows * 4 : 0));
   constexpr int by_regs = ((BM / WM) * (BN / WN) >= 128 * 128 ? 4 : (BM / WM) * (BN / WN) >= 128 * 64 ? 8 : 16) / (WM * WN);
   return by_lds < by_regs ? by_lds : by_regs;
 }
 
-template <int BM, int BN, int WM, int WN, int BK, int ST, bool AT, bool BT, int EPI>
-__global__ void __launch_bounds__(WM* WN * 64, (tile_wgs<BM, BN, WM, WN, BK, ST>() * WM * WN / 4))
+// Group and position of element x of the sequence that lists, group by group, ceil(rows / per) entries
+// (at least `least`): {group or -1, index in the group, entries of the group}.  One wave looks at 64
+// groups at a time.
+__device__ __forceinline__ int3 tile_group(const int32_t* goff, int G, int per, int least, int x, int lane) {
+  int base = 0;
+  for (int c0 = 0; c0 < G; c0 += 64) {
+    const int gg = c0 + lane;
+    int cnt = 0;
+    if (gg < G) {
+      cnt = (goff[gg + 1] - goff[gg] + per - 1) / per;
+      if (cnt < least) cnt = least;
+    }
+    int incl = cnt;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += y;
+    }
+    const unsigned long long hit = __ballot(cnt > 0 && x >= base + incl - cnt && x < base + incl);
+    if (hit) {
+      const int l = __ffsll((long long)hit) - 1;
+      const int n = __shfl(cnt, l, 64);
+      return make_int3(c0 + l, x - base - __shfl(incl, l, 64) + n, n);
+    }
+    base += __shfl(incl, 63, 64);
+  }
+  return make_int3(-1, 0, 0);
+}
+
+// SwiGLU backward of neurons n .. n + 7 of row m: v holds their dZ; up / gate values sit 32 columns
+// apart.  Writes dUG, returns the neurons' part of <z, dZ>.
+__device__ __forceinline__ float swiglu_bwd8(const Epilogue& e, int m, int n, const float* v) {
+  const int64_t at = (int64_t)m * e.ld_ug + (int64_t)(n >> 5) * 64 + (n & 31);
+  const uint4 uq = *reinterpret_cast<const uint4*>(e.ug_in + at);
+  const uint4 gq = *reinterpret_cast<const uint4*>(e.ug_in + at + 32);
+  const uint32_t uw[4] = {uq.x, uq.y, uq.z, uq.w}, gw[4] = {gq.x, gq.y, gq.z, gq.w};
+  const float rs = e.row_scale ? e.row_scale[m] : 1.0f;
+  uint32_t du[4], dg[4];
+  float part = 0.0f;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const float2 d2 = *reinterpret_cast<const float2*>(v + 2 * t);
+    float a[2], b[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float up = h ? __uint_as_float(uw[t] & 0xffff0000u) : __uint_as_float(uw[t] << 16);
+      const float gt = h ? __uint_as_float(gw[t] & 0xffff0000u) : __uint_as_float(gw[t] << 16);
+      const float draw = h ? d2.y : d2.x;
+      const float s = sigmoidf_(gt), silu = gt * s, dz = draw * rs;
+      a[h] = dz * silu;
+      b[h] = dz * up * s * (1.0f + gt * (1.0f - s));
+      part += up * silu * draw;
+    }
+    du[t] = pack_bf2(a[0], a[1]);
+    dg[t] = pack_bf2(b[0], b[1]);
+  }
+  *reinterpret_cast<uint4*>(e.ug + at) = make_uint4(du[0], du[1], du[2], du[3]);
+  *reinterpret_cast<uint4*>(e.ug + at + 32) = make_uint4(dg[0], dg[1], dg[2], dg[3]);
+  return part;
+}
+
+template <int BM, int BN, int WM, int WN, int BK, int ST, bool AT, bool BT, int EPI, int MODE>
+__global__ void __launch_bounds__(WM* WN * 64, (tile_wgs<BM, BN, WM, WN, BK, ST, MODE>() * WM * WN / 4))
     gemm_tile_kernel(GemmArgs p, int vec) {
   constexpr int NT = WM * WN * 64;
   constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32, KS = BK / 16;
@@ -120,24 +188,70 @@ __global__ void __launch_bounds__(WM* WN * 64, (tile_wgs<BM, BN, WM, WN, BK, ST>
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;
 
-  // Tile order: dispatch id d runs on XCD d % 8, so each XCD takes a contiguous run of tiles, and
-  // a run walks kBand tile rows column by column: the tiles an XCD works on at one time share
-  // few A and B panels of its L2.
-  const int gx = (p.M + BM - 1) / BM, gy = (p.N + BN - 1) / BN, total = gx * gy;
-  int lin = blockIdx.x;
-  {
-    const int q = total >> 3, r = total & 7, xcd = lin & 7;
-    lin = xcd * q + (xcd < r ? xcd : r) + (lin >> 3);
-  }
-  const int bw = kBand * gy, bi = lin / bw;
-  const int rows = gx - bi * kBand < kBand ? gx - bi * kBand : kBand;
-  const int m0 = (bi * kBand + (lin - bi * bw) % rows) * BM, n0 = ((lin - bi * bw) / rows) * BN;
-  int kbeg = 0, kend = p.K;
+  const int gy = (p.N + BN - 1) / BN;
+  int g = 0, m0, n0, mlim = p.M, kbeg = 0, kend = p.K;
   float* partial = nullptr;
-  if (p.splits > 1) {
-    kbeg = blockIdx.y * p.k_chunk;
-    kend = kbeg + p.k_chunk < p.K ? kbeg + p.k_chunk : p.K;
-    partial = p.splitk_ws + (int64_t)blockIdx.y * p.M * p.N;
+  if constexpr (MODE == MODE_DENSE) {
+    // Tile order: dispatch id d runs on XCD d % 8, so each XCD takes a contiguous run of tiles, and
+    // a run walks kBand tile rows column by column: the tiles an XCD works on at one time share
+    // few A and B panels of its L2.
+    const int gx = (p.M + BM - 1) / BM, total = gx * gy;
+    int lin = blockIdx.x;
+    {
+      const int q = total >> 3, r = total & 7, xcd = lin & 7;
+      lin = xcd * q + (xcd < r ? xcd : r) + (lin >> 3);
+    }
+    const int bw = kBand * gy, bi = lin / bw;
+    const int rows = gx - bi * kBand < kBand ? gx - bi * kBand : kBand;
+    m0 = (bi * kBand + (lin - bi * bw) % rows) * BM;
+    n0 = ((lin - bi * bw) / rows) * BN;
+    if (p.splits > 1) {
+      kbeg = blockIdx.y * p.k_chunk;
+      kend = kbeg + p.k_chunk < p.K ? kbeg + p.k_chunk : p.K;
+      partial = p.splitk_ws + (int64_t)blockIdx.y * p.M * p.N;
+    }
+  } else {
+    // Grouped: of every 256 dispatch ids, an XCD takes 32 consecutive tiles, so the tiles of a group
+    // meet in one L2.
+    const int lin = (blockIdx.x & ~255) + (blockIdx.x & 7) * 32 + ((blockIdx.x & 255) >> 3);
+    if constexpr (MODE == MODE_GROUP_M) {
+      const int3 f = tile_group(p.goff, p.G, BM, 0, lin / gy, lane);
+      g = f.x;
+      if (g < 0) return;
+      m0 = p.goff[g] + f.y * BM;
+      n0 = (lin % gy) * BN;
+      mlim = p.goff[g + 1];
+    } else {
+      const int per = (p.M + BM - 1) / BM * gy, item = lin / per, tile = lin - item * per;
+      if (blockIdx.x == 0 && wave == 0) {  // the groups' first items, for the sum of the partials
+        int base = 0;
+        for (int c0 = 0; c0 < p.G; c0 += 64) {
+          const int gg = c0 + lane;
+          int cnt = 0;
+          if (gg < p.G) {
+            cnt = (p.goff[gg + 1] - p.goff[gg] + p.gk_chunk - 1) / p.gk_chunk;
+            if (cnt < 1) cnt = 1;
+          }
+          int incl = cnt;
+#pragma unroll
+          for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += y;
+          }
+          if (gg < p.G) const_cast<int32_t*>(p.gk_first)[gg] = base + incl - cnt;
+          base += __shfl(incl, 63, 64);
+        }
+        if (lane == 0) const_cast<int32_t*>(p.gk_first)[p.G] = base;
+      }
+      const int3 f = tile_group(p.goff, p.G, p.gk_chunk, 1, item, lane);
+      g = f.x;
+      if (g < 0) return;
+      m0 = (tile / gy) * BM;
+      n0 = (tile % gy) * BN;
+      kbeg = p.goff[g] + f.y * p.gk_chunk;
+      kend = kbeg + p.gk_chunk < p.goff[g + 1] ? kbeg + p.gk_chunk : p.goff[g + 1];
+      if (f.z > 1) partial = p.gk_part + (int64_t)item * p.M * p.N;
+    }
   }
 
   f32x16_v acc[TM][TN];
@@ -150,21 +264,60 @@ __global__ void __launch_bounds__(WM* WN * 64, (tile_wgs<BM, BN, WM, WN, BK, ST>
 
   OpA la;
   OpB lb;
-  la.init(p.a, m0, p.M, tid);
-  lb.init(p.b, n0, p.N, tid);
+  // a grouped reduction's output rows and columns are shifted by the epilogue, its operands are not
+  la.init(p.a, MODE == MODE_GROUP_M ? g : 0, m0, mlim, tid, MODE == MODE_GROUP_K);
+  lb.init(p.b, MODE == MODE_GROUP_M ? g : 0, n0, p.N, tid, MODE == MODE_GROUP_K);
   const int alda = (int)p.a.ld, blda = (int)p.b.ld, ailv = p.a.ilv, bilv = p.b.ilv;
   const BufferRsrc ra = buffer_rsrc(p.a.ptr, p.a_bytes), rb = buffer_rsrc(p.b.ptr, p.b_bytes);
 
-  // A ragged reduction (both operands layout T) reads k rows past its end in its last tile: they lie
-  // past the operands' buffer bounds, which the hardware turns into zeros.
+  // Grouped reductions gather the memory rows of one operand (or none): the range's indices sit in
+  // LDS, and the rows of the next refill are looked up a tile ahead.
+  __shared__ int s_idx[MODE == MODE_GROUP_K ? kIdxRows : 1];
+  const bool a_gather = MODE == MODE_GROUP_K && p.a.rows, b_gather = MODE == MODE_GROUP_K && p.b.rows;
+  const int klen = kend - kbeg;
+  uint32_t ar[OpA::INS], br[OpB::INS];  // byte offsets of the next refill's rows (past the range: no row)
+  auto look = [&](int kt) {
+    if constexpr (MODE == MODE_GROUP_K) {
+#pragma unroll
+      for (int u = 0; u < OpA::INS; ++u) {
+        const int k = kt * BK + OpA::krow(u, tid);
+        const int row = a_gather ? s_idx[k < klen ? k : 0] : kbeg + k;
+        ar[u] = k < klen ? (uint32_t)row * (uint32_t)alda * 2u + la.off[u] : 0x80000000u;
+      }
+#pragma unroll
+      for (int u = 0; u < OpB::INS; ++u) {
+        const int k = kt * BK + OpB::krow(u, tid);
+        const int row = b_gather ? s_idx[k < klen ? k : 0] : kbeg + k;
+        br[u] = k < klen ? (uint32_t)row * (uint32_t)blda * 2u + lb.off[u] : 0x80000000u;
+      }
+    }
+  };
+  if constexpr (MODE == MODE_GROUP_K) {
+    const int32_t* rows = p.a.rows ? p.a.rows : p.b.rows;
+    if (rows)
+      for (int i = tid; i < klen; i += NT) s_idx[i] = rows[kbeg + i];
+    if (klen <= 0 && tid == 0) s_idx[0] = 0;
+    __syncthreads();
+  }
+
+  // A ragged dense reduction (both operands layout T) reads k rows past its end in its last tile:
+  // they lie past the operands' buffer bounds, as the rows past a group's range are made to, and the
+  // hardware turns them into zeros.
   auto issue = [&](unsigned char* st, int kt) {
-    const int k0 = kbeg + kt * BK;
-    const int ao = OpA::advance(alda, ailv, k0), bo = OpB::advance(blda, bilv, k0);
     unsigned char* dst = st + wave * 1024;
+    if constexpr (MODE == MODE_GROUP_K) {
 #pragma unroll
-    for (int u = 0; u < OpA::INS; ++u) lds_dma16_buf(ra, dst + u * NT * 16, la.off[u], ao);
+      for (int u = 0; u < OpA::INS; ++u) lds_dma16_buf(ra, dst + u * NT * 16, ar[u], 0);
 #pragma unroll
-    for (int u = 0; u < OpB::INS; ++u) lds_dma16_buf(rb, dst + A_BYTES + u * NT * 16, lb.off[u], bo);
+      for (int u = 0; u < OpB::INS; ++u) lds_dma16_buf(rb, dst + A_BYTES + u * NT * 16, br[u], 0);
+    } else {
+      const int k0 = kbeg + kt * BK;
+      const int ao = OpA::advance(alda, ailv, k0), bo = OpB::advance(blda, bilv, k0);
+#pragma unroll
+      for (int u = 0; u < OpA::INS; ++u) lds_dma16_buf(ra, dst + u * NT * 16, la.off[u], ao);
+#pragma unroll
+      for (int u = 0; u < OpB::INS; ++u) lds_dma16_buf(rb, dst + A_BYTES + u * NT * 16, lb.off[u], bo);
+    }
   };
 
   int aof[TM], bof[TN];
@@ -197,8 +350,9 @@ __global__ void __launch_bounds__(WM* WN * 64, (tile_wgs<BM, BN, WM, WN, BK, ST>
 
   // Tile kt sits in stage (kt + off) % ST, with off so that the last round ends at stage ST - 1:
   // a first round of ST - off tiles, full rounds, and a last one that fetches nothing.  The host
-  // gives every k range at least ST tiles.
-  const int nk = (kend - kbeg + BK - 1) / BK;
+  // gives every dense k range at least ST tiles.
+  int nk = (kend - kbeg + BK - 1) / BK;
+  if (MODE == MODE_GROUP_K && nk < ST) nk = ST;  // few rows: the missing ones read zeros
   const int rounds = (nk + ST - 1) / ST, off = rounds * ST - nk;
 
   // One operand read after each product: the LDS and the matrix cores work at the same time.
@@ -218,6 +372,7 @@ __global__ void __launch_bounds__(WM* WN * 64, (tile_wgs<BM, BN, WM, WN, BK, ST>
   auto step = [&](auto s, auto younger, auto more, int refill) {
     constexpr int S = decltype(s)::value;
     const unsigned char* st = stage_of(s);
+    if constexpr (decltype(more)::value) look(refill);
 #pragma unroll
     for (int ks = 0; ks < KS - 1; ++ks) {
       if ((ks & 1) == 0) {
@@ -248,6 +403,7 @@ __global__ void __launch_bounds__(WM* WN * 64, (tile_wgs<BM, BN, WM, WN, BK, ST>
 
   each_stage([&](auto s) {
     const int t = decltype(s)::value - off;
+    look(t < 0 ? t + ST : t);
     issue(stage_of(s), t < 0 ? t + ST : t);
   });
   if (off == 0) wait_vmcnt_lgkm0<(ST - 1) * INS>();  // tile 0 came first
@@ -294,7 +450,7 @@ __global__ void __launch_bounds__(WM* WN * 64, (tile_wgs<BM, BN, WM, WN, BK, ST>
 #pragma unroll
           for (int u = 0; u < 8; ++u) {
             const int row = u * 4 + (lane >> 4), m = mb + row;
-            if (m >= p.M || n >= p.N) continue;
+            if (m >= mlim || n >= p.N) continue;
             const float4 x = *reinterpret_cast<const float4*>(pt + row * kPatchPitch + cc);
             if (partial) {
               float* dst = partial + (int64_t)m * p.N + n;
@@ -306,7 +462,7 @@ __global__ void __launch_bounds__(WM* WN * 64, (tile_wgs<BM, BN, WM, WN, BK, ST>
               }
             } else {
               float v[4] = {x.x, x.y, x.z, x.w};
-              store_chunk<4>(e, 0, m, n, p.N, v, vec);
+              store_chunk<4>(e, g, m, n, p.N, v, vec);
             }
           }
           continue;
@@ -319,7 +475,7 @@ __global__ void __launch_bounds__(WM* WN * 64, (tile_wgs<BM, BN, WM, WN, BK, ST>
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           const int row = u * 16 + (lane >> 2), m = mb + row;
-          if (m >= p.M || nb >= p.N) continue;
+          if (m >= mlim || nb >= p.N) continue;
           const float* src = pt + row * kPatchPitch + c8;
           const float rs = e.row_scale ? e.row_scale[m] : 1.0f;
           uint32_t uw[4], gw[4], zw[4];
@@ -342,37 +498,27 @@ __global__ void __launch_bounds__(WM* WN * 64, (tile_wgs<BM, BN, WM, WN, BK, ST>
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const int row = u * 8 + (lane >> 3), m = mb + row, n = nb + cc;
-          if (m >= p.M || n >= p.N) continue;
+          if constexpr (EPI == EPI_SWIGLU_BWD && MODE == MODE_GROUP_M) {
+            // <z, dZ> of the row (the pair weight's gradient): all of its neurons are in this patch
+            float part = 0.0f;
+            const bool here = m < mlim && n < p.N;
+            if (here) part = swiglu_bwd8(e, m, n, pt + row * kPatchPitch + cc);
+#pragma unroll
+            for (int o = 1; o <= 4; o <<= 1) part += __shfl_xor(part, o, 64);
+            if (e.dw_row && m < mlim && (lane & 7) == 0) e.dw_row[m] = part;
+            continue;
+          }
+          if (m >= mlim || n >= p.N) continue;
+          if constexpr (EPI == EPI_SWIGLU_BWD && MODE != MODE_GROUP_M) {
+            swiglu_bwd8(e, m, n, pt + row * kPatchPitch + cc);
+            continue;
+          }
           const float4 x = *reinterpret_cast<const float4*>(pt + row * kPatchPitch + cc);
           const float4 y = *reinterpret_cast<const float4*>(pt + row * kPatchPitch + cc + 4);
           float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
           if constexpr (EPI == EPI_STORE) {
-            store_chunk<8>(e, 0, m, n, p.N, v, vec);
-          } else if constexpr (EPI == EPI_SWIGLU_BWD) {
-            // v = dZ of neurons n .. n + 7; their up / gate values sit 32 columns apart
-            const int64_t at = (int64_t)m * e.ld_ug + (int64_t)(n >> 5) * 64 + (n & 31);
-            const uint4 uq = *reinterpret_cast<const uint4*>(e.ug_in + at);
-            const uint4 gq = *reinterpret_cast<const uint4*>(e.ug_in + at + 32);
-            const uint32_t uw[4] = {uq.x, uq.y, uq.z, uq.w}, gw[4] = {gq.x, gq.y, gq.z, gq.w};
-            const float rs = e.row_scale ? e.row_scale[m] : 1.0f;
-            uint32_t du[4], dg[4];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-              float a[2], b[2];
-#pragma unroll
-              for (int h = 0; h < 2; ++h) {
-                const float up = h ? __uint_as_float(uw[t] & 0xffff0000u) : __uint_as_float(uw[t] << 16);
-                const float gt = h ? __uint_as_float(gw[t] & 0xffff0000u) : __uint_as_float(gw[t] << 16);
-                const float s = sigmoidf_(gt), dz = v[2 * t + h] * rs;
-                a[h] = dz * (gt * s);
-                b[h] = dz * up * s * (1.0f + gt * (1.0f - s));
-              }
-              du[t] = pack_bf2(a[0], a[1]);
-              dg[t] = pack_bf2(b[0], b[1]);
-            }
-            *reinterpret_cast<uint4*>(e.ug + at) = make_uint4(du[0], du[1], du[2], du[3]);
-            *reinterpret_cast<uint4*>(e.ug + at + 32) = make_uint4(dg[0], dg[1], dg[2], dg[3]);
-          } else {  // EPI_ROPE_QKV: 8 columns of one head; RoPE pairs (2i, 2i + 1)
+            store_chunk<8>(e, g, m, n, p.N, v, vec);
+          } else if constexpr (EPI == EPI_ROPE_QKV) {  // 8 columns of one head; RoPE pairs (2i, 2i + 1)
             const int part = n / e.dmodel, within = n - part * e.dmodel;
             const int hh = within / e.hd, dim = within - hh * e.hd;
             const int b = m / e.S, s = m - b * e.S;
@@ -398,10 +544,15 @@ __global__ void __launch_bounds__(WM* WN * 64, (tile_wgs<BM, BN, WM, WN, BK, ST>
   }
 }
 
-template <int BM, int BN, int WM, int WN, int BK, int ST, bool AT, bool BT, int EPI>
+template <int BM, int BN, int WM, int WN, int BK, int ST, bool AT, bool BT, int EPI, int MODE = MODE_DENSE>
 int launch(const GemmArgs& p, hipStream_t stream, int vec) {
-  auto fn = gemm_tile_kernel<BM, BN, WM, WN, BK, ST, AT, BT, EPI>;
-  const int64_t tiles = (int64_t)((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
+  auto fn = gemm_tile_kernel<BM, BN, WM, WN, BK, ST, AT, BT, EPI, MODE>;
+  const int64_t gx = (p.M + BM - 1) / BM, gy = (p.N + BN - 1) / BN;
+  int64_t tiles = gx * gy;
+  if (MODE == MODE_GROUP_M) tiles = p.max_tiles_m * gy;
+  if (MODE == MODE_GROUP_K) tiles *= ((int64_t)p.K + p.gk_chunk - 1) / p.gk_chunk + p.G;
+  if (MODE != MODE_DENSE) tiles = (tiles + 255) / 256 * 256;
+  RTE_REQUIRE(tiles < ((int64_t)1 << 31), "gemm: too many tiles");
   hipLaunchKernelGGL(fn, dim3((unsigned)tiles, (unsigned)(p.splits > 1 ? p.splits : 1)), dim3(WM * WN * 64), 0, stream,
                      p, vec);
   return check_launch("gemm_tile");
@@ -469,6 +620,17 @@ int launch_tile(const GemmArgs& p, hipStream_t stream, int vec, int tile) {
 }
 
 }  // namespace
+
+int gemm_tile_group_launch(const GemmArgs& p, int epi_kind, hipStream_t stream, int vec) {
+  if (p.mode == MODE_GROUP_M) {
+    if (epi_kind == EPI_SWIGLU_FWD)
+      return launch<128, 128, 2, 2, 64, 2, false, false, EPI_SWIGLU_FWD, MODE_GROUP_M>(p, stream, vec);
+    return launch<128, 64, 4, 1, 64, 2, false, true, EPI_SWIGLU_BWD, MODE_GROUP_M>(p, stream, vec);
+  }
+  if (p.M <= 64) return launch<64, 128, 2, 2, 32, 4, true, true, EPI_STORE, MODE_GROUP_K>(p, stream, vec);
+  if (p.N <= 64) return launch<128, 64, 4, 1, 32, 4, true, true, EPI_STORE, MODE_GROUP_K>(p, stream, vec);
+  return launch<128, 128, 2, 2, 32, 4, true, true, EPI_STORE, MODE_GROUP_K>(p, stream, vec);
+}
 
 int gemm_tile_launch(const GemmArgs& p0, int epi_kind, hipStream_t stream, int vec, void* ws, size_t ws_bytes,
                      int* splits) {

@@ -12,6 +12,13 @@ constexpr int kTileMaxSplits = 32;
 // x 512 8.7 and 8.6.
 constexpr int kTileRowK = 512;
 
+constexpr int kTileGroupChunk = 2048;  // longest k range of a grouped reduction's workgroup
+
+// Launches a grouped product: GROUP_M with the SwiGLU epilogues (forward: layout-N operands; backward:
+// layout-T B, at most 64 neurons) or GROUP_K with the plain store (chunked: gk_chunk <=
+// kTileGroupChunk, gk_first, gk_part set).  a_bytes / b_bytes set.
+int gemm_tile_group_launch(const GemmArgs& p, int epi_kind, hipStream_t stream, int vec);
+
 // Launches p (MODE_DENSE, operands in plain layouts with a_bytes / b_bytes set) on the tile the
 // estimate picks.  EPI_STORE with a workspace may split the reduction: *splits > 1 then says how
 // many fp32 [M, N] partials the launch leaves in ws for the caller to sum in order.
