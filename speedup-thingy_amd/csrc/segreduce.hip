@@ -1,30 +1,40 @@
 // Deterministic segmented row reduction (the weight-gradient scatter of
 // rte/kernels/cluster_pool_ffn.py:218-241 and of every index/gather backward):
 //   out[v] (+)= sum over pairs p with keys[p] = v of w[p] * rows[p / row_div]
-// The pairs are counting-sorted by key (stable: ascending p), each key's run is summed in
-// 256-pair chunks by one wave, and chunk partials are added in chunk order; up to 4096 pairs
-// over up to 1024 keys take a one-launch path (per-key pair lists, summed in ascending p).  No
-// floating-point atomics: the result is bitwise repeatable for a given input.
+// The pairs are counting-sorted by key (stable: ascending p), each key's run is summed in chunks by
+// one wave per 128 columns, and chunk partials are added in chunk order; up to 4096 pairs over up to
+// 1024 keys take a one-launch path (per-key pair lists, summed in ascending p).  No floating-point
+// atomics: the result is bitwise repeatable for a given input.
+//
+// Bounds, at the shortlist head's 2.1 M pairs over 8192 keys (rows of 1024 bf16): the sums read 4.3 GB of
+// rows.  A wave takes 128 columns and the waves of one column slab run on one XCD, whose 4 MB L2 then
+// holds that slab of every row, so the reads run at L2 and not at memory rate (573 us with whole
+// rows).  The sort moves a histogram of sort blocks x keys, kept block-major so it is written and
+// read in whole lines (312 us key-major with 1024-pair blocks).
 #include "common.hpp"
 
 namespace rte {
 
 namespace {
 
-constexpr int kSortChunk = 1024;      // pairs per counting-sort block
 constexpr int kSortSub = 256;         // pairs ranked together inside a sort block
 constexpr int kMaxSortKeys = 32768;   // LDS histogram of the sort: 128 KB
-constexpr int kSegChunk = 64;         // pairs per partial sum (a long run is cut into many)
+constexpr int kSlab = 128;            // columns of a wave in the sums
 
-// hist[v * nblk + b] = pairs of sort block b whose key is v.
+// Pairs per sort block and per partial sum.  Few pairs: more, shorter pieces (latency); many: fewer
+// histograms and partials.
+int sort_block(int64_t P) { return P > (1 << 19) ? 4096 : 1024; }
+int seg_chunk(int64_t P) { return P >= (1 << 18) ? 128 : 64; }
 
-__global__ void __launch_bounds__(256) sort_count_kernel(const int32_t* __restrict__ keys, int P, int V,
-                                                         int32_t* __restrict__ hist, int nblk) {
+// hist[b * V + v] = pairs of sort block b whose key is v.
+
+__global__ void __launch_bounds__(256) sort_count_kernel(const int32_t* __restrict__ keys, int P, int V, int per,
+                                                         int32_t* __restrict__ hist) {
   extern __shared__ int32_t hcount[];
   for (int c = threadIdx.x; c < V; c += 256) hcount[c] = 0;
   __syncthreads();
-  const int64_t p0 = (int64_t)blockIdx.x * kSortChunk;
-  for (int i = threadIdx.x; i < kSortChunk; i += 256) {
+  const int64_t p0 = (int64_t)blockIdx.x * per;
+  for (int i = threadIdx.x; i < per; i += 256) {
     const int64_t p = p0 + i;
     if (p < P) {
       const int k = keys[p];
@@ -32,114 +42,151 @@ __global__ void __launch_bounds__(256) sort_count_kernel(const int32_t* __restri
     }
   }
   __syncthreads();
-  for (int c = threadIdx.x; c < V; c += 256) hist[(int64_t)c * nblk + blockIdx.x] = hcount[c];
+  int32_t* row = hist + (int64_t)blockIdx.x * V;
+  for (int c = threadIdx.x; c < V; c += 256) row[c] = hcount[c];
 }
 
-// Exclusive scan of each key's row of hist (one wave per key), totals[v] = row sum.
+// Exclusive scan of each key's column of hist, totals[v] = column sum.  A workgroup takes 32 keys
+// (whole 128-byte lines) in 8 ranges of sort blocks.
 __global__ void __launch_bounds__(256) sort_rowscan_kernel(int32_t* __restrict__ hist, int V, int nblk,
                                                            int32_t* __restrict__ totals) {
-  const int lane = threadIdx.x & 63;
-  const int v = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (v >= V) return;
-  int32_t* row = hist + (int64_t)v * nblk;
-  int32_t run = 0;
-  for (int b0 = 0; b0 < nblk; b0 += 64) {
-    const int b = b0 + lane;
-    const int32_t x = b < nblk ? row[b] : 0;
-    int32_t inc = x;
+  __shared__ int32_t part[8][33];
+  const int vi = threadIdx.x & 31, seg = threadIdx.x >> 5;
+  const int v = blockIdx.x * 32 + vi;
+  const int per = (nblk + 7) / 8, b0 = seg * per, b1 = min(nblk, b0 + per);
+  int32_t sum = 0;
+  if (v < V) {
+    int b = b0;
+    for (; b + 8 <= b1; b += 8) {
+      int32_t x[8];
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int32_t y = __shfl_up(inc, off, 64);
-      if (lane >= off) inc += y;
+      for (int u = 0; u < 8; ++u) x[u] = hist[(int64_t)(b + u) * V + v];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) sum += x[u];
     }
-    if (b < nblk) row[b] = run + inc - x;
-    run += __shfl(inc, 63, 64);
+    for (; b < b1; ++b) sum += hist[(int64_t)b * V + v];
   }
-  if (lane == 0) totals[v] = run;
+  part[seg][vi] = sum;
+  __syncthreads();
+  if (v >= V) return;
+  int32_t run = 0;
+  for (int q = 0; q < seg; ++q) run += part[q][vi];
+  int b = b0;
+  for (; b + 8 <= b1; b += 8) {
+    int32_t x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = hist[(int64_t)(b + u) * V + v];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      hist[(int64_t)(b + u) * V + v] = run;
+      run += x[u];
+    }
+  }
+  for (; b < b1; ++b) {
+    const int32_t x = hist[(int64_t)b * V + v];
+    hist[(int64_t)b * V + v] = run;
+    run += x;
+  }
+  if (seg == 7) totals[v] = run;
 }
 
-// offsets = exclusive scan of totals, chunk_off = exclusive scan of ceil(totals / 256).
-__global__ void __launch_bounds__(1024) sort_keyscan_kernel(const int32_t* __restrict__ totals, int V,
+// offsets = exclusive scan of totals, chunk_off = exclusive scan of ceil(totals / chunk).
+__global__ void __launch_bounds__(1024) sort_keyscan_kernel(const int32_t* __restrict__ totals, int V, int chunk,
                                                             int32_t* __restrict__ offsets,
                                                             int32_t* __restrict__ chunk_off) {
-  __shared__ int32_t ps[1024], pc[1024];
-  const int tid = threadIdx.x;
+  __shared__ int32_t ws[16], wc[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int seg = (V + 1023) / 1024;
   const int b0 = tid * seg, b1 = min(V, b0 + seg);
   int32_t s = 0, sc = 0;
   for (int v = b0; v < b1; ++v) {
     s += totals[v];
-    sc += (totals[v] + kSegChunk - 1) / kSegChunk;
+    sc += (totals[v] + chunk - 1) / chunk;
   }
-  ps[tid] = s;
-  pc[tid] = sc;
+  int32_t is = s, ic = sc;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int32_t y = __shfl_up(is, o, 64), yc = __shfl_up(ic, o, 64);
+    if (lane >= o) {
+      is += y;
+      ic += yc;
+    }
+  }
+  if (lane == 63) {
+    ws[wave] = is;
+    wc[wave] = ic;
+  }
   __syncthreads();
-  for (int o = 1; o < 1024; o <<= 1) {
-    const int32_t y = tid >= o ? ps[tid - o] : 0;
-    const int32_t yc = tid >= o ? pc[tid - o] : 0;
-    __syncthreads();
-    ps[tid] += y;
-    pc[tid] += yc;
-    __syncthreads();
+  int32_t run = is - s, runc = ic - sc;
+  for (int q = 0; q < wave; ++q) {
+    run += ws[q];
+    runc += wc[q];
   }
-  int32_t run = ps[tid] - s, runc = pc[tid] - sc;
   for (int v = b0; v < b1; ++v) {
     offsets[v] = run;
     chunk_off[v] = runc;
     run += totals[v];
-    runc += (totals[v] + kSegChunk - 1) / kSegChunk;
+    runc += (totals[v] + chunk - 1) / chunk;
   }
   if (tid == 1023) {
-    offsets[V] = ps[1023];
-    chunk_off[V] = pc[1023];
+    offsets[V] = run;
+    chunk_off[V] = runc;
   }
 }
 
-// Stable scatter: pair p of block b with key v goes to slot offsets[v] + hist[v, b] +
-// (pairs of block b before p with key v).  Writes the pair's row (p / row_div) and weight.
-__global__ void __launch_bounds__(256) sort_scatter_kernel(const int32_t* __restrict__ keys, int P, int V,
-                                                           int row_div, const int32_t* __restrict__ hist, int nblk,
+// Stable scatter: pair p of block b with key v goes to slot offsets[v] + hist[b, v] +
+// (pairs of block b before p with key v).  Writes the pair's row (p / row_div) and weight.  A wave finds
+// the lanes that share a key with one ballot per key bit; the waves take the cursors in turn.  Also
+// item_key[i] = the key whose run chunk i of the sums belongs to.
+__global__ void __launch_bounds__(256) sort_scatter_kernel(const int32_t* __restrict__ keys, int P, int V, int per,
+                                                           int row_div, const int32_t* __restrict__ hist,
                                                            const int32_t* __restrict__ offsets,
-                                                           const float* __restrict__ g,
-                                                           int32_t* __restrict__ tok_of_slot,
-                                                           float* __restrict__ w_of_slot) {
+                                                           const float* __restrict__ g, int2* __restrict__ pairs,
+                                                           const int32_t* __restrict__ chunk_off,
+                                                           int32_t* __restrict__ item_key) {
   extern __shared__ int32_t cursor[];
-  __shared__ __align__(16) int32_t sk[kSortSub];
-  const int tid = threadIdx.x;
-  for (int c = tid; c < V; c += 256) cursor[c] = offsets[c] + hist[(int64_t)c * nblk + blockIdx.x];
-  const int64_t p0 = (int64_t)blockIdx.x * kSortChunk;
-  constexpr int NQ = kSortChunk / kSortSub;
-  int kq[NQ];  // every key of the block loaded up front (one memory latency, not one per sub-chunk)
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const int64_t p = p0 + q * kSortSub + tid;
-    kq[q] = p < P ? keys[p] : -1;
-  }
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const int64_t p = p0 + q * kSortSub + tid;
-    const int k = kq[q];
-    const bool valid = k >= 0 && k < V;
-    __syncthreads();  // cursor ready / previous sub-chunk done with sk
-    sk[tid] = valid ? k : -1;
-    __syncthreads();
-    int rank = 0;  // pairs of this sub-chunk before tid with the same key (16-byte LDS reads)
-    if (valid) {
-      const int4* s4 = reinterpret_cast<const int4*>(sk);
-#pragma unroll 4
-      for (int i4 = 0; 4 * i4 < tid; ++i4) {
-        const int4 v = s4[i4];
-        const int b = 4 * i4;
-        rank += (b < tid && v.x == k) + (b + 1 < tid && v.y == k) + (b + 2 < tid && v.z == k) +
-                (b + 3 < tid && v.w == k);
-      }
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int32_t* row = hist + (int64_t)blockIdx.x * V;
+  for (int c = tid; c < V; c += 256) cursor[c] = offsets[c] + row[c];
+  const int64_t p0 = (int64_t)blockIdx.x * per;
+  const int bits = V > 1 ? 32 - __clz(V - 1) : 0;
+  const int nsub = (int)((P - p0 < per ? P - p0 : per) + kSortSub - 1) / kSortSub;
+  int next = p0 + tid < P ? keys[p0 + tid] : -1;
+  const int items = chunk_off[V];
+  for (int i = blockIdx.x * 256 + tid; i < items; i += gridDim.x * 256) {
+    int lo = 0, hi = V;  // largest v with chunk_off[v] <= i
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (chunk_off[mid] <= i) lo = mid; else hi = mid;
     }
-    const int slot = valid ? cursor[k] + rank : 0;
-    __syncthreads();
+    item_key[i] = lo;
+  }
+  __syncthreads();
+  for (int q = 0; q < nsub; ++q) {
+    const int64_t p = p0 + (int64_t)q * kSortSub + tid;
+    const int k = next;
+    if (q + 1 < nsub) next = p + kSortSub < P && (q + 1) * kSortSub + tid < per ? keys[p + kSortSub] : -1;
+    const bool valid = k >= 0 && k < V;
+    unsigned long long same = __ballot(valid);
+    for (int b = 0; b < bits; ++b) {
+      const bool one = (k >> b) & 1;
+      const unsigned long long m = __ballot(one);
+      same &= one ? m : ~m;
+    }
+    const int rank = __popcll(same & ((1ull << lane) - 1ull)), count = __popcll(same);
+    int slot = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      if (wave == w && valid) {
+        slot = cursor[k] + rank;
+        __builtin_amdgcn_wave_barrier();  // every lane has read its cursor
+        if (rank == 0) cursor[k] = slot + count;
+      }
+      __syncthreads();
+    }
     if (valid) {
-      atomicAdd(&cursor[k], 1);
-      tok_of_slot[slot] = (int32_t)(p / row_div);
-      w_of_slot[slot] = g ? g[p] : 1.0f;
+      const float wp = g ? g[p] : 1.0f;
+      pairs[slot] = make_int2((int32_t)(p / row_div), __float_as_int(wp));
     }
   }
 }
@@ -160,84 +207,65 @@ __device__ __forceinline__ void load8(const float* p, float* v) {
   v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
 }
 
-// One wave per 64-pair chunk of one key's run: sum_s w[s] * rows[tok[s]].  A key with a
-// single chunk writes out directly; otherwise the chunk's partial goes to part[item].
-template <int NC2, typename RowT>
+__device__ __forceinline__ float2 load2(const bf16* p) {
+  const uint32_t w = *reinterpret_cast<const uint32_t*>(p);
+  return make_float2(__uint_as_float(w << 16), __uint_as_float(w & 0xffff0000u));
+}
+__device__ __forceinline__ float2 load2(const float* p) { return *reinterpret_cast<const float2*>(p); }
+
+// One wave per chunk of one key's run and slab of 128 columns (two per lane): sum_s w[s] * rows[tok[s]].  A
+// key with a single chunk writes out directly; otherwise the chunk's partial goes to part[item].
+// Dispatch id b runs on XCD b % 8: each XCD takes a contiguous run of (slab, chunk) in slab order.
+template <typename RowT>
 __global__ void __launch_bounds__(256) sort_segsum_kernel(const int32_t* __restrict__ offsets,
-                                                          const int32_t* __restrict__ chunk_off, int V,
-                                                          const int32_t* __restrict__ tok,
-                                                          const float* __restrict__ w,
+                                                          const int32_t* __restrict__ chunk_off,
+                                                          const int32_t* __restrict__ item_key, int V, int chunk,
+                                                          int max_items, int nslab, const int2* __restrict__ pairs,
                                                           const RowT* __restrict__ hidden, int d,
                                                           float* __restrict__ part, float* __restrict__ dW,
                                                           int accumulate) {
   const int lane = threadIdx.x & 63;
-  const int item = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (item >= chunk_off[V]) return;
-  int lo = 0, hi = V;  // largest v with chunk_off[v] <= item
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (chunk_off[mid] <= item) lo = mid; else hi = mid;
-  }
-  const int v = lo;
-  const int nq = chunk_off[v + 1] - chunk_off[v];
-  const int s0 = offsets[v] + (item - chunk_off[v]) * kSegChunk;
-  const int s1 = min(offsets[v + 1], s0 + kSegChunk);
-  const int nch = d >> 3;
-  float acc[NC2][8];
-#pragma unroll
-  for (int c = 0; c < NC2; ++c)
-#pragma unroll
-    for (int i = 0; i < 8; ++i) acc[c][i] = 0.0f;
-  auto fma_row = [&](int s) {
-    const RowT* row = hidden + (int64_t)tok[s] * d;
-    const float gs = w[s];
-#pragma unroll
-    for (int c = 0; c < NC2; ++c) {
-      if (lane + 64 * c >= nch) continue;
-      float v[8];
-      load8(row + (lane + 64 * c) * 8, v);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) acc[c][i] += gs * v[i];
-    }
-  };
+  const int nb = gridDim.x, xcd = blockIdx.x & 7, q8 = nb >> 3, r8 = nb & 7;
+  const int blk = xcd * q8 + (xcd < r8 ? xcd : r8) + (blockIdx.x >> 3);
+  const int64_t id = (int64_t)blk * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int slab = (int)(id / max_items), item = (int)(id - (int64_t)slab * max_items);
+  if (slab >= nslab || item >= chunk_off[V]) return;
+  const int v = item_key[item];
+  const int first = chunk_off[v], nq = chunk_off[v + 1] - first;
+  const int s0 = offsets[v] + (item - first) * chunk;
+  const int s1 = min(offsets[v + 1], s0 + chunk);
+  const int col = slab * kSlab + lane * 2;
+  const bool on = col < d;
+  const RowT* base = hidden + (on ? col : 0);
+  float2 acc = make_float2(0.0f, 0.0f);
   int s = s0;
-  for (; s + 8 <= s1; s += 8) {  // 8 rows in flight: indices and weights first, then the rows
-    int t8[8];
-    float g8[8];
+  for (; s + 8 <= s1; s += 8) {  // 8 rows in flight
+    int2 pr[8];
+    float2 x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) pr[j] = pairs[s + j];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = load2(base + (int64_t)pr[j].x * d);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      t8[j] = tok[s + j];
-      g8[j] = w[s + j];
-    }
-#pragma unroll
-    for (int c = 0; c < NC2; ++c) {
-      if (lane + 64 * c >= nch) continue;
-      float v[8][8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) load8(hidden + (int64_t)t8[j] * d + (lane + 64 * c) * 8, v[j]);
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[c][i] += g8[j] * v[j][i];
+      acc.x += __int_as_float(pr[j].y) * x[j].x;
+      acc.y += __int_as_float(pr[j].y) * x[j].y;
     }
   }
-  for (; s < s1; ++s) fma_row(s);
-  float* dst = nq == 1 ? dW + (int64_t)v * d : part + (int64_t)item * d;
-  const bool add = nq == 1 && accumulate;
-#pragma unroll
-  for (int c = 0; c < NC2; ++c) {
-    if (lane + 64 * c >= nch) continue;
-    float4* o = reinterpret_cast<float4*>(dst + (lane + 64 * c) * 8);
-    float4 a = make_float4(acc[c][0], acc[c][1], acc[c][2], acc[c][3]);
-    float4 b = make_float4(acc[c][4], acc[c][5], acc[c][6], acc[c][7]);
-    if (add) {
-      const float4 a0 = o[0], b0 = o[1];
-      a.x += a0.x; a.y += a0.y; a.z += a0.z; a.w += a0.w;
-      b.x += b0.x; b.y += b0.y; b.z += b0.z; b.w += b0.w;
-    }
-    o[0] = a;
-    o[1] = b;
+  for (; s < s1; ++s) {
+    const int2 pr = pairs[s];
+    const float2 x = load2(base + (int64_t)pr.x * d);
+    acc.x += __int_as_float(pr.y) * x.x;
+    acc.y += __int_as_float(pr.y) * x.y;
   }
+  if (!on) return;
+  float2* o = reinterpret_cast<float2*>((nq == 1 ? dW + (int64_t)v * d : part + (int64_t)item * d) + col);
+  if (nq == 1 && accumulate) {
+    const float2 old = *o;
+    acc.x += old.x;
+    acc.y += old.y;
+  }
+  *o = acc;
 }
 
 // Keys with zero or several chunks: dW[v] (+)= sum of the key's partials in chunk order.
@@ -281,15 +309,16 @@ struct SegCarve {
   int32_t* totals;
   int32_t* offsets;
   int32_t* chunk_off;
-  int32_t* tok;
-  float* wslot;
+  int32_t* item_key;
+  int2* pairs;
   float* part;
   size_t bytes;
 };
 
 SegCarve carve(void* base, int64_t P, int V, int d) {
-  const size_t nblk = ((size_t)P + kSortChunk - 1) / kSortChunk;
-  const size_t max_items = ((size_t)P + kSegChunk - 1) / kSegChunk + (size_t)V;
+  const size_t per = sort_block(P), chunk = seg_chunk(P);
+  const size_t nblk = ((size_t)P + per - 1) / per;
+  const size_t max_items = ((size_t)P + chunk - 1) / chunk + (size_t)V;
   SegCarve c{};
   size_t off = 0;
   auto take = [&](size_t bytes) {
@@ -301,8 +330,8 @@ SegCarve carve(void* base, int64_t P, int V, int d) {
   c.totals = static_cast<int32_t*>(take((size_t)V * 4));
   c.offsets = static_cast<int32_t*>(take((size_t)(V + 1) * 4));
   c.chunk_off = static_cast<int32_t*>(take((size_t)(V + 1) * 4));
-  c.tok = static_cast<int32_t*>(take((size_t)P * 4));
-  c.wslot = static_cast<float*>(take((size_t)P * 4));
+  c.item_key = static_cast<int32_t*>(take(max_items * 4));
+  c.pairs = static_cast<int2*>(take((size_t)P * 8));
   c.part = static_cast<float*>(take(max_items * (size_t)d * 4));
   c.bytes = off;
   return c;
@@ -358,21 +387,6 @@ __global__ void __launch_bounds__(256) segsum_small_kernel(const int32_t* __rest
   }
 }
 
-template <typename RowT>
-int launch_segsum(int nc2, dim3 grid, hipStream_t s, const SegCarve& c, int V, const RowT* rows, int d, float* out,
-                  int accumulate) {
-  if (nc2 <= 1)
-    hipLaunchKernelGGL((sort_segsum_kernel<1, RowT>), grid, dim3(256), 0, s, c.offsets, c.chunk_off, V, c.tok,
-                       c.wslot, rows, d, c.part, out, accumulate);
-  else if (nc2 <= 2)
-    hipLaunchKernelGGL((sort_segsum_kernel<2, RowT>), grid, dim3(256), 0, s, c.offsets, c.chunk_off, V, c.tok,
-                       c.wslot, rows, d, c.part, out, accumulate);
-  else
-    hipLaunchKernelGGL((sort_segsum_kernel<4, RowT>), grid, dim3(256), 0, s, c.offsets, c.chunk_off, V, c.tok,
-                       c.wslot, rows, d, c.part, out, accumulate);
-  return check_launch("segment_reduce_sum");
-}
-
 }  // namespace
 
 size_t segreduce_workspace_bytes(int64_t P, int V, int d) {
@@ -403,28 +417,35 @@ int segreduce_rows(const int32_t* keys, int64_t P, int V, int row_div, const flo
                          static_cast<const bf16*>(rows), d, out, accumulate);
     return check_launch("segment_reduce_small");
   }
-  const int nblk = (Pi + kSortChunk - 1) / kSortChunk;
+  const int per = sort_block(P), chunk = seg_chunk(P);
+  const int nblk = (Pi + per - 1) / per;
   const dim3 block(256);
   const size_t lds_hist = (size_t)V * sizeof(int32_t);
   RTE_TRY(set_lds_limit(sort_count_kernel, lds_hist, "segment_reduce"));
-  RTE_TRY(set_lds_limit(sort_scatter_kernel, lds_hist + kSortSub * sizeof(int32_t), "segment_reduce"));
-  hipLaunchKernelGGL(sort_count_kernel, dim3(nblk), block, lds_hist, s, keys, Pi, V, c.hist, nblk);
+  RTE_TRY(set_lds_limit(sort_scatter_kernel, lds_hist, "segment_reduce"));
+  hipLaunchKernelGGL(sort_count_kernel, dim3(nblk), block, lds_hist, s, keys, Pi, V, per, c.hist);
   RTE_TRY(check_launch("segment_reduce_count"));
-  hipLaunchKernelGGL(sort_rowscan_kernel, dim3((V + 3) / 4), block, 0, s, c.hist, V, nblk, c.totals);
+  hipLaunchKernelGGL(sort_rowscan_kernel, dim3((V + 31) / 32), block, 0, s, c.hist, V, nblk, c.totals);
   RTE_TRY(check_launch("segment_reduce_rowscan"));
-  hipLaunchKernelGGL(sort_keyscan_kernel, dim3(1), dim3(1024), 0, s, c.totals, V, c.offsets, c.chunk_off);
+  hipLaunchKernelGGL(sort_keyscan_kernel, dim3(1), dim3(1024), 0, s, c.totals, V, chunk, c.offsets, c.chunk_off);
   RTE_TRY(check_launch("segment_reduce_keyscan"));
-  hipLaunchKernelGGL(sort_scatter_kernel, dim3(nblk), block, lds_hist, s, keys, Pi, V, row_div, c.hist, nblk,
-                     c.offsets, w, c.tok, c.wslot);
-  RTE_TRY(check_launch("segment_reduce_scatter"));
   // the chunk count lives on the device: launch its upper bound, extra waves exit at once
-  const int64_t max_items = ((int64_t)Pi + kSegChunk - 1) / kSegChunk + V;
-  const dim3 grid_i((unsigned)((max_items + 3) / 4));
-  const int nc2 = (d / 8 + 63) / 64;
+  const int64_t max_items = ((int64_t)Pi + chunk - 1) / chunk + V;
+  hipLaunchKernelGGL(sort_scatter_kernel, dim3(nblk), block, lds_hist, s, keys, Pi, V, per, row_div, c.hist, c.offsets,
+                     w, c.pairs, c.chunk_off, c.item_key);
+  RTE_TRY(check_launch("segment_reduce_scatter"));
+  const int nslab = (d + kSlab - 1) / kSlab;
+  const int64_t nwg = (max_items * nslab + 3) / 4;
+  RTE_REQUIRE(nwg < ((int64_t)1 << 31), "segment_reduce: too many partial sums");
   if (rows_f32)
-    RTE_TRY(launch_segsum(nc2, grid_i, s, c, V, static_cast<const float*>(rows), d, out, accumulate));
+    hipLaunchKernelGGL(sort_segsum_kernel<float>, dim3((unsigned)nwg), block, 0, s, c.offsets, c.chunk_off, c.item_key, V,
+                       chunk, (int)max_items, nslab, c.pairs, static_cast<const float*>(rows), d, c.part, out,
+                       accumulate);
   else
-    RTE_TRY(launch_segsum(nc2, grid_i, s, c, V, static_cast<const bf16*>(rows), d, out, accumulate));
+    hipLaunchKernelGGL(sort_segsum_kernel<bf16>, dim3((unsigned)nwg), block, 0, s, c.offsets, c.chunk_off, c.item_key, V,
+                       chunk, (int)max_items, nslab, c.pairs, static_cast<const bf16*>(rows), d, c.part, out,
+                       accumulate);
+  RTE_TRY(check_launch("segment_reduce_sum"));
   const int64_t n4 = (int64_t)V * (d / 4);
   hipLaunchKernelGGL(sort_final_kernel, dim3((unsigned)((n4 + 255) / 256)), block, 0, s, c.chunk_off, V, d, c.part,
                      out, accumulate);
