@@ -1,6 +1,6 @@
 // SVD low-rank SwiGLU FFN with the wide activations kept on chip (rte/layers.py:342-643, the
-// low-rank factor products of SVDFactorSparseFFN; BASELINE cfg4 uses U diag(S) V^T as the up,
-// gate and down weights):
+// low-rank factor products of SVDFactorSparseFFN, with U diag(S) V^T as the up, gate and down
+// weights):
 //
 //   a    = x @ [A_up | A_gate]                  [T, 2r]   (A = U diag(S), GEMM)
 //   u, g = a_up V_up^T, a_gate V_gate^T         [T, F]    never written
@@ -30,22 +30,10 @@
 // 8 (l / 32) .. +7 of each 16-step; output register r of lane l holds row 8 (r / 4) + 4 (l / 32)
 // + r % 4, column l % 32.
 #include "common.hpp"
-#include "gemm.hpp"
+#include "gemm_dev.hpp"
 
 namespace rte {
 namespace {
-
-// LDS pitch (bf16) of a transposed [R][32] tile: 72-byte rows.  Its reads (sv_ld_perm: 8 bytes per
-// lane from 32 consecutive rows) then start at 32 distinct even banks, so a wave's read covers the
-// 64 banks once (an 80-byte pitch maps rows r and r + 16 to the same banks).  Rows are 8-byte
-// aligned only: the tiles are written with 8-byte stores (sv_st16).
-constexpr int kTP = 36;
-
-// 16 bytes at an 8-byte aligned LDS address
-__device__ __forceinline__ void sv_st16(bf16* dst, uint4 v) {
-  *reinterpret_cast<uint2*>(dst) = make_uint2(v.x, v.y);
-  *reinterpret_cast<uint2*>(dst + 4) = make_uint2(v.z, v.w);
-}
 
 __device__ __forceinline__ f32x16_v sv_mfma(bf16x8_v a, bf16x8_v b, f32x16_v c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
@@ -53,21 +41,6 @@ __device__ __forceinline__ f32x16_v sv_mfma(bf16x8_v a, bf16x8_v b, f32x16_v c) 
 
 __device__ __forceinline__ bf16x8_v sv_ld8(const bf16* p) {
   return __builtin_bit_cast(bf16x8_v, *reinterpret_cast<const uint4*>(p));
-}
-
-// the 8 k-slots of a reduction over the 32 entries of an accumulator block, for step s and lane
-// half h: entries 16 s + 4 h + (0..3) and 16 s + 8 + 4 h + (0..3), read from a row of a
-// transposed [.][kTP] LDS tile
-__device__ __forceinline__ bf16x8_v sv_ld_perm(const bf16* row, int s, int h) {
-  const uint2 a = *reinterpret_cast<const uint2*>(row + 16 * s + 4 * h);
-  const uint2 b = *reinterpret_cast<const uint2*>(row + 16 * s + 8 + 4 * h);
-  return __builtin_bit_cast(bf16x8_v, make_uint4(a.x, a.y, b.x, b.y));
-}
-
-// accumulator registers 8 s .. 8 s + 7 as a B operand (the matching k-slots of sv_ld_perm)
-__device__ __forceinline__ bf16x8_v sv_pack(const float* v) {
-  return __builtin_bit_cast(bf16x8_v, make_uint4(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]),
-                                                 pack_bf2(v[4], v[5]), pack_bf2(v[6], v[7])));
 }
 
 __device__ __forceinline__ f32x16_v sv_zero() {
@@ -81,419 +54,385 @@ __device__ __forceinline__ f32x16_v sv_zero() {
 // feed bf16 MFMA operands)
 __device__ __forceinline__ float sv_sigmoid(float x) { return __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
 
-// v where m is all ones, zeros where m is 0 (loads stay unconditional at a clamped address)
-__device__ __forceinline__ uint4 sv_mask(uint4 v, uint32_t m) { return make_uint4(v.x & m, v.y & m, v.z & m, v.w & m); }
+// A 32-row tile of one operand in LDS: rows of R bf16 as the matrix has them, 16-byte chunk c of
+// row r stored at c ^ swz(r).  The operand reads of 16 consecutive rows (one chunk each) and the
+// transposing reads (four consecutive rows, 64 bytes each) then both cover all banks once.
+template <int R>
+struct SvTile {
+  static constexpr int CPR = R / 8, BYTES = 32 * R * 2, NV = R / 64;
+  __device__ __forceinline__ static int swz(int r) {
+    return CPR == 16 ? ((r & 3) << 2) | ((r >> 2) & 3) : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
+  }
+};
+
+// The loop over 32-row tiles that the three kernels share.  Tile i of three matrices (m0, m1, m2:
+// rows 32 i .. of `rows`, R columns at the given pitch) meets the wave's 32 columns (bu, bg, bd):
+//   u = m0 bu, g = m1 bg, dz = m2 bd                              (rows x columns, over R)
+//   acc_u += m0^T du, acc_g += m1^T dg (UG), acc_d += m2^T z (D)  (R x columns, over rows)
+// Rows at or past `rows` read as zeros and add nothing.
+//
+// Tiles go from memory straight into LDS and serve both products: the second reads its operand
+// transposed (ds_read_b64_tr_b16) from the same rows.  (With transposed copies of the matrices in
+// memory a tile took 64 bytes from each of R rows that lie a power of two apart, all in one L2
+// channel: 5300 - 9500 cycles a tile against 1300 - 1500 of matrix instructions.)  The accumulators leave
+// room for one wave per SIMD in the backward kernels, so nothing else hides an LDS read or the
+// vector work: both are spread by hand over slots of matrix instructions (without: 300 / 247 us for
+// bwdw / bwdx).  What is left is issue: a wave issues about 400 instructions of 4 cycles a tile.
+//
+// T 32768, F 4096, R 128, us before and now: fwd 141, 108; bwdx 288, 186; bwdw 509, 217; and four
+// transposes (22) gone.
+template <int R, bool GRAD, bool UG, bool D>
+struct SvMid {
+  static constexpr int KS = R / 16, JB = R / 32, NV = SvTile<R>::NV, CPR = SvTile<R>::CPR, TB = SvTile<R>::BYTES;
+  static constexpr int NM = 3;                               // matrices
+  static constexpr int NB = (UG ? 2 : 0) + (D ? 1 : 0);          // second products
+  static constexpr int NG = KS / 4, NU = GRAD ? KS / 2 : KS / 4;  // slots of the gate and up products
+  static constexpr int NS = JB / 2;                              // slots of a step of the second
+  f32x16_v acc_u[UG ? JB : 1], acc_g[UG ? JB : 1], acc_d[D ? JB : 1];
+  bf16x8_v bu[KS], bg[KS], bd[GRAD ? KS : 1];
+  f32x16_v u, g, dz, sl;         // of the tile in work; sl: silu(g)
+  uint32_t pz[8], pu[8], pg[8];  // bf16 pairs of z, du, dg by accumulator row
+  int ra[KS], ta[JB][2];
+  const bf16* m[NM];
+  int pitch[NM];
+  uint32_t voff[NM][NV];
+  int rows, wave;
+
+  __device__ __forceinline__ void init(const bf16* m0, int p0, const bf16* m1, int p1, const bf16* m2, int p2,
+                                       int nrows) {
+    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
+    wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    rows = nrows;
+    m[0] = m0; m[1] = m1; m[2] = m2;
+    pitch[0] = p0; pitch[1] = p1; pitch[2] = p2;
+#pragma unroll
+    for (int k = 0; k < NM; ++k)
+#pragma unroll
+      for (int q = 0; q < NV; ++q) {
+        const int r = (tid + 256 * q) / CPR, c = (tid + 256 * q) % CPR;
+        voff[k][q] = (uint32_t)(r * pitch[k] + (c ^ SvTile<R>::swz(r)) * 8) * 2;
+      }
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) ra[ks] = (l32 * CPR + ((2 * ks + h) ^ SvTile<R>::swz(l32))) * 16;
+    const int i = lane & 15, sub = (lane >> 4) & 1;
+#pragma unroll
+    for (int jb = 0; jb < JB; ++jb)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int r = 8 * j + 4 * h + (i >> 2), col = 32 * jb + 16 * sub + 4 * (i & 3);
+        ta[jb][j] = (r * CPR + ((col >> 3) ^ SvTile<R>::swz(r))) * 16 + (col & 7) * 2;
+      }
+#pragma unroll
+    for (int jb = 0; jb < JB; ++jb) {
+      if constexpr (UG) acc_u[jb] = acc_g[jb] = sv_zero();
+      if constexpr (D) acc_d[jb] = sv_zero();
+    }
+  }
+
+  // tile i into a stage; tiles at or past `end` load nothing (zero-length descriptors)
+  __device__ __forceinline__ void load(unsigned char* st, int i, int end) const {
+    const int left = rows - i * 32, nr = i < end ? (left < 32 ? left : 32) : 0;
+#pragma unroll
+    for (int k = 0; k < NM; ++k) {
+      const BufferRsrc rs = buffer_rsrc(m[k] + (int64_t)(i < end ? i : 0) * 32 * pitch[k],
+                                        nr ? (uint32_t)((nr - 1) * pitch[k] + R) * 2 : 0u);
+#pragma unroll
+      for (int q = 0; q < NV; ++q) lds_dma16_buf(rs, st + k * TB + (q * 256 + wave * 64) * 16, voff[k][q], 0);
+    }
+  }
+
+  // Operands of a slot and its matrix instructions.  Gate: k steps 4n .. 4n + 3 of g = m1 bg.
+  __device__ __forceinline__ void read_gate(const unsigned char* st, int n, bf16x8_v* f) const {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f[e] = *reinterpret_cast<const bf16x8_v*>(st + TB + ra[4 * n + e]);
+  }
+  __device__ __forceinline__ void mm_gate(const bf16x8_v* f, int n) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) g = sv_mfma(f[e], bg[4 * n + e], n + e == 0 ? sv_zero() : g);
+  }
+  // Up: k steps 2n, 2n + 1 of u = m0 bu and dz = m2 bd (4n .. 4n + 3 without dz).
+  __device__ __forceinline__ void read_up(const unsigned char* st, int n, bf16x8_v* f) const {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int k = GRAD ? e & 1 : 0, ks = GRAD ? 2 * n + (e >> 1) : 4 * n + e;
+      f[e] = *reinterpret_cast<const bf16x8_v*>(st + 2 * k * TB + ra[ks]);
+    }
+  }
+  __device__ __forceinline__ void mm_up(const bf16x8_v* f, int n) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int ks = GRAD ? 2 * n + (e >> 1) : 4 * n + e;
+      if (GRAD && (e & 1)) dz = sv_mfma(f[e], bd[GRAD ? ks : 0], ks == 0 ? sv_zero() : dz);
+      else u = sv_mfma(f[e], bu[ks], ks == 0 ? sv_zero() : u);
+    }
+  }
+  // Second products of step s (accumulator rows 8 s ..), blocks 2n, 2n + 1: rows of the tile turned
+  // into columns, in the accumulators' row order.
+  __device__ __forceinline__ void read_second(const unsigned char* st, int s, int n, bf16x8_v* f) const {
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int k = 0; k < NB; ++k) {
+        const unsigned char* t = st + (UG ? k : 2) * TB + s * 16 * CPR * 16;
+        const short4_v lo = lds_read_tr4(t + ta[2 * n + e][0]), hi = lds_read_tr4(t + ta[2 * n + e][1]);
+        typedef short short8_v __attribute__((ext_vector_type(8)));
+        f[e * NB + k] = __builtin_bit_cast(bf16x8_v, (short8_v)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      }
+  }
+  __device__ __forceinline__ void mm_second(const bf16x8_v* f, int s, int n) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int k = 0; k < NB; ++k) {
+        const uint32_t* p = (UG ? (k == 0 ? pu : k == 1 ? pg : pz) : pz) + 4 * s;
+        const bf16x8_v b = __builtin_bit_cast(bf16x8_v, make_uint4(p[0], p[1], p[2], p[3]));
+        f32x16_v& acc = UG ? (k == 0 ? acc_u[2 * n + e] : k == 1 ? acc_g[2 * n + e] : acc_d[D ? 2 * n + e : 0])
+                           : acc_d[D ? 2 * n + e : 0];
+        acc = sv_mfma(f[e * NB + k], b, acc);
+      }
+  }
+
+  // Vector work on accumulator rows r0 .. r0 + N - 1: silu(g) and silu'(g) (left in g) ...
+  template <int N>
+  __device__ __forceinline__ void gate(int r0) {
+#pragma unroll
+    for (int r = r0; r < r0 + N; ++r) {
+      const float sg = sv_sigmoid(g[r]);
+      sl[r] = g[r] * sg;
+      if constexpr (UG) g[r] = sg + sl[r] * (1.0f - sg);
+    }
+  }
+  // ... and the bf16 operands of the second products.
+  template <int N>
+  __device__ __forceinline__ void act(int r0) {
+#pragma unroll
+    for (int r = r0; r < r0 + N; r += 2) {
+      if constexpr (D) pz[r / 2] = pack_bf2(u[r] * sl[r], u[r + 1] * sl[r + 1]);
+      if constexpr (UG) {
+        pu[r / 2] = pack_bf2(dz[r] * sl[r], dz[r + 1] * sl[r + 1]);
+        pg[r / 2] = pack_bf2(dz[r] * u[r] * g[r], dz[r + 1] * u[r + 1] * g[r + 1]);
+      }
+    }
+  }
+
+  __device__ __forceinline__ static void fence() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+  }
+  // Order within a slot: M matrix instructions, V vector and X exp / reciprocal instructions after each.
+  template <int M, int V, int X, int L>
+  __device__ __forceinline__ static void weave() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    constexpr int kVector = 0x2, kMatrix = 0x8, kLdsRead = 0x100, kTrans = 0x400;
+#pragma unroll
+    for (int n = 0; n < M; ++n) {
+      __builtin_amdgcn_sched_group_barrier(kMatrix, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(kLdsRead, L, 0);
+      if constexpr (X > 0) __builtin_amdgcn_sched_group_barrier(kTrans, X, 0);
+      if constexpr (V > 0) __builtin_amdgcn_sched_group_barrier(kVector, V, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+  }
+
+  // Tile i in slots of 4 to 6 matrix instructions.  A slot begins with the LDS reads of the slot after it
+  // and carries a share of the vector work, so that a wave alone on its SIMD keeps the matrix cores
+  // busy.  Order: gate products; up products (gate functions of the vector unit); second products of
+  // step 1 of tile i - 1 (operands of step 0); barrier; second products of step 0 (operands of step 1).
+  template <bool START>
+  __device__ __forceinline__ void tile(const unsigned char* cur, unsigned char* prev, const unsigned char* next, int i,
+                                       int end, bf16x8_v (*f)[6]) {
+    constexpr int GV = UG ? 5 : 3;                       // vector instructions per gate row
+    constexpr int AV = (UG ? 4 : 0) + (D ? 2 : 0);       // per operand row, about
+    constexpr int UR = 16 / NU, SR = 8 / NS;             // rows per slot
+    int q = 0;
+#pragma unroll
+    for (int n = 0; n < NG; ++n, ++q) {
+      if (n + 1 < NG) read_gate(cur, n + 1, f[(q + 1) & 1]);
+      else read_up(cur, 0, f[(q + 1) & 1]);
+      mm_gate(f[q & 1], n);
+      weave<4, 0, 0, 1>();
+    }
+#pragma unroll
+    for (int n = 0; n < NU; ++n, ++q) {
+      if (n + 1 < NU) read_up(cur, n + 1, f[(q + 1) & 1]);
+      else if (START) read_second(cur, 0, 0, f[(q + 1) & 1]);
+      else read_second(prev, 1, 0, f[(q + 1) & 1]);
+      mm_up(f[q & 1], n);
+      gate<UR>(n * UR);
+      weave<4, (UR * GV + 3) / 4, (UR * 2 + 3) / 4, 1>();
+    }
+#pragma unroll
+    for (int n = 0; n < NS; ++n) {
+      if (!START) {
+        if (n + 1 < NS) read_second(prev, 1, n + 1, f[(q + 1) & 1]);
+        else read_second(cur, 0, 0, f[(q + 1) & 1]);
+        mm_second(f[q & 1], 1, n);
+        ++q;
+      }
+      act<SR>(n * SR);
+      if (!START) weave<2 * NB, (SR * AV + 2 * NB - 1) / (2 * NB), 0, 2>();
+    }
+    wait_vmcnt_lgkm0<0>();
+    wg_barrier();  // tile i + 1 is in LDS, every wave is done with tile i - 1
+    load(prev, i + 2, end);
+    fence();
+    bf16x8_v ahead[4];
+#pragma unroll
+    for (int n = 0; n < NS; ++n, ++q) {
+      if (n + 1 < NS) read_second(cur, 0, n + 1, f[(q + 1) & 1]);
+      else read_gate(next, 0, ahead);
+      mm_second(f[q & 1], 0, n);
+      act<SR>(8 + n * SR);
+      weave<2 * NB, (SR * AV + 2 * NB - 1) / (2 * NB), 0, 2>();
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f[0][e] = ahead[e];
+  }
+  __device__ __forceinline__ void run(unsigned char* s0, unsigned char* s1, unsigned char* s2, int i0, int i1) {
+    if (i0 >= i1) return;
+    load(s0, i0, i1);
+    load(s1, i0 + 1, i1);
+    bf16x8_v f[2][6];
+    wait_vmcnt_lgkm0<NM * NV>();
+    wg_barrier();
+    read_gate(s0, 0, f[0]);
+    tile<true>(s0, s2, s1, i0, i1, f);
+    int i = i0 + 1;
+    for (; i + 2 < i1; i += 3) {
+      tile<false>(s1, s0, s2, i, i1, f);
+      tile<false>(s2, s1, s0, i + 1, i1, f);
+      tile<false>(s0, s2, s1, i + 2, i1, f);
+    }
+    if (i < i1) tile<false>(s1, s0, s2, i, i1, f);
+    if (i + 1 < i1) tile<false>(s2, s1, s0, i + 1, i1, f);
+    const int last = (i1 - 1 - i0) % 3;
+    const unsigned char* st = last == 0 ? s0 : last == 1 ? s1 : s2;
+#pragma unroll
+    for (int n = 0; n < NS; ++n) {  // step 1 of the last tile
+      read_second(st, 1, n, f[0]);
+      mm_second(f[0], 1, n);
+    }
+    wait_vmcnt<0>();
+  }
+};
+
+// One row of a wave's R x 32 accumulator blocks per lane column: element j of row `out` (16-byte
+// fp32 or 8-byte bf16 stores)
+template <int JB>
+__device__ __forceinline__ void sv_store(const f32x16_v* acc, int h, float* f32_row, bf16* bf16_row) {
+#pragma unroll
+  for (int jb = 0; jb < JB; ++jb) {
+    const f32x16_v& a = acc[jb];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int j = jb * 32 + 8 * q + 4 * h;
+      if (f32_row != nullptr)
+        *reinterpret_cast<float4*>(f32_row + j) = make_float4(a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]);
+      else
+        *reinterpret_cast<uint2*>(bf16_row + j) =
+            make_uint2(pack_bf2(a[4 * q], a[4 * q + 1]), pack_bf2(a[4 * q + 2], a[4 * q + 3]));
+    }
+  }
+}
+
+// Stages are arrays of their own: from one array the transposing reads wait for every load in flight.
+#define SVD_STAGE(name) __shared__ __align__(1024) unsigned char name[3 * SvTile<R>::BYTES]
 
 // Forward middle: b (or fp32 partials over neuron splits) from a = [a_up | a_gate].
 // grid (ceil(T / 128), splits), 256 threads; wave w owns tokens blockIdx.x * 128 + 32 w + (0..31);
 // split y covers neuron chunks [y cps, (y + 1) cps) of 32 neurons.
 template <int R>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void svd_mid_fwd_kernel(const bf16* __restrict__ a_ug,
-                                                          const bf16* __restrict__ v_ug,
-                                                          const bf16* __restrict__ v_dnT, int T, int F, int cps,
-                                                          bf16* __restrict__ b_out, float* __restrict__ part) {
-  constexpr int KS = R / 16, JB = R / 32, P = R + 8, NV = R / 64;
-  __shared__ __align__(16) bf16 s_vu[32 * P];
-  __shared__ __align__(16) bf16 s_vg[32 * P];
-  __shared__ __align__(16) bf16 s_vdT[R * kTP];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, l32 = lane & 31;
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void svd_mid_fwd_kernel(
+    const bf16* __restrict__ a_ug, const bf16* __restrict__ v_ug, const bf16* __restrict__ v_dn, int T, int F, int cps,
+    bf16* __restrict__ b_out, float* __restrict__ part) {
+  SVD_STAGE(s0);
+  SVD_STAGE(s1);
+  SVD_STAGE(s2);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, h = lane >> 5, l32 = lane & 31;
   const int t = blockIdx.x * 128 + w * 32 + l32;
   const int tl = t < T ? t : T - 1;
   const int nc = F / 32;
   const int c0 = blockIdx.y * cps;
   const int c1 = c0 + cps < nc ? c0 + cps : nc;
-
-  bf16x8_v bu[KS], bg[KS];
-  {
-    const bf16* arow = a_ug + (int64_t)tl * 2 * R + 8 * h;
+  SvMid<R, false, false, true> k;
+  k.init(v_ug, R, v_ug + (int64_t)F * R, R, v_dn, R, F);
+  const bf16* arow = a_ug + (int64_t)tl * 2 * R + 8 * h;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      bu[ks] = sv_ld8(arow + 16 * ks);
-      bg[ks] = sv_ld8(arow + R + 16 * ks);
-    }
+  for (int ks = 0; ks < k.KS; ++ks) {
+    k.bu[ks] = sv_ld8(arow + 16 * ks);
+    k.bg[ks] = sv_ld8(arow + R + 16 * ks);
   }
-  f32x16_v acc[JB];
-#pragma unroll
-  for (int jb = 0; jb < JB; ++jb) acc[jb] = sv_zero();
-
-  // staging: chunk c's three tiles go global -> registers (issued one chunk ahead) -> LDS
-  uint4 rv0_0, rv1_0, rv2_0, rv0_1, rv1_1, rv2_1;  // [matrix]_[vector]
-#define SVD_FWD_GLOAD1(c, q) \
-  { \
-    const int f0 = (c) * 32; \
-    const int i = tid + 256 * (q); \
-    const int row = i / (R / 8), col = (i % (R / 8)) * 8; \
-    rv0_##q = *reinterpret_cast<const uint4*>(v_ug + (int64_t)(f0 + row) * R + col); \
-    rv1_##q = *reinterpret_cast<const uint4*>(v_ug + (int64_t)(F + f0 + row) * R + col); \
-    const int j = i >> 2, cj = (i & 3) * 8; \
-    rv2_##q = *reinterpret_cast<const uint4*>(v_dnT + (int64_t)j * F + f0 + cj); \
-  }
-#define SVD_FWD_GLOAD(c) \
-  { \
-    SVD_FWD_GLOAD1(c, 0) \
-    if constexpr (NV > 1) SVD_FWD_GLOAD1(c, 1) \
-  }
-  if (c0 < c1) SVD_FWD_GLOAD(c0)
-  for (int c = c0; c < c1; ++c) {
-    __syncthreads();  // every wave is done reading the previous chunk
-    {
-      const int i = tid + 256 * 0;
-      const int row = i / (R / 8), col = (i % (R / 8)) * 8;
-      *reinterpret_cast<uint4*>(s_vu + row * P + col) = rv0_0;
-      *reinterpret_cast<uint4*>(s_vg + row * P + col) = rv1_0;
-      const int j = i >> 2, cj = (i & 3) * 8;
-      sv_st16(s_vdT + j * kTP + cj, rv2_0);
-    }
-    if constexpr (NV > 1) {
-      const int i = tid + 256 * 1;
-      const int row = i / (R / 8), col = (i % (R / 8)) * 8;
-      *reinterpret_cast<uint4*>(s_vu + row * P + col) = rv0_1;
-      *reinterpret_cast<uint4*>(s_vg + row * P + col) = rv1_1;
-      const int j = i >> 2, cj = (i & 3) * 8;
-      sv_st16(s_vdT + j * kTP + cj, rv2_1);
-    }
-    __syncthreads();
-    if (c + 1 < c1) SVD_FWD_GLOAD(c + 1)  // in flight during this chunk's products
-    f32x16_v u = sv_zero(), g = sv_zero();
-    const bf16* vu = s_vu + l32 * P + 8 * h;
-    const bf16* vg = s_vg + l32 * P + 8 * h;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      u = sv_mfma(sv_ld8(vu + 16 * ks), bu[ks], u);
-      g = sv_mfma(sv_ld8(vg + 16 * ks), bg[ks], g);
-    }
-    bf16x8_v zb[2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      float zz[8];
-#pragma unroll
-      for (int m = 0; m < 8; ++m) {
-        const float gv = g[8 * s + m];
-        zz[m] = u[8 * s + m] * gv * sv_sigmoid(gv);
-      }
-      zb[s] = sv_pack(zz);
-    }
-#pragma unroll
-    for (int jb = 0; jb < JB; ++jb) {
-      const bf16* row = s_vdT + (jb * 32 + l32) * kTP;
-#pragma unroll
-      for (int s = 0; s < 2; ++s) acc[jb] = sv_mfma(sv_ld_perm(row, s, h), zb[s], acc[jb]);
-    }
-  }
+  k.run(s0, s1, s2, c0, c1);
   if (t >= T) return;
-#pragma unroll
-  for (int jb = 0; jb < JB; ++jb) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int j = jb * 32 + 8 * q + 4 * h;
-      if (part != nullptr) {
-        *reinterpret_cast<float4*>(part + ((int64_t)blockIdx.y * T + t) * R + j) =
-            make_float4(acc[jb][4 * q], acc[jb][4 * q + 1], acc[jb][4 * q + 2], acc[jb][4 * q + 3]);
-      } else {
-        *reinterpret_cast<uint2*>(b_out + (int64_t)t * R + j) =
-            make_uint2(pack_bf2(acc[jb][4 * q], acc[jb][4 * q + 1]), pack_bf2(acc[jb][4 * q + 2], acc[jb][4 * q + 3]));
-      }
-    }
-  }
+  sv_store<R / 32>(k.acc_d, h, part ? part + ((int64_t)blockIdx.y * T + t) * R : nullptr, b_out + (int64_t)t * R);
 }
 
 // Backward to the low-rank codes: da = [du V_up | dg V_gate] per token tile (fp32 partials over
-// neuron splits when splits > 1).  Layout and grid as svd_mid_fwd_kernel; v_ugT = [V_up; V_gate]^T
-// ([R][2F]).
+// neuron splits when splits > 1).  Layout and grid as svd_mid_fwd_kernel.
 template <int R>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void svd_mid_bwdx_kernel(const bf16* __restrict__ a_ug, const bf16* __restrict__ db,
-                                                           const bf16* __restrict__ v_ug,
-                                                           const bf16* __restrict__ v_dn,
-                                                           const bf16* __restrict__ v_ugT, int T, int F, int cps,
-                                                           bf16* __restrict__ da_out, float* __restrict__ part) {
-  constexpr int KS = R / 16, JB = R / 32, P = R + 8, NV = R / 64;
-  __shared__ __align__(16) bf16 s_vu[32 * P];
-  __shared__ __align__(16) bf16 s_vg[32 * P];
-  __shared__ __align__(16) bf16 s_vd[32 * P];
-  __shared__ __align__(16) bf16 s_vuT[R * kTP];
-  __shared__ __align__(16) bf16 s_vgT[R * kTP];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, l32 = lane & 31;
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void svd_mid_bwdx_kernel(
+    const bf16* __restrict__ a_ug, const bf16* __restrict__ db, const bf16* __restrict__ v_ug,
+    const bf16* __restrict__ v_dn, int T, int F, int cps, bf16* __restrict__ da_out, float* __restrict__ part) {
+  SVD_STAGE(s0);
+  SVD_STAGE(s1);
+  SVD_STAGE(s2);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, h = lane >> 5, l32 = lane & 31;
   const int t = blockIdx.x * 128 + w * 32 + l32;
   const int tl = t < T ? t : T - 1;
   const int nc = F / 32;
   const int c0 = blockIdx.y * cps;
   const int c1 = c0 + cps < nc ? c0 + cps : nc;
-
-  bf16x8_v bu[KS], bg[KS], bd[KS];
-  {
-    const bf16* arow = a_ug + (int64_t)tl * 2 * R + 8 * h;
-    const bf16* drow = db + (int64_t)tl * R + 8 * h;
+  SvMid<R, true, true, false> k;
+  k.init(v_ug, R, v_ug + (int64_t)F * R, R, v_dn, R, F);
+  const bf16* arow = a_ug + (int64_t)tl * 2 * R + 8 * h;
+  const bf16* drow = db + (int64_t)tl * R + 8 * h;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      bu[ks] = sv_ld8(arow + 16 * ks);
-      bg[ks] = sv_ld8(arow + R + 16 * ks);
-      bd[ks] = sv_ld8(drow + 16 * ks);
-    }
+  for (int ks = 0; ks < k.KS; ++ks) {
+    k.bu[ks] = sv_ld8(arow + 16 * ks);
+    k.bg[ks] = sv_ld8(arow + R + 16 * ks);
+    k.bd[ks] = sv_ld8(drow + 16 * ks);
   }
-  f32x16_v acc_u[JB], acc_g[JB];
-#pragma unroll
-  for (int kb = 0; kb < JB; ++kb) {
-    acc_u[kb] = sv_zero();
-    acc_g[kb] = sv_zero();
-  }
-
-  uint4 rv0_0, rv1_0, rv2_0, rv3_0, rv4_0, rv0_1, rv1_1, rv2_1, rv3_1, rv4_1;
-#define SVD_BWDX_GLOAD1(c, q) \
-  { \
-    const int f0 = (c) * 32; \
-    const int i = tid + 256 * (q); \
-    const int row = i / (R / 8), col = (i % (R / 8)) * 8; \
-    rv0_##q = *reinterpret_cast<const uint4*>(v_ug + (int64_t)(f0 + row) * R + col); \
-    rv1_##q = *reinterpret_cast<const uint4*>(v_ug + (int64_t)(F + f0 + row) * R + col); \
-    rv2_##q = *reinterpret_cast<const uint4*>(v_dn + (int64_t)(f0 + row) * R + col); \
-    const int k = i >> 2, ck = (i & 3) * 8; \
-    rv3_##q = *reinterpret_cast<const uint4*>(v_ugT + (int64_t)k * 2 * F + f0 + ck); \
-    rv4_##q = *reinterpret_cast<const uint4*>(v_ugT + (int64_t)k * 2 * F + F + f0 + ck); \
-  }
-#define SVD_BWDX_GLOAD(c) \
-  { \
-    SVD_BWDX_GLOAD1(c, 0) \
-    if constexpr (NV > 1) SVD_BWDX_GLOAD1(c, 1) \
-  }
-  if (c0 < c1) SVD_BWDX_GLOAD(c0)
-  for (int c = c0; c < c1; ++c) {
-    __syncthreads();
-    {
-      const int i = tid + 256 * 0;
-      const int row = i / (R / 8), col = (i % (R / 8)) * 8;
-      *reinterpret_cast<uint4*>(s_vu + row * P + col) = rv0_0;
-      *reinterpret_cast<uint4*>(s_vg + row * P + col) = rv1_0;
-      *reinterpret_cast<uint4*>(s_vd + row * P + col) = rv2_0;
-      const int k = i >> 2, ck = (i & 3) * 8;
-      sv_st16(s_vuT + k * kTP + ck, rv3_0);
-      sv_st16(s_vgT + k * kTP + ck, rv4_0);
-    }
-    if constexpr (NV > 1) {
-      const int i = tid + 256 * 1;
-      const int row = i / (R / 8), col = (i % (R / 8)) * 8;
-      *reinterpret_cast<uint4*>(s_vu + row * P + col) = rv0_1;
-      *reinterpret_cast<uint4*>(s_vg + row * P + col) = rv1_1;
-      *reinterpret_cast<uint4*>(s_vd + row * P + col) = rv2_1;
-      const int k = i >> 2, ck = (i & 3) * 8;
-      sv_st16(s_vuT + k * kTP + ck, rv3_1);
-      sv_st16(s_vgT + k * kTP + ck, rv4_1);
-    }
-    __syncthreads();
-    if (c + 1 < c1) SVD_BWDX_GLOAD(c + 1)
-    f32x16_v u = sv_zero(), g = sv_zero(), dz = sv_zero();
-    const int off = l32 * P + 8 * h;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      u = sv_mfma(sv_ld8(s_vu + off + 16 * ks), bu[ks], u);
-      g = sv_mfma(sv_ld8(s_vg + off + 16 * ks), bg[ks], g);
-      dz = sv_mfma(sv_ld8(s_vd + off + 16 * ks), bd[ks], dz);
-    }
-    bf16x8_v dub[2], dgb[2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      float du[8], dg[8];
-#pragma unroll
-      for (int m = 0; m < 8; ++m) {
-        const int r = 8 * s + m;
-        const float sg = sv_sigmoid(g[r]);
-        du[m] = dz[r] * g[r] * sg;
-        dg[m] = dz[r] * u[r] * sg * (1.0f + g[r] * (1.0f - sg));
-      }
-      dub[s] = sv_pack(du);
-      dgb[s] = sv_pack(dg);
-    }
-#pragma unroll
-    for (int kb = 0; kb < JB; ++kb) {
-      const bf16* ru = s_vuT + (kb * 32 + l32) * kTP;
-      const bf16* rg = s_vgT + (kb * 32 + l32) * kTP;
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        acc_u[kb] = sv_mfma(sv_ld_perm(ru, s, h), dub[s], acc_u[kb]);
-        acc_g[kb] = sv_mfma(sv_ld_perm(rg, s, h), dgb[s], acc_g[kb]);
-      }
-    }
-  }
+  k.run(s0, s1, s2, c0, c1);
   if (t >= T) return;
-#pragma unroll
-  for (int half = 0; half < 2; ++half) {
-#pragma unroll
-    for (int kb = 0; kb < JB; ++kb) {
-      const f32x16_v& a = half ? acc_g[kb] : acc_u[kb];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int k = half * R + kb * 32 + 8 * q + 4 * h;
-        if (part != nullptr) {
-          *reinterpret_cast<float4*>(part + ((int64_t)blockIdx.y * T + t) * 2 * R + k) =
-              make_float4(a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]);
-        } else {
-          *reinterpret_cast<uint2*>(da_out + (int64_t)t * 2 * R + k) =
-              make_uint2(pack_bf2(a[4 * q], a[4 * q + 1]), pack_bf2(a[4 * q + 2], a[4 * q + 3]));
-        }
-      }
-    }
-  }
+  float* prow = part ? part + ((int64_t)blockIdx.y * T + t) * 2 * R : nullptr;
+  bf16* orow = da_out + (int64_t)t * 2 * R;
+  sv_store<R / 32>(k.acc_u, h, prow, orow);
+  sv_store<R / 32>(k.acc_g, h, prow ? prow + R : nullptr, orow + R);
 }
 
-// Backward to the factors V_up, V_gate, V_dn: grid (F / 128, splits), 256 threads; wave w owns
-// neurons blockIdx.x * 128 + 32 w + (0..31) (the lane index); split y reduces token tiles
-// [y tps, (y + 1) tps) of 32 tokens.  Writes [dV_up; dV_gate] ([2F][R]) and dV_dn ([F][R]) in
-// fp32, or fp32 partials [split][3F][R] when splits > 1.  a_ugT ([2R][T]) and dbT ([R][T]) are
-// the transposes of a_ug and db.  T % 8 == 0.
+// Backward to the factors V_up, V_gate, V_dn: grid (splits, F / 128), 256 threads; wave w owns
+// neurons blockIdx.y * 128 + 32 w + (0..31) (the lane index); split x reduces token tiles
+// [x tps, (x + 1) tps) of 32 tokens (consecutive workgroups run on different XCDs, so one L2 mostly
+// sees one token range).  Writes [dV_up; dV_gate] ([2F][R]) and dV_dn ([F][R]) in fp32, or fp32
+// partials [split][3F][R] when splits > 1.
 template <int R>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void svd_mid_bwdw_kernel(const bf16* __restrict__ a_ug, const bf16* __restrict__ db,
-                                                           const bf16* __restrict__ a_ugT,
-                                                           const bf16* __restrict__ dbT,
-                                                           const bf16* __restrict__ v_ug,
-                                                           const bf16* __restrict__ v_dn, int T, int F, int tps,
-                                                           float* __restrict__ dv_ug, float* __restrict__ dv_dn,
-                                                           float* __restrict__ part) {
-  constexpr int KS = R / 16, JB = R / 32, P = R + 8, NV = R / 64;
-  // dynamic LDS (svd_bwdw_lds_bytes): the token tile's rows and transposes, then the workgroup's
-  // 128 rows of V_up and V_gate (the B operands of the recomputed products; V_dn's rows stay in
-  // registers)
-  extern __shared__ __align__(16) unsigned char sm_raw[];
-  bf16* s_au = reinterpret_cast<bf16*>(sm_raw);
-  bf16* s_ag = s_au + 32 * P;
-  bf16* s_db = s_ag + 32 * P;
-  bf16* s_auT = s_db + 32 * P;
-  bf16* s_agT = s_auT + R * kTP;
-  bf16* s_dbT = s_agT + R * kTP;
-  bf16* s_wu = s_dbT + R * kTP;
-  bf16* s_wg = s_wu + 128 * P;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, l32 = lane & 31;
-  const int f = blockIdx.x * 128 + w * 32 + l32;
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void svd_mid_bwdw_kernel(
+    const bf16* __restrict__ a_ug, const bf16* __restrict__ db, const bf16* __restrict__ v_ug,
+    const bf16* __restrict__ v_dn, int T, int F, int tps, float* __restrict__ dv_ug, float* __restrict__ dv_dn,
+    float* __restrict__ part) {
+  SVD_STAGE(s0);
+  SVD_STAGE(s1);
+  SVD_STAGE(s2);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, h = lane >> 5, l32 = lane & 31;
+  const int64_t f = (int64_t)blockIdx.y * 128 + w * 32 + l32;
   const int nt = (T + 31) / 32;
-  const int t0 = blockIdx.y * tps;
+  const int t0 = blockIdx.x * tps;
   const int t1 = t0 + tps < nt ? t0 + tps : nt;
-
-  // the workgroup's 128 V_up / V_gate rows -> LDS (made visible by the loop's first barrier)
-  for (int i = tid; i < 128 * R / 8; i += 256) {
-    const int row = i / (R / 8), col = (i % (R / 8)) * 8;
-    const int64_t fr = (int64_t)blockIdx.x * 128 + row;
-    *reinterpret_cast<uint4*>(s_wu + row * P + col) = *reinterpret_cast<const uint4*>(v_ug + fr * R + col);
-    *reinterpret_cast<uint4*>(s_wg + row * P + col) = *reinterpret_cast<const uint4*>(v_ug + (F + fr) * R + col);
+  SvMid<R, true, true, true> k;
+  k.init(a_ug, 2 * R, a_ug + R, 2 * R, db, R, T);
+#pragma unroll
+  for (int ks = 0; ks < k.KS; ++ks) {
+    k.bu[ks] = sv_ld8(v_ug + f * R + 16 * ks + 8 * h);
+    k.bg[ks] = sv_ld8(v_ug + (F + f) * R + 16 * ks + 8 * h);
+    k.bd[ks] = sv_ld8(v_dn + f * R + 16 * ks + 8 * h);
   }
-  bf16x8_v wd[KS];
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) wd[ks] = sv_ld8(v_dn + (int64_t)f * R + 16 * ks + 8 * h);
-  f32x16_v acc_u[JB], acc_g[JB], acc_d[JB];
-#pragma unroll
-  for (int kb = 0; kb < JB; ++kb) {
-    acc_u[kb] = sv_zero();
-    acc_g[kb] = sv_zero();
-    acc_d[kb] = sv_zero();
-  }
-
-  uint4 rv0_0, rv1_0, rv2_0, rv3_0, rv4_0, rv5_0, rv0_1, rv1_1, rv2_1, rv3_1, rv4_1, rv5_1;
-  // rows of tokens at or past T load as zeros (T % 8 == 0: a vector of 8 tokens is all in or
-  // all out), so they add nothing to the reductions
-#define SVD_BWDW_GLOAD1(tt, q) \
-  { \
-    const int tb = (tt) * 32; \
-    const int i = tid + 256 * (q); \
-    const int row = i / (R / 8), col = (i % (R / 8)) * 8; \
-    const uint32_t rm = tb + row < T ? 0xffffffffu : 0u; \
-    const int64_t tr = rm ? tb + row : 0; \
-    rv0_##q = sv_mask(*reinterpret_cast<const uint4*>(a_ug + tr * 2 * R + col), rm); \
-    rv1_##q = sv_mask(*reinterpret_cast<const uint4*>(a_ug + tr * 2 * R + R + col), rm); \
-    rv2_##q = sv_mask(*reinterpret_cast<const uint4*>(db + tr * R + col), rm); \
-    const int k = i >> 2, ct = (i & 3) * 8; \
-    const uint32_t cm = tb + ct < T ? 0xffffffffu : 0u; \
-    const int64_t tc = cm ? tb + ct : 0; \
-    rv3_##q = sv_mask(*reinterpret_cast<const uint4*>(a_ugT + (int64_t)k * T + tc), cm); \
-    rv4_##q = sv_mask(*reinterpret_cast<const uint4*>(a_ugT + (int64_t)(R + k) * T + tc), cm); \
-    rv5_##q = sv_mask(*reinterpret_cast<const uint4*>(dbT + (int64_t)k * T + tc), cm); \
-  }
-#define SVD_BWDW_GLOAD(tt) \
-  { \
-    SVD_BWDW_GLOAD1(tt, 0) \
-    if constexpr (NV > 1) SVD_BWDW_GLOAD1(tt, 1) \
-  }
-  if (t0 < t1) SVD_BWDW_GLOAD(t0)
-  for (int tt = t0; tt < t1; ++tt) {
-    __syncthreads();
-    {
-      const int i = tid + 256 * 0;
-      const int row = i / (R / 8), col = (i % (R / 8)) * 8;
-      *reinterpret_cast<uint4*>(s_au + row * P + col) = rv0_0;
-      *reinterpret_cast<uint4*>(s_ag + row * P + col) = rv1_0;
-      *reinterpret_cast<uint4*>(s_db + row * P + col) = rv2_0;
-      const int k = i >> 2, ct = (i & 3) * 8;
-      sv_st16(s_auT + k * kTP + ct, rv3_0);
-      sv_st16(s_agT + k * kTP + ct, rv4_0);
-      sv_st16(s_dbT + k * kTP + ct, rv5_0);
-    }
-    if constexpr (NV > 1) {
-      const int i = tid + 256 * 1;
-      const int row = i / (R / 8), col = (i % (R / 8)) * 8;
-      *reinterpret_cast<uint4*>(s_au + row * P + col) = rv0_1;
-      *reinterpret_cast<uint4*>(s_ag + row * P + col) = rv1_1;
-      *reinterpret_cast<uint4*>(s_db + row * P + col) = rv2_1;
-      const int k = i >> 2, ct = (i & 3) * 8;
-      sv_st16(s_auT + k * kTP + ct, rv3_1);
-      sv_st16(s_agT + k * kTP + ct, rv4_1);
-      sv_st16(s_dbT + k * kTP + ct, rv5_1);
-    }
-    __syncthreads();
-    if (tt + 1 < t1) SVD_BWDW_GLOAD(tt + 1)
-    // token index as the MFMA row dimension: u[t][f] etc. with the neuron across lanes
-    f32x16_v u = sv_zero(), g = sv_zero(), dz = sv_zero();
-    const int off = l32 * P + 8 * h;
-    const int woff = (w * 32 + l32) * P + 8 * h;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      u = sv_mfma(sv_ld8(s_au + off + 16 * ks), sv_ld8(s_wu + woff + 16 * ks), u);
-      g = sv_mfma(sv_ld8(s_ag + off + 16 * ks), sv_ld8(s_wg + woff + 16 * ks), g);
-      dz = sv_mfma(sv_ld8(s_db + off + 16 * ks), wd[ks], dz);
-    }
-    bf16x8_v zb[2], dub[2], dgb[2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      float zz[8], du[8], dg[8];
-#pragma unroll
-      for (int m = 0; m < 8; ++m) {
-        const int r = 8 * s + m;
-        const float sg = sv_sigmoid(g[r]);
-        zz[m] = u[r] * g[r] * sg;
-        du[m] = dz[r] * g[r] * sg;
-        dg[m] = dz[r] * u[r] * sg * (1.0f + g[r] * (1.0f - sg));
-      }
-      zb[s] = sv_pack(zz);
-      dub[s] = sv_pack(du);
-      dgb[s] = sv_pack(dg);
-    }
-#pragma unroll
-    for (int kb = 0; kb < JB; ++kb) {
-      const bf16* ru = s_auT + (kb * 32 + l32) * kTP;
-      const bf16* rg = s_agT + (kb * 32 + l32) * kTP;
-      const bf16* rd = s_dbT + (kb * 32 + l32) * kTP;
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        acc_u[kb] = sv_mfma(sv_ld_perm(ru, s, h), dub[s], acc_u[kb]);
-        acc_g[kb] = sv_mfma(sv_ld_perm(rg, s, h), dgb[s], acc_g[kb]);
-        acc_d[kb] = sv_mfma(sv_ld_perm(rd, s, h), zb[s], acc_d[kb]);
-      }
-    }
-  }
-#pragma unroll
-  for (int m3 = 0; m3 < 3; ++m3) {
-#pragma unroll
-    for (int kb = 0; kb < JB; ++kb) {
-      const f32x16_v& a = m3 == 0 ? acc_u[kb] : (m3 == 1 ? acc_g[kb] : acc_d[kb]);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int k = kb * 32 + 8 * q + 4 * h;
-        const float4 v = make_float4(a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]);
-        float* dst;
-        if (part != nullptr) {
-          dst = part + ((int64_t)blockIdx.y * 3 * F + (int64_t)m3 * F + f) * R + k;
-        } else {
-          dst = m3 < 2 ? dv_ug + ((int64_t)m3 * F + f) * R + k : dv_dn + (int64_t)f * R + k;
-        }
-        *reinterpret_cast<float4*>(dst) = v;
-      }
-    }
-  }
+  k.run(s0, s1, s2, t0, t1);
+  float* p = part ? part + ((int64_t)blockIdx.x * 3 * F + f) * R : nullptr;
+  sv_store<R / 32>(k.acc_u, h, p ? p : dv_ug + f * R, nullptr);
+  sv_store<R / 32>(k.acc_g, h, p ? p + (int64_t)F * R : dv_ug + (F + f) * R, nullptr);
+  sv_store<R / 32>(k.acc_d, h, p ? p + (int64_t)2 * F * R : dv_dn + f * R, nullptr);
 }
 
 // out = sum over splits y (in order) of part[y][e]; elements e < n0 go to out0 (fp32 or bf16),
@@ -520,42 +459,6 @@ __global__ __launch_bounds__(256) void svd_split_sum_kernel(const float* __restr
   }
 }
 
-// out[c][r] = in[r][c] (bf16), 64 x 64 tiles through LDS; rows % 4 == 0, cols % 4 == 0.
-__global__ __launch_bounds__(256) void svd_transpose_kernel(const bf16* __restrict__ in, int rows, int cols,
-                                                            int64_t ld_in, bf16* __restrict__ out, int64_t ld_out) {
-  __shared__ bf16 tile[64][66];
-  const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;  // 16 x 16 threads, 4 elements each way
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int r = r0 + ty + 16 * k, c = c0 + 4 * tx;
-    if (r < rows && c < cols) {
-      const uint2 v = *reinterpret_cast<const uint2*>(in + (int64_t)r * ld_in + c);
-      tile[ty + 16 * k][4 * tx] = (bf16)(v.x & 0xffffu);
-      tile[ty + 16 * k][4 * tx + 1] = (bf16)(v.x >> 16);
-      tile[ty + 16 * k][4 * tx + 2] = (bf16)(v.y & 0xffffu);
-      tile[ty + 16 * k][4 * tx + 3] = (bf16)(v.y >> 16);
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int c = c0 + ty + 16 * k, r = r0 + 4 * tx;
-    if (c < cols && r < rows) {
-      const int lc = ty + 16 * k, lr = 4 * tx;
-      const uint32_t lo = (uint32_t)tile[lr][lc] | ((uint32_t)tile[lr + 1][lc] << 16);
-      const uint32_t hi = (uint32_t)tile[lr + 2][lc] | ((uint32_t)tile[lr + 3][lc] << 16);
-      *reinterpret_cast<uint2*>(out + (int64_t)c * ld_out + r) = make_uint2(lo, hi);
-    }
-  }
-}
-
-int transpose_bf16(const bf16* in, int rows, int cols, int64_t ld_in, bf16* out, int64_t ld_out, hipStream_t s) {
-  dim3 grid((cols + 63) / 64, (rows + 63) / 64);
-  hipLaunchKernelGGL(svd_transpose_kernel, grid, dim3(256), 0, s, in, rows, cols, ld_in, out, ld_out);
-  return check_launch("svd_transpose");
-}
-
 int split_sum(const float* part, int splits, int64_t n, int64_t n0, void* out0, void* out1, int out_bf16,
               hipStream_t s) {
   const int64_t blocks = (n / 4 + 255) / 256;
@@ -573,31 +476,8 @@ Operand op_plain(const void* p, int64_t ld) {
 
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
-constexpr size_t svd_bwdw_lds_bytes(int R) {
-  return ((size_t)3 * 32 * (R + 8) + (size_t)3 * R * kTP + (size_t)2 * 128 * (R + 8)) * 2;
-}
-
-template <int R>
-int launch_bwdw(dim3 grid, hipStream_t st, const bf16* a_ug, const bf16* db, const bf16* a_ugT, const bf16* dbT,
-                const bf16* v_ug, const bf16* v_dn, int T, int F, int tps, float* dv_ug, float* dv_dn, float* part) {
-  constexpr size_t lds = svd_bwdw_lds_bytes(R);
-  static bool attr_done = false;
-  if (!attr_done) {
-    hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(svd_mid_bwdw_kernel<R>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (err != hipSuccess) {
-      set_error("svd_ffn_fused: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(err));
-      return -1;
-    }
-    attr_done = true;
-  }
-  hipLaunchKernelGGL(svd_mid_bwdw_kernel<R>, grid, dim3(256), lds, st, a_ug, db, a_ugT, dbT, v_ug, v_dn, T, F, tps,
-                     dv_ug, dv_dn, part);
-  return check_launch("svd_mid_bwdw");
-}
-
-// neuron-range splits of the per-token-tile kernels: enough workgroups for `target` (two per CU
-// for the forward, one for bwdx), at least 2 chunks of 32 neurons per split
+// neuron-range splits of the per-token-tile kernels: enough workgroups for one per CU, at least 2
+// chunks of 32 neurons per split
 int mid_splits(int T, int F, int target) {
   const int gx = (T + 127) / 128;
   int fs = (target + gx - 1) / gx;
@@ -615,7 +495,7 @@ int w_splits(int T, int F) {
 }
 
 struct FusedWs {
-  size_t gemm = 0, v_t = 0, a_t = 0, db_t = 0, part = 0, total = 0;
+  size_t gemm = 0, part = 0, total = 0;
 };
 
 FusedWs fused_layout(int T, int d, int F, int r) {
@@ -623,16 +503,13 @@ FusedWs fused_layout(int T, int d, int F, int r) {
   size_t g = gemm_splitk_bytes(d, 2 * r, T);
   const size_t g2 = gemm_splitk_bytes(d, r, T);
   L.gemm = align256(g > g2 ? g : g2);
-  L.v_t = align256((size_t)r * 2 * F * 2);  // v_dnT [r][F] (fwd) / v_ugT [r][2F] (bwd)
-  L.a_t = align256((size_t)2 * r * T * 2);
-  L.db_t = align256((size_t)r * T * 2);
   const size_t p_fwd = (size_t)mid_splits(T, F, 512) * T * r * 4;
   const size_t p_bx = (size_t)mid_splits(T, F, 256) * T * 2 * r * 4;
   const size_t p_bw = (size_t)w_splits(T, F) * 3 * F * r * 4;
   size_t p = p_fwd > p_bx ? p_fwd : p_bx;
   p = p > p_bw ? p : p_bw;
   L.part = align256(p);
-  L.total = L.gemm + L.v_t + L.a_t + L.db_t + L.part;
+  L.total = L.gemm + L.part;
   return L;
 }
 
@@ -660,8 +537,7 @@ int rte_svd_ffn_fused_fwd(const void* x, int T, int d, int F, int r, const void*
               "svd_ffn_fused: workspace of %zu bytes needed", L.total);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
-  bf16* v_dnT = reinterpret_cast<bf16*>(ws + L.gemm);
-  float* part = reinterpret_cast<float*>(ws + L.gemm + L.v_t + L.a_t + L.db_t);
+  float* part = reinterpret_cast<float*>(ws + L.gemm);
   {
     GemmArgs p;  // a_ug = x @ us_ug : B(n=j, k=dcol) = us_ug[dcol][j]
     p.M = T;
@@ -674,7 +550,6 @@ int rte_svd_ffn_fused_fwd(const void* x, int T, int d, int F, int r, const void*
     p.epi.ldc = 2 * r;
     RTE_TRY(gemm_launch(p, EPI_STORE, st));
   }
-  RTE_TRY(transpose_bf16(static_cast<const bf16*>(v_dn), F, r, r, v_dnT, F, st));
   const int fs = mid_splits(T, F, 512);
   const int nc = F / 32;
   const int cps = (nc + fs - 1) / fs;
@@ -682,10 +557,10 @@ int rte_svd_ffn_fused_fwd(const void* x, int T, int d, int F, int r, const void*
   float* pp = fs > 1 ? part : nullptr;
   if (r == 128)
     hipLaunchKernelGGL(svd_mid_fwd_kernel<128>, grid, dim3(256), 0, st, static_cast<const bf16*>(a_ug),
-                       static_cast<const bf16*>(v_ug), v_dnT, T, F, cps, static_cast<bf16*>(b), pp);
+                       static_cast<const bf16*>(v_ug), static_cast<const bf16*>(v_dn), T, F, cps, static_cast<bf16*>(b), pp);
   else
     hipLaunchKernelGGL(svd_mid_fwd_kernel<64>, grid, dim3(256), 0, st, static_cast<const bf16*>(a_ug),
-                       static_cast<const bf16*>(v_ug), v_dnT, T, F, cps, static_cast<bf16*>(b), pp);
+                       static_cast<const bf16*>(v_ug), static_cast<const bf16*>(v_dn), T, F, cps, static_cast<bf16*>(b), pp);
   RTE_TRY(check_launch("svd_mid_fwd"));
   if (fs > 1) RTE_TRY(split_sum(part, fs, (int64_t)T * r, (int64_t)T * r, b, b, 1, st));
   {
@@ -724,10 +599,7 @@ int rte_svd_ffn_fused_bwd(const void* dy, const void* x, int T, int d, int F, in
               "svd_ffn_fused: workspace of %zu bytes needed", L.total);
   char* ws = static_cast<char*>(workspace);
   void* gws = ws;
-  bf16* v_ugT = reinterpret_cast<bf16*>(ws + L.gemm);
-  bf16* a_ugT = reinterpret_cast<bf16*>(ws + L.gemm + L.v_t);
-  bf16* dbT = reinterpret_cast<bf16*>(ws + L.gemm + L.v_t + L.a_t);
-  float* part = reinterpret_cast<float*>(ws + L.gemm + L.v_t + L.a_t + L.db_t);
+  float* part = reinterpret_cast<float*>(ws + L.gemm);
   {
     GemmArgs p;  // db = dy @ us_dn : B(n=j, k=dcol) = us_dn[dcol][j]
     p.M = T;
@@ -754,7 +626,6 @@ int rte_svd_ffn_fused_bwd(const void* dy, const void* x, int T, int d, int F, in
     p.epi.c_f32 = 1;
     RTE_TRY(gemm_launch(p, EPI_STORE, st, gws, L.gemm));
   }
-  RTE_TRY(transpose_bf16(static_cast<const bf16*>(v_ug), 2 * F, r, r, v_ugT, 2 * F, st));
   {
     const int fs = mid_splits(T, F, 256);
     const int nc = F / 32;
@@ -764,30 +635,29 @@ int rte_svd_ffn_fused_bwd(const void* dy, const void* x, int T, int d, int F, in
     if (r == 128)
       hipLaunchKernelGGL(svd_mid_bwdx_kernel<128>, grid, dim3(256), 0, st, static_cast<const bf16*>(a_ug),
                          static_cast<const bf16*>(db), static_cast<const bf16*>(v_ug),
-                         static_cast<const bf16*>(v_dn), v_ugT, T, F, cps, static_cast<bf16*>(da_ug), pp);
+                         static_cast<const bf16*>(v_dn), T, F, cps, static_cast<bf16*>(da_ug), pp);
     else
       hipLaunchKernelGGL(svd_mid_bwdx_kernel<64>, grid, dim3(256), 0, st, static_cast<const bf16*>(a_ug),
                          static_cast<const bf16*>(db), static_cast<const bf16*>(v_ug),
-                         static_cast<const bf16*>(v_dn), v_ugT, T, F, cps, static_cast<bf16*>(da_ug), pp);
+                         static_cast<const bf16*>(v_dn), T, F, cps, static_cast<bf16*>(da_ug), pp);
     RTE_TRY(check_launch("svd_mid_bwdx"));
     if (fs > 1) RTE_TRY(split_sum(part, fs, (int64_t)T * 2 * r, (int64_t)T * 2 * r, da_ug, da_ug, 1, st));
   }
-  RTE_TRY(transpose_bf16(static_cast<const bf16*>(a_ug), T, 2 * r, 2 * r, a_ugT, T, st));
-  RTE_TRY(transpose_bf16(static_cast<const bf16*>(db), T, r, r, dbT, T, st));
   {
     const int ts = w_splits(T, F);
     const int nt = (T + 31) / 32;
     const int tps = (nt + ts - 1) / ts;
-    dim3 grid(F / 128, ts);
+    dim3 grid(ts, F / 128);
     float* pp = ts > 1 ? part : nullptr;
     if (r == 128)
-      RTE_TRY(launch_bwdw<128>(grid, st, static_cast<const bf16*>(a_ug), static_cast<const bf16*>(db), a_ugT, dbT,
-                               static_cast<const bf16*>(v_ug), static_cast<const bf16*>(v_dn), T, F, tps, dv_ug,
-                               dv_dn, pp));
+      hipLaunchKernelGGL(svd_mid_bwdw_kernel<128>, grid, dim3(256), 0, st, static_cast<const bf16*>(a_ug),
+                         static_cast<const bf16*>(db), static_cast<const bf16*>(v_ug),
+                         static_cast<const bf16*>(v_dn), T, F, tps, dv_ug, dv_dn, pp);
     else
-      RTE_TRY(launch_bwdw<64>(grid, st, static_cast<const bf16*>(a_ug), static_cast<const bf16*>(db), a_ugT, dbT,
-                              static_cast<const bf16*>(v_ug), static_cast<const bf16*>(v_dn), T, F, tps, dv_ug, dv_dn,
-                              pp));
+      hipLaunchKernelGGL(svd_mid_bwdw_kernel<64>, grid, dim3(256), 0, st, static_cast<const bf16*>(a_ug),
+                         static_cast<const bf16*>(db), static_cast<const bf16*>(v_ug),
+                         static_cast<const bf16*>(v_dn), T, F, tps, dv_ug, dv_dn, pp);
+    RTE_TRY(check_launch("svd_mid_bwdw"));
     if (ts > 1) RTE_TRY(split_sum(part, ts, (int64_t)3 * F * r, (int64_t)2 * F * r, dv_ug, dv_dn, 0, st));
   }
   {
