@@ -430,6 +430,8 @@ int rte_grouped_swiglu_fwd(const void* x, int T, int d, const int32_t* offsets, 
     p.epi.c = y_pairs;
     p.epi.ldc = d;
     p.epi.c_rows = pair_of_slot;
+    p.a.extent = (int64_t)P * n * 2;
+    p.b.extent = ((int64_t)(d - 1) * ld_wd + dff) * 2;
     RTE_TRY(gemm_launch(p, EPI_STORE, S(stream)));
   }
   (void)T;
@@ -488,6 +490,8 @@ int rte_grouped_swiglu_bwd(const void* dout, const void* x, int T, int d, const 
     p.epi.c = dx_pairs;
     p.epi.ldc = d;
     p.epi.c_rows = pair_of_slot;
+    p.a.extent = (int64_t)P * 2 * n * 2;
+    p.b.extent = (int64_t)2 * G * n * d * 2;
     RTE_TRY(gemm_launch(p, EPI_STORE, S(stream)));
   }
   RTE_TRY(pool_wgrad(dout, x, T, d, offsets, G, n, P, tok_of_slot, ld_wd, zw, dug, dwug, dwd, w_t, beta, workspace,

@@ -1221,12 +1221,27 @@ bool tile_ok(GemmArgs& p, int epi_kind) {
 
 // Grouped products on the tile kernels: whole 64-k stages of known extent (GROUP_M), or reductions
 // over layout-T rows with at most one gathered operand, in chunks (GROUP_K).
+bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15) == 0; }
+
+// Grouped rows through a weight held in LDS: plain bf16 stores of K 64 or 128.  From 4096 rows on: 64 groups
+// of 512 columns take 7.9 / 8.6 us (K 64 / 128) at 2048 rows where the tiles took 7.0 / 9.0, and 8.0 / 9.1
+// against 8.2 / 10.4 at 4096.
+bool rows_ok(const GemmArgs& p) {
+  const Epilogue& e = p.epi;
+  if ((p.K != 64 && p.K != 128) || p.M < 4096 || p.N < 128 || p.N % 8 != 0) return false;
+  if (p.a_t || p.a.rows || p.a.ilv || p.a.gstride || p.a.growstride || p.a_koff2 || p.b.rows) return false;
+  if (p.b_t && p.b.ilv && p.b.growstride % 64 != 0) return false;  // a group starts on an interleave period
+  return !e.c_f32 && !e.row_scale && !e.resid && !e.c_ilv && !e.c_col_ilv && !e.c_gstride && !e.c_growstride &&
+         e.alpha == 1.0f && e.beta == 0.0f && e.ldc % 8 == 0 && aligned16(e.c);
+}
+
 bool tile_group_ok(GemmArgs& p, int epi_kind, void* ws, size_t ws_bytes) {
   const int64_t lim = (int64_t)1 << 31;
   for (const Operand* o : {&p.a, &p.b})
     if (o->cdiv || o->rdiv || o->extent <= 0 || o->extent >= lim) return false;
   p.a_bytes = (uint32_t)p.a.extent;
   p.b_bytes = (uint32_t)p.b.extent;
+  if (p.mode == MODE_GROUP_M && epi_kind == EPI_STORE) return rows_ok(p);
   if (p.mode == MODE_GROUP_M) {
     if (p.K % 64 != 0 || p.K < kTileMinK || p.a_t || p.a.ilv || p.b.rows || p.a_koff2) return false;
     if (epi_kind == EPI_SWIGLU_FWD) return !p.b_t;
@@ -1234,7 +1249,7 @@ bool tile_group_ok(GemmArgs& p, int epi_kind, void* ws, size_t ws_bytes) {
   }
   if (p.mode != MODE_GROUP_K || epi_kind != EPI_STORE || !p.a_t || !p.b_t || p.K <= 0) return false;
   if (p.a.ilv || p.b.ilv || p.a.gstride || p.b.gstride || p.a.growstride || p.b.growstride) return false;
-  if ((p.a.rows && p.b.rows) || p.M < 64 || p.N < 64 || p.N % 4 != 0 || !ws) return false;
+  if ((p.a.rows && p.b.rows) || p.M < 64 || p.N < 64 || p.N % 8 != 0 || !ws) return false;
   const int chunk = groupk_chunk(p.M, p.N, p.K, p.G);
   if (chunk > kTileGroupChunk || ws_bytes < gemm_groupk_bytes(p.M, p.N, p.K, p.G)) return false;
   p.gk_chunk = chunk;
@@ -1266,7 +1281,6 @@ int launch_tiles(const GemmArgs& p, int epi_kind, hipStream_t stream, int vec, v
 
 bool pow2_or_zero(int v) { return v == 0 || (v > 0 && (v & (v - 1)) == 0); }
 
-bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15) == 0; }
 
 }  // namespace
 

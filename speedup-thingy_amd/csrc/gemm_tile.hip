@@ -619,10 +619,129 @@ int launch_tile(const GemmArgs& p, hipStream_t stream, int vec, int tile) {
   return layouts<128, 128, 2, 2, 64, 2, EPI>(p, stream, vec);
 }
 
+// Grouped rows times a short-k weight (the pools' output and input-gradient pairs): C[row] = A[row] B_g
+// for K = 64 KT, bf16 out, rows optionally scattered.  Bound by writing C (N values per row against K
+// read).  A workgroup keeps 256 columns of one group's weight in LDS and its four waves stream
+// `chunk` rows past it, 32 at a time, with the next rows on their way: no load, barrier or wait of one
+// block of rows stands in front of the next one's stores.  With a tile of 128 x 128 per workgroup each
+// tile paid a load and a store latency in turn (262144 rows of 1024 columns, 537 MB written: K 64 240 us
+// and now 134, K 128 324 us and now 181).  The weight is the product's row operand, so a lane holds one row's
+// columns in fours and 64 columns of 32 rows leave through a 4 KB patch in whole 128-byte lines.
+constexpr int kRowsCols = 256;
+template <int KT, bool BT>
+__global__ void __launch_bounds__(256, KT == 1 ? 3 : 2) gemm_rows_kernel(GemmArgs p, int chunk) {
+  using OpB = TileOperand<kRowsCols, 256, 64, BT>;
+  __shared__ __align__(16) unsigned char slab[KT * OpB::BYTES];
+  __shared__ __align__(16) unsigned char patches[4 * 4096];
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int gy = (p.N + kRowsCols - 1) / kRowsCols;
+  const int lin = (blockIdx.x & ~255) + (blockIdx.x & 7) * 32 + ((blockIdx.x & 255) >> 3);  // as the tiles
+  const int3 f = tile_group(p.goff, p.G, chunk, 0, lin / gy, lane);
+  const int g = f.x;
+  if (g < 0) return;
+  const int n0 = (lin % gy) * kRowsCols;
+  const int mbeg = p.goff[g] + f.y * chunk;
+  const int mend = mbeg + chunk < p.goff[g + 1] ? mbeg + chunk : p.goff[g + 1];
+
+  // layout T leaves the group's k rows (whole interleave periods of 64) to the descriptor
+  const int64_t shift = BT ? (int64_t)g * (p.b.ilv ? p.b.growstride / 2 : p.b.growstride) * p.b.ld : 0;
+  OpB lb;
+  lb.init(p.b, g, n0, p.N, tid, false);
+  const BufferRsrc rb = buffer_rsrc(p.b.ptr + shift, p.b_bytes - (uint32_t)(shift * 2));
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) {
+    const int bo = OpB::advance((int)p.b.ld, p.b.ilv, kt * 64);
+#pragma unroll
+    for (int u = 0; u < OpB::INS; ++u)
+      lds_dma16_buf(rb, slab + kt * OpB::BYTES + wave * 1024 + u * 4096, lb.off[u], bo);
+  }
+  int bof[kRowsCols / 32];
+#pragma unroll
+  for (int j = 0; j < kRowsCols / 32; ++j) bof[j] = OpB::frag_off(0, lane, j, 0);
+
+  bf16x8_v x[KT * 4];
+  auto rows_of = [&](int m) {  // rows past the chunk repeat its last one and are not stored
+    const int r = m + l32 < mend ? m + l32 : mend - 1;
+    const bf16* a = p.a.ptr + (int64_t)r * p.a.ld + 8 * h;
+#pragma unroll
+    for (int k = 0; k < KT * 4; ++k) x[k] = ld_frag16(a + 16 * k);
+  };
+  int m = mbeg + wave * 32;
+  if (m < mend) rows_of(m);
+  wait_vmcnt_lgkm0<0>();
+  wg_barrier();  // the slab is in LDS
+
+  unsigned char* patch = patches + wave * 4096;
+  bf16* c = static_cast<bf16*>(p.epi.c);
+  for (; m < mend; m += 128) {
+    bf16x8_v cur[KT * 4];
+#pragma unroll
+    for (int k = 0; k < KT * 4; ++k) cur[k] = x[k];
+    int64_t at[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = m + i * 8 + (lane >> 3);
+      at[i] = r < mend ? (int64_t)(p.epi.c_rows ? p.epi.c_rows[r] : r) * p.epi.ldc : -1;
+    }
+    if (m + 128 < mend) rows_of(m + 128);
+#pragma unroll
+    for (int j = 0; j < kRowsCols / 64; ++j) {
+      if (n0 + j * 64 >= p.N) break;
+      f32x16_v acc[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[e][r] = 0.0f;
+#pragma unroll
+      for (int k = 0; k < KT * 4; ++k)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const int off = bof[2 * j + e];
+          const unsigned char* w = slab + (k >> 2) * OpB::BYTES + (BT ? off + (k & 3) * 16 * OpB::ROWB : off ^ ((k & 3) * 32));
+          acc[e] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(OpB::frag(w), cur[k], acc[e], 0, 0, 0);
+        }
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<uint2*>(patch + l32 * 128 + (((4 * e + q) ^ (l32 & 7)) << 4) + h * 8) =
+              make_uint2(pack_bf2(acc[e][4 * q], acc[e][4 * q + 1]), pack_bf2(acc[e][4 * q + 2], acc[e][4 * q + 3]));
+      wave_lds_fence();
+      const int ch = lane & 7, col = n0 + j * 64 + ch * 8;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = i * 8 + (lane >> 3);
+        const uint4 v = *reinterpret_cast<const uint4*>(patch + r * 128 + ((ch ^ (r & 7)) << 4));
+        if (at[i] >= 0 && col < p.N) *reinterpret_cast<uint4*>(c + at[i] + col) = v;
+      }
+      wave_lds_fence();
+    }
+  }
+}
+
+int launch_rows(const GemmArgs& p, hipStream_t stream) {
+  // rows per workgroup: 512 unless that leaves fewer than four workgroups per CU
+  const int gy = (p.N + kRowsCols - 1) / kRowsCols;
+  int chunk = 512;
+  while (chunk > 128 && (int64_t)p.M / chunk * gy < 1024) chunk /= 2;
+  const int64_t items = ((int64_t)p.M / chunk + p.G) * gy;
+  const int64_t grid = (items + 255) / 256 * 256;
+  RTE_REQUIRE(grid < ((int64_t)1 << 31), "gemm: too many row chunks");
+  if (p.K == 64)
+    hipLaunchKernelGGL((p.b_t ? gemm_rows_kernel<1, true> : gemm_rows_kernel<1, false>), dim3((unsigned)grid), dim3(256),
+                       0, stream, p, chunk);
+  else
+    hipLaunchKernelGGL((p.b_t ? gemm_rows_kernel<2, true> : gemm_rows_kernel<2, false>), dim3((unsigned)grid), dim3(256),
+                       0, stream, p, chunk);
+  return check_launch("gemm_rows");
+}
+
 }  // namespace
 
 int gemm_tile_group_launch(const GemmArgs& p, int epi_kind, hipStream_t stream, int vec) {
   if (p.mode == MODE_GROUP_M) {
+    if (epi_kind == EPI_STORE) return launch_rows(p, stream);
     if (epi_kind == EPI_SWIGLU_FWD)
       return launch<128, 128, 2, 2, 64, 2, false, false, EPI_SWIGLU_FWD, MODE_GROUP_M>(p, stream, vec);
     return launch<128, 64, 4, 1, 64, 2, false, true, EPI_SWIGLU_BWD, MODE_GROUP_M>(p, stream, vec);
