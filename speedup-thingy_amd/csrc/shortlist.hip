@@ -187,82 +187,69 @@ __global__ void __launch_bounds__(256) shortlist_fwd_kernel(const bf16* __restri
   }
 }
 
-// g[t, :] and dhidden[t] = sum_j g[t, j] W[sl[t, j]].  One wave per token, lanes across
-// d (lane owns 16-byte chunks lane, lane + 64, ...); rows are taken four at a time
-// (220 us for 16384 tokens of 128 rows of 1024; 265 us eight at a time, 330 us by column slab).
-template <int NC2>
+// g[t, :] and dhidden[t] = sum_j g[t, j] W[sl[t, j]].  One wave per token and slab of 128 columns (64
+// ids and g values at a time in its lanes); 16 lanes of 8 columns take a row, the four groups of lanes
+// every fourth row.  The waves of a slab run together on an XCD (dispatch id b runs on XCD b % 8), whose
+// L2 then holds that slab of W: 16384 tokens of 128 rows of 1024, V 8192: 196 us, 226 with whole
+// rows (330 with two columns per lane and one row per load).
 __global__ void __launch_bounds__(256) shortlist_bwd_dh_kernel(
     const float* __restrict__ dloss, const float* __restrict__ dlext, const bf16* __restrict__ W, int d, int V,
     const int32_t* __restrict__ sl, int L, int T, const float* __restrict__ logits, const float* __restrict__ lse,
-    float* __restrict__ g_out, bf16* __restrict__ dh) {
-  extern __shared__ float gl_all[];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int t = blockIdx.x * 4 + wave;
-  const bool active = t < T;
-  float* gl = gl_all + wave * L;
-  if (active) {
-    const float gt = dloss ? dloss[t] : 0.0f;
-    const float l = lse[t];
-    for (int j = lane; j < L; j += 64) {
+    float* __restrict__ g_out, bf16* __restrict__ dh, int nslab) {
+  const int lane = threadIdx.x & 63;
+  const int nb = gridDim.x, xcd = blockIdx.x & 7, q8 = nb >> 3, r8 = nb & 7;
+  const int blk = xcd * q8 + (xcd < r8 ? xcd : r8) + (blockIdx.x >> 3);
+  const int64_t id = (int64_t)blk * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int slab = (int)(id / T), t = (int)(id - (int64_t)slab * T);
+  if (slab >= nslab) return;
+  const float gt = dloss ? dloss[t] : 0.0f;
+  const float ls = lse[t];
+  const int grp = lane >> 4, col = slab * 128 + (lane & 15) * 8;
+  const bool on = dh != nullptr && col < d;
+  const bf16* base = W + (on ? col : 0);
+  float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  for (int j0 = 0; j0 < L; j0 += 64) {
+    const int j = j0 + lane;
+    int vid = -1;
+    float gj = 0.0f;
+    if (j < L) {
       const int64_t o = (int64_t)t * L + j;
-      float gj = dloss ? gt * (__expf(logits[o] - l) - (j == 0 ? 1.0f : 0.0f)) : 0.0f;
+      vid = sl[o];
+      if (dloss) gj = gt * (__expf(logits[o] - ls) - (j == 0 ? 1.0f : 0.0f));
       if (dlext) gj += dlext[o];
-      gl[j] = gj;
-      g_out[o] = gj;
+      if (slab == 0) g_out[o] = gj;
     }
-  }
-  __syncthreads();
-  if (!active || dh == nullptr) return;
-  const int nch = d >> 3;
-  float acc[NC2][8];
-#pragma unroll
-  for (int c = 0; c < NC2; ++c)
-#pragma unroll
-    for (int i = 0; i < 8; ++i) acc[c][i] = 0.0f;
-  const int32_t* srow = sl + (int64_t)t * L;
-  auto load_row = [&](int j, uint4* u) {
-    const int v = srow[j];
-    const bool ok = v >= 0 && v < V;
-    const bf16* row = W + (int64_t)(ok ? v : 0) * d;
-#pragma unroll
-    for (int c = 0; c < NC2; ++c)
-      u[c] = (ok && lane + 64 * c < nch) ? *reinterpret_cast<const uint4*>(row + (lane + 64 * c) * 8)
-                                         : make_uint4(0u, 0u, 0u, 0u);
-  };
-  auto fma_row = [&](float gj, const uint4* u) {
-#pragma unroll
-    for (int c = 0; c < NC2; ++c) {
-      const uint32_t w[4] = {u[c].x, u[c].y, u[c].z, u[c].w};
+    if (vid >= V) vid = -1;
+    if (dh == nullptr) continue;
+    const int n = L - j0 < 64 ? L - j0 : 64;
+    for (int q0 = 0; q0 < n; q0 += 16) {
+      uint4 u[4];
+      float gq[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        acc[c][2 * i] += gj * __uint_as_float(w[i] << 16);
-        acc[c][2 * i + 1] += gj * __uint_as_float(w[i] & 0xffff0000u);
+        const int q = q0 + 4 * i + grp, v = __shfl(vid, q, 64);
+        gq[i] = __shfl(gj, q, 64);
+        u[i] = on && v >= 0 ? *reinterpret_cast<const uint4*>(base + (int64_t)v * d) : make_uint4(0u, 0u, 0u, 0u);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t w[4] = {u[i].x, u[i].y, u[i].z, u[i].w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          acc[2 * k] += gq[i] * __uint_as_float(w[k] << 16);
+          acc[2 * k + 1] += gq[i] * __uint_as_float(w[k] & 0xffff0000u);
+        }
       }
     }
-  };
-  int j = 0;
-  for (; j + 4 <= L; j += 4) {
-    uint4 u[4][NC2];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) load_row(j + q, u[q]);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) fma_row(gl[j + q], u[q]);
-  }
-  for (; j < L; ++j) {
-    uint4 u0[NC2];
-    load_row(j, u0);
-    fma_row(gl[j], u0);
   }
 #pragma unroll
-  for (int c = 0; c < NC2; ++c) {
-    if (lane + 64 * c >= nch) continue;
-    uint4 o;
-    o.x = pack_bf2(acc[c][0], acc[c][1]);
-    o.y = pack_bf2(acc[c][2], acc[c][3]);
-    o.z = pack_bf2(acc[c][4], acc[c][5]);
-    o.w = pack_bf2(acc[c][6], acc[c][7]);
-    *reinterpret_cast<uint4*>(dh + (int64_t)t * d + (lane + 64 * c) * 8) = o;
+  for (int i = 0; i < 8; ++i) {
+    acc[i] += __shfl_xor(acc[i], 16, 64);
+    acc[i] += __shfl_xor(acc[i], 32, 64);
   }
+  if (!on || grp) return;
+  *reinterpret_cast<uint4*>(dh + (int64_t)t * d + col) =
+      make_uint4(pack_bf2(acc[0], acc[1]), pack_bf2(acc[2], acc[3]), pack_bf2(acc[4], acc[5]), pack_bf2(acc[6], acc[7]));
 }
 
 }  // namespace
@@ -327,18 +314,11 @@ int shortlist_bwd(const float* dloss, const float* dlext, const bf16* hidden, co
   }
   float* g = static_cast<float*>(ws);
   const size_t g_bytes = (((size_t)T * L * 4 + 255) / 256) * 256;
-  const size_t lds_g = (size_t)4 * L * sizeof(float);
-  const dim3 grid_t((T + 3) / 4), block(256);
-  const int nc2 = (d / 8 + 63) / 64;
-  if (nc2 <= 1)
-    hipLaunchKernelGGL(shortlist_bwd_dh_kernel<1>, grid_t, block, lds_g, s, dloss, dlext, W, d, V, sl, L, T, logits,
-                       lse, g, dhidden);
-  else if (nc2 <= 2)
-    hipLaunchKernelGGL(shortlist_bwd_dh_kernel<2>, grid_t, block, lds_g, s, dloss, dlext, W, d, V, sl, L, T, logits,
-                       lse, g, dhidden);
-  else
-    hipLaunchKernelGGL(shortlist_bwd_dh_kernel<4>, grid_t, block, lds_g, s, dloss, dlext, W, d, V, sl, L, T, logits,
-                       lse, g, dhidden);
+  const int nslab = dhidden ? (d + 127) / 128 : 1;
+  const int64_t nwg = ((int64_t)T * nslab + 3) / 4;
+  RTE_REQUIRE(nwg < ((int64_t)1 << 31), "shortlist_bwd: too many tokens");
+  hipLaunchKernelGGL(shortlist_bwd_dh_kernel, dim3((unsigned)nwg), dim3(256), 0, s, dloss, dlext, W, d, V, sl, L, T,
+                     logits, lse, g, dhidden, nslab);
   RTE_TRY(check_launch("shortlist_bwd_dhidden"));
   if (!dW) return 0;
   // dW[v] = sum over pairs (t, j) with sl[t, j] = v of g[t, j] hidden[t]: key = sl, row = p / L
