@@ -213,7 +213,8 @@ __device__ __forceinline__ float2 load2(const bf16* p) {
 }
 __device__ __forceinline__ float2 load2(const float* p) { return *reinterpret_cast<const float2*>(p); }
 
-// One wave per chunk of one key's run and slab of 128 columns (two per lane): sum_s w[s] * rows[tok[s]].  A
+// One wave per chunk of one key's run and slab of 128 columns (two per lane): sum_s w[s] * rows[tok[s]], the
+// pairs read a batch ahead of their rows (2.1 M pairs of 1024 columns: 269 us without, 236 us).  A
 // key with a single chunk writes out directly; otherwise the chunk's partial goes to part[item].
 // Dispatch id b runs on XCD b % 8: each XCD takes a contiguous run of (slab, chunk) in slab order.
 template <typename RowT>
@@ -239,17 +240,24 @@ __global__ void __launch_bounds__(256) sort_segsum_kernel(const int32_t* __restr
   const RowT* base = hidden + (on ? col : 0);
   float2 acc = make_float2(0.0f, 0.0f);
   int s = s0;
-  for (; s + 8 <= s1; s += 8) {  // 8 rows in flight
-    int2 pr[8];
-    float2 x[8];
+  if (s + 8 <= s1) {  // 8 rows in flight, the next 8 pairs on their way
+    int2 pr[8], nx[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) pr[j] = pairs[s + j];
+    for (; s + 8 <= s1; s += 8) {
+      float2 x[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = load2(base + (int64_t)pr[j].x * d);
+      for (int j = 0; j < 8; ++j) x[j] = load2(base + (int64_t)pr[j].x * d);
+      const int n = s + 16 <= s1 ? s + 8 : s;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      acc.x += __int_as_float(pr[j].y) * x[j].x;
-      acc.y += __int_as_float(pr[j].y) * x[j].y;
+      for (int j = 0; j < 8; ++j) nx[j] = pairs[n + j];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        acc.x += __int_as_float(pr[j].y) * x[j].x;
+        acc.y += __int_as_float(pr[j].y) * x[j].y;
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) pr[j] = nx[j];
     }
   }
   for (; s < s1; ++s) {
