@@ -18,7 +18,7 @@ def _hip():
     from rte_amd import _lib
 
     if not _lib.device_ready():
-        pytest.fail("HIP backend not ready on this GPU box (library or gfx950 device missing)")
+        pytest.fail("HIP backend not ready (library or gfx950 device missing)")
     yield
 
 
