@@ -44,8 +44,9 @@ int rte_gemm_bf16(const void* a, int64_t lda, int a_t, const int32_t* a_rows,
                   float alpha, float beta, const float* resid, int64_t ld_resid,
                   void* workspace, size_t workspace_bytes, void* stream);
 /* Workspace that lets a dense problem of this shape split its reduction along K
- * (fp32 partials summed in a fixed order: deterministic).  A smaller or NULL
- * workspace only disables the split. */
+ * (fp32 partials summed in a fixed order: deterministic).  The number of splits is
+ * the shape's; a longer workspace changes nothing, a smaller or NULL one only disables the split
+ * (narrow outputs: gives fewer splits). */
 size_t rte_gemm_workspace_bytes(int M, int N, int K);
 
 /* Same, with attention-layout operands: row r -> (r / rdiv)*rs_hi + (r % rdiv)*ld and
@@ -194,7 +195,7 @@ int rte_dense_swiglu_fwd(const void* x, int T, int d, int F, const void* wug, co
 /* dout bf16 [T, d]; writes dug [T, 2F] bf16, dx [T, d] bf16, dwug [2F, d] f32,
  * dwd f32 in the layout of wd (overwritten).  workspace: split-K partials of the dx and weight
  * gradients, max of rte_gemm_workspace_bytes(T, d, 2F), (2F, d, T) and (d, F, T) bytes (fewer
- * bytes: fewer splits). */
+ * bytes: fewer splits or none). */
 int rte_dense_swiglu_bwd(const void* dout, const void* x, int T, int d, int F, const void* wug,
                          const void* wd, int wd_rows, const void* ug, const void* z, void* dug, void* dx,
                          float* dwug, float* dwd, void* workspace, size_t workspace_bytes, void* stream);
@@ -212,7 +213,7 @@ int rte_qkv_rope_fwd(const void* x, const void* wqkv, const float* cos_t, const 
  * by rte_attention_bwd_qkv); dx [B*S, d] bf16; dw [3d, d] f32 (overwritten; NULL: no weight
  * gradient, for callers that form it in another layout).
  * workspace: split-K partials of dx and dw, max of rte_gemm_workspace_bytes(B*S, d, 3d) and
- * (3d, d, B*S) bytes (fewer bytes: fewer splits). */
+ * (3d, d, B*S) bytes (fewer bytes: fewer splits or none). */
 int rte_qkv_rope_bwd(const void* dq, const int64_t* sq, const void* dk, const int64_t* sk, const void* dv,
                      const int64_t* sv, const void* x, const void* wqkv, const float* cos_t,
                      const float* sin_t, int B, int S, int H, int hd, void* dqkv, void* dx, float* dw,

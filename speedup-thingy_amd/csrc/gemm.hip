@@ -1295,8 +1295,10 @@ size_t gemm_splitk_bytes(int M, int N, int K) {
   int splits = K / 128;
   if (splits > kMaxSplits) splits = kMaxSplits;
   if (splits < 2) return 0;
-  const size_t b = (size_t)splits * M * N * sizeof(float);
-  return b < kMaxSplitBytes ? b : kMaxSplitBytes;  // the launch uses fewer splits to fit
+  size_t b = (size_t)splits * M * N * sizeof(float);
+  if (b > kMaxSplitBytes) b = kMaxSplitBytes;  // more than the general kernel's splits ever take
+  const size_t tiles = gemm_tile_split_bytes(M, N, K);
+  return b > tiles ? b : tiles;
 }
 
 int gemm_launch(const GemmArgs& p, int epi_kind, hipStream_t stream, void* ws, size_t ws_bytes) {

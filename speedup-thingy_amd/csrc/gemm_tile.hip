@@ -587,17 +587,16 @@ struct TilePick {
   double us;
 };
 
-TilePick pick_tile(int M, int N, int K, int lo, int hi, size_t max_split_bytes) {
+TilePick pick_tile(int M, int N, int K, int lo, int hi) {
   TilePick best{128, 1, 1e30};
   for (int tile : {256, 128}) {
     const int64_t tiles = (int64_t)((M + tile - 1) / tile) * ((N + tile - 1) / tile);
     const int64_t slots = tile == 256 ? 256 : 512;
     for (int s = lo; s <= hi; ++s) {
       const int kc = ((K + s - 1) / s + 63) / 64 * 64;
-      if (s > 1 && (kc < 256 || (K + kc - 1) / kc != s || K - (s - 1) * kc < kTileMinK)) continue;
+      if (s > 1 && (kc < kTileSplitK || (K + kc - 1) / kc != s || K - (s - 1) * kc < kTileMinK)) continue;
       if (tiles * s > 2 * slots && s > lo) break;  // two rounds of splits never pay
       const double part = 4.0 * M * N * s;
-      if (s > 1 && part > (double)max_split_bytes) break;
       const int64_t wgs = tiles * s, rounds = (wgs + slots - 1) / slots;
       const double per_k = tile == 256 ? 0.0268 : (wgs <= 64 ? 0.0085 : (wgs <= 256 ? 0.0104 : 0.0155));
       const double us = rounds * (per_k * (s > 1 ? kc : K) + 4.5) + (s > 1 ? 2.0 * part / 5e6 + 6.0 : 0.0);
@@ -605,6 +604,21 @@ TilePick pick_tile(int M, int N, int K, int lo, int hi, size_t max_split_bytes) 
     }
   }
   return best;
+}
+
+// Rows of activations: the number of splits sets the order of an element's sum, so it is chosen for
+// the power of two nearest to M (a bucket of rows: from 1 / 1.4142 to 1.4142 times it).
+int row_bucket(int M) {
+  int m2 = 64;
+  while (m2 < (1 << 30) && (double)M > 1.4142 * m2) m2 *= 2;
+  return m2;
+}
+
+// Splits of a product with room for its partials, by the shape alone: the same call gives the same
+// bits whatever ran before it, and so do a sample's rows beside others of their bucket.
+int tile_splits(int M, int N, int K, bool a_t) {
+  if (a_t) return pick_tile(M, N, K, 1, kTileMaxSplits).splits;
+  return K > kTileRowK ? pick_tile(row_bucket(M), N, K, 1, kTileMaxSplits).splits : 1;
 }
 
 template <int EPI>
@@ -751,33 +765,29 @@ int gemm_tile_group_launch(const GemmArgs& p, int epi_kind, hipStream_t stream, 
   return launch<128, 128, 2, 2, 32, 4, true, true, EPI_STORE, MODE_GROUP_K>(p, stream, vec);
 }
 
+size_t gemm_tile_split_bytes(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K < kTileSplitK + kTileMinK) return 0;
+  const int wgrad = tile_splits(M, N, K, true), rows = tile_splits(M, N, K, false);
+  const int most = wgrad > rows ? wgrad : rows;
+  return most > 1 ? (size_t)most * M * N * sizeof(float) : 0;
+}
+
 int gemm_tile_launch(const GemmArgs& p0, int epi_kind, hipStream_t stream, int vec, void* ws, size_t ws_bytes,
                      int* splits) {
   GemmArgs p = p0;
-  const bool may_split = epi_kind == EPI_STORE && ws;
-  int lo = 1, hi = 1;
-  if (may_split && p.a_t) {
-    hi = kTileMaxSplits;
-  } else if (may_split && p.K > kTileRowK) {
-    // Rows of activations: the number of splits sets the order of an element's sum, so it is
-    // chosen for the nearest power of two of M: a sample's rows give the same bits whether a few
-    // other rows share their call or not.
-    int m2 = 64;
-    while ((double)p.M > 1.4142 * m2) m2 *= 2;
-    lo = hi = pick_tile(m2, p.N, p.K, 1, kTileMaxSplits, ws_bytes / 2).splits;
-  }
-  const TilePick pick = pick_tile(p.M, p.N, p.K, lo, hi, ws_bytes);
-  p.splits = pick.splits;
+  p.splits = epi_kind == EPI_STORE && ws ? tile_splits(p.M, p.N, p.K, p.a_t) : 1;
+  if ((size_t)p.splits * p.M * p.N * sizeof(float) > ws_bytes) p.splits = 1;
+  const int tile = pick_tile(p.M, p.N, p.K, p.splits, p.splits).tile;
   if (p.splits > 1) {
     p.k_chunk = ((p.K + p.splits - 1) / p.splits + 63) / 64 * 64;
     p.splitk_ws = static_cast<float*>(ws);
   }
   *splits = p.splits;
   switch (epi_kind) {
-    case EPI_STORE: return launch_tile<EPI_STORE>(p, stream, vec, pick.tile);
-    case EPI_SWIGLU_FWD: return launch_tile<EPI_SWIGLU_FWD>(p, stream, vec, pick.tile);
-    case EPI_SWIGLU_BWD: return launch_tile<EPI_SWIGLU_BWD>(p, stream, vec, pick.tile);
-    default: return launch_tile<EPI_ROPE_QKV>(p, stream, vec, pick.tile);
+    case EPI_STORE: return launch_tile<EPI_STORE>(p, stream, vec, tile);
+    case EPI_SWIGLU_FWD: return launch_tile<EPI_SWIGLU_FWD>(p, stream, vec, tile);
+    case EPI_SWIGLU_BWD: return launch_tile<EPI_SWIGLU_BWD>(p, stream, vec, tile);
+    default: return launch_tile<EPI_ROPE_QKV>(p, stream, vec, tile);
   }
 }
 

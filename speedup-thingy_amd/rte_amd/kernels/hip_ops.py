@@ -61,10 +61,11 @@ _WS: dict[tuple[int, int], torch.Tensor] = {}
 
 
 def workspace(nbytes: int, device: torch.device) -> tuple[int, int]:
-    """(pointer, bytes) of a cached scratch buffer of at least nbytes, one per (device, stream).
+    """(pointer, nbytes) of a cached scratch buffer, one per (device, stream).
 
     Launches on one stream are ordered, so they may share that stream's buffer; work issued
-    on another stream gets its own."""
+    on another stream gets its own.  The buffer may be longer (it grows with its largest user): what a
+    launch does with its workspace depends on its own request alone."""
     if nbytes <= 0:
         return 0, 0
     idx = device.index if device.index is not None else torch.cuda.current_device()
@@ -73,7 +74,7 @@ def workspace(nbytes: int, device: torch.device) -> tuple[int, int]:
     if buf is None or buf.numel() < nbytes:
         buf = torch.empty(((nbytes + 255) // 256) * 256, dtype=torch.uint8, device=device)
         _WS[key] = buf
-    return buf.data_ptr(), buf.numel()
+    return buf.data_ptr(), nbytes
 
 
 def _gemm_ws(M: int, N: int, K: int, device) -> tuple[int, int]:
@@ -2635,7 +2636,7 @@ class SVDFFNFn(torch.autograd.Function):
         else:
             ug, z = wide
             dug = torch.empty((T, 2 * F), dtype=BF16, device=dev)
-            wsp, wsn = _gemm_ws(max(d, F), 2 * r, T, dev)
+            wsp, wsn = _gemm_ws_max(dev, (d, r, T), (F, r, T), (d, 2 * r, T))
             call("rte_svd_ffn_bwd", ptr(dyb), ptr(xb), T, d, F, r, ptr(us_ug), ptr(v_ug), ptr(v_dn), ptr(us_dn),
                  ptr(a_ug), ptr(ug), ptr(z), ptr(b), ptr(db), ptr(dug), ptr(da), ptr(dx), *[ptr(t) for t in g],
                  wsp, wsn, _s())

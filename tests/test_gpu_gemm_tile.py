@@ -75,17 +75,61 @@ def test_epilogue_terms(M, K):
     assert _rel(got, ref) <= 8 * K**0.5 * 2**-24
 
 
+def _fresh():
+    """Every stream's workspace is given back: the next call asks for its own."""
+    from rte_amd.kernels import hip_ops as H
+
+    torch.cuda.synchronize()
+    H._WS.clear()
+
+
 def test_rows_do_not_depend_on_their_company():
     """An activation row's product has the same bits alone, in a small call and in a larger one
-    (unsplit k, and a split k within one power of two of rows)."""
+    (unsplit k: any sizes; a split k: those of one bucket, 1 / 1.4142 to 1.4142 times a power of two),
+    with the workspace each call asks for."""
     from rte_amd.kernels import hip_ops as H
 
     g = torch.Generator().manual_seed(5)
-    for K, sizes in ((512, (64, 1088, 8192)), (2048, (1024, 1088))):
-        a, b = _mat(max(sizes), K, g).to(DEV), _mat(520, K, g).to(DEV)
-        outs = [H.gemm(a[:m].contiguous(), b, out_f32=True)[:64] for m in sizes]
-        for o in outs[1:]:
-            assert torch.equal(o, outs[0])
+    for N, K, sizes in ((520, 512, (64, 1088, 8192)), (520, 2048, (1024, 1088)), (512, 1024, (91, 96, 127, 128, 176)),
+                        (512, 2048, (91, 96, 112, 128, 181)), (512, 2048, (363, 400, 511, 512, 724)),
+                        (512, 8192, (65, 80, 90))):
+        a, b = _mat(max(sizes), K, g).to(DEV), _mat(N, K, g).to(DEV)
+        outs = []
+        for m in sizes:
+            _fresh()
+            outs.append(H.gemm(a[:m].contiguous(), b, out_f32=True)[:min(sizes)])
+        for m, o in zip(sizes, outs):
+            assert torch.equal(o, outs[0]), (N, K, m)
+
+
+@pytest.mark.parametrize("lay,M,N,K", [
+    ("nn", 65, 512, 8192), ("nn", 100, 512, 1024), ("nn", 200, 512, 4096), ("nn", 96, 512, 2048),
+    ("nt", 96, 512, 4096),         # the dense SwiGLU's input gradient of 96 tokens
+    ("tt", 6144, 1024, 16384),     # its weight gradient: partials past 64 MiB
+    ("tt", 1024, 3072, 8192), ("tt", 512, 512, 8192),
+])
+def test_splits_come_from_the_shape(lay, M, N, K):
+    """The same product has the same bits with the workspace it asks for, with a longer one, and
+    through the stream's workspace before and after a larger user has grown it."""
+    from rte_amd import _lib
+    from rte_amd.kernels import hip_ops as H
+
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    at, bt = lay[0] == "t", lay[1] == "t"
+    a = torch.randn((K, M) if at else (M, K), device=DEV, generator=g).to(torch.bfloat16)
+    b = torch.randn((K, N) if bt else (N, K), device=DEV, generator=g).to(torch.bfloat16)
+    need = _lib.load().rte_gemm_workspace_bytes(M, N, K)
+    outs = []
+    for nbytes in (need, need + (512 << 20)):
+        ws, out = torch.empty(nbytes, dtype=torch.uint8, device=DEV), torch.empty(M, N, device=DEV)
+        _lib.call("rte_gemm_bf16", a.data_ptr(), a.shape[1], int(at), None, b.data_ptr(), b.shape[1], int(bt), None,
+                  out.data_ptr(), N, 1, M, N, K, 1.0, 0.0, None, 0, ws.data_ptr(), nbytes, _lib.stream_ptr())
+        outs.append(out)
+    _fresh()
+    outs.append(H.gemm(a, b, a_t=at, b_t=bt, out_f32=True))
+    H.workspace(512 << 20, torch.device(DEV))
+    outs.append(H.gemm(a, b, a_t=at, b_t=bt, out_f32=True))
+    assert all(torch.equal(o, outs[0]) for o in outs[1:])
 
 
 @pytest.mark.parametrize("T,d,F", [(5, 128, 32), (70, 192, 96), (300, 256, 1056), (2048, 512, 2048)])
