@@ -57,19 +57,22 @@ def _s() -> int:
     return _lib.stream_ptr()
 
 
-_WS: dict[tuple[int, int], torch.Tensor] = {}
+_WS: dict[tuple[int, int, int], torch.Tensor] = {}
 
 
 def workspace(nbytes: int, device: torch.device) -> tuple[int, int]:
-    """(pointer, nbytes) of a cached scratch buffer, one per (device, stream).
+    """(pointer, nbytes) of a cached scratch buffer, one per (device, stream, thread).
 
-    Launches on one stream are ordered, so they may share that stream's buffer; work issued
-    on another stream gets its own.  The buffer may be longer (it grows with its largest user): what a
-    launch does with its workspace depends on its own request alone."""
+    One thread's launches on one stream are ordered, so they may share a buffer; work issued on
+    another stream gets its own, and so does another thread on the same stream: an operator of
+    several launches would else find its partial sums overwritten by launches of the other thread that
+    came between (a new thread that takes an ended one's identity takes over its buffers).  The buffer
+    may be longer (it grows with its largest user): what a launch does with its workspace depends on its
+    own request alone."""
     if nbytes <= 0:
         return 0, 0
     idx = device.index if device.index is not None else torch.cuda.current_device()
-    key = (idx, _lib.stream_ptr(idx))
+    key = (idx, _lib.stream_ptr(idx), threading.get_ident())
     buf = _WS.get(key)
     if buf is None or buf.numel() < nbytes:
         buf = torch.empty(((nbytes + 255) // 256) * 256, dtype=torch.uint8, device=device)
