@@ -22,7 +22,12 @@ constexpr int kMaxSortKeys = 32768;   // LDS histogram of the sort: 128 KB
 constexpr int kSlab = 128;            // columns of a wave in the sums
 
 // Pairs per sort block and per partial sum.  Few pairs: more, shorter pieces (latency); many: fewer
-// histograms and partials.
+// histograms and partials.  Whole call in us, blocks of 1024 / 4096 (chunks of 128): 2^18 pairs 49 / 62,
+// 72 / 86 and 245 / 260 over 2048, 8192 and 32768 keys (512, 512 and 1024 columns); 2^19 64 / 77, 86 / 97
+// and 332 / 277; 2^20 97 / 99, 129 / 129 and 509 / 318; 2^21 179 / 164, 236 / 196 and 1020 / 519: the line
+// costs least where it is wrong.  Chunks of 64 / 128 (blocks of 1024, the same keys): 2^16 37.4 / 38.0, 63.9
+// / 64.1, 247 / 246; 2^18 50.6 / 49.1, 71.7 / 71.6, 245 / 245; 2^19 66.5 / 64.3, 94.2 / 86.2, 333 / 332; a
+// tie up to 2^18, 2 - 8% from there.
 int sort_block(int64_t P) { return P > (1 << 19) ? 4096 : 1024; }
 int seg_chunk(int64_t P) { return P >= (1 << 18) ? 128 : 64; }
 
@@ -216,21 +221,26 @@ __device__ __forceinline__ float2 load2(const float* p) { return *reinterpret_ca
 // One wave per chunk of one key's run and slab of 128 columns (two per lane): sum_s w[s] * rows[tok[s]], the
 // pairs read a batch ahead of their rows (2.1 M pairs of 1024 columns: 269 us without, 236 us).  A
 // key with a single chunk writes out directly; otherwise the chunk's partial goes to part[item].
-// Dispatch id b runs on XCD b % 8: each XCD takes a contiguous run of (slab, chunk) in slab order.
+// Dispatch id b runs on XCD b % 8: each XCD takes an equal, contiguous run of the (slab, chunk) pairs
+// that exist, in slab order.  The launch is sized by a bound on the chunks; with the bound shared out
+// instead of chunk_off[V], the XCDs of a sum of few slabs had unequal work (whole call, 8192 keys, 512
+// columns: 2^19 pairs 188 us and now 174, 2^20 146 and 129; 8192 pairs over 2048 keys 36.6 and 35.4).
 template <typename RowT>
 __global__ void __launch_bounds__(256) sort_segsum_kernel(const int32_t* __restrict__ offsets,
                                                           const int32_t* __restrict__ chunk_off,
                                                           const int32_t* __restrict__ item_key, int V, int chunk,
-                                                          int max_items, int nslab, const int2* __restrict__ pairs,
+                                                          int nslab, const int2* __restrict__ pairs,
                                                           const RowT* __restrict__ hidden, int d,
                                                           float* __restrict__ part, float* __restrict__ dW,
                                                           int accumulate) {
   const int lane = threadIdx.x & 63;
-  const int nb = gridDim.x, xcd = blockIdx.x & 7, q8 = nb >> 3, r8 = nb & 7;
-  const int blk = xcd * q8 + (xcd < r8 ? xcd : r8) + (blockIdx.x >> 3);
-  const int64_t id = (int64_t)blk * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int slab = (int)(id / max_items), item = (int)(id - (int64_t)slab * max_items);
-  if (slab >= nslab || item >= chunk_off[V]) return;
+  const int items = chunk_off[V];
+  const int nb = (int)(((int64_t)items * nslab + 3) / 4);  // workgroups with work: at most the grid
+  const int xcd = blockIdx.x & 7, q8 = nb >> 3, r8 = nb & 7, at = blockIdx.x >> 3;
+  if (at >= q8 + (xcd < r8 ? 1 : 0)) return;
+  const int64_t id = (int64_t)(xcd * q8 + (xcd < r8 ? xcd : r8) + at) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int slab = (int)(id / items), item = (int)(id - (int64_t)slab * items);
+  if (slab >= nslab) return;
   const int v = item_key[item];
   const int first = chunk_off[v], nq = chunk_off[v + 1] - first;
   const int s0 = offsets[v] + (item - first) * chunk;
@@ -312,6 +322,14 @@ int set_lds_limit(K kernel, size_t bytes, const char* what) {
   return 0;
 }
 
+// Bound on the chunks of all keys: every chunk holds a pair, and all but each key's last are full.
+// (Without the first, 5000 pairs over 32768 keys of 2048 columns kept 270 MB of partials, 42 now, and
+// started half a million waves with nothing to do: 249 us, 210 now.)
+size_t max_chunks(int64_t P, int V) {
+  const size_t n = ((size_t)P + seg_chunk(P) - 1) / seg_chunk(P) + (size_t)V;
+  return n < (size_t)P ? n : (size_t)P;
+}
+
 struct SegCarve {
   int32_t* hist;
   int32_t* totals;
@@ -324,9 +342,9 @@ struct SegCarve {
 };
 
 SegCarve carve(void* base, int64_t P, int V, int d) {
-  const size_t per = sort_block(P), chunk = seg_chunk(P);
+  const size_t per = sort_block(P);
   const size_t nblk = ((size_t)P + per - 1) / per;
-  const size_t max_items = ((size_t)P + chunk - 1) / chunk + (size_t)V;
+  const size_t max_items = max_chunks(P, V);
   SegCarve c{};
   size_t off = 0;
   auto take = [&](size_t bytes) {
@@ -438,7 +456,7 @@ int segreduce_rows(const int32_t* keys, int64_t P, int V, int row_div, const flo
   hipLaunchKernelGGL(sort_keyscan_kernel, dim3(1), dim3(1024), 0, s, c.totals, V, chunk, c.offsets, c.chunk_off);
   RTE_TRY(check_launch("segment_reduce_keyscan"));
   // the chunk count lives on the device: launch its upper bound, extra waves exit at once
-  const int64_t max_items = ((int64_t)Pi + chunk - 1) / chunk + V;
+  const int64_t max_items = (int64_t)max_chunks(P, V);
   hipLaunchKernelGGL(sort_scatter_kernel, dim3(nblk), block, lds_hist, s, keys, Pi, V, per, row_div, c.hist, c.offsets,
                      w, c.pairs, c.chunk_off, c.item_key);
   RTE_TRY(check_launch("segment_reduce_scatter"));
@@ -447,11 +465,11 @@ int segreduce_rows(const int32_t* keys, int64_t P, int V, int row_div, const flo
   RTE_REQUIRE(nwg < ((int64_t)1 << 31), "segment_reduce: too many partial sums");
   if (rows_f32)
     hipLaunchKernelGGL(sort_segsum_kernel<float>, dim3((unsigned)nwg), block, 0, s, c.offsets, c.chunk_off, c.item_key, V,
-                       chunk, (int)max_items, nslab, c.pairs, static_cast<const float*>(rows), d, c.part, out,
+                       chunk, nslab, c.pairs, static_cast<const float*>(rows), d, c.part, out,
                        accumulate);
   else
     hipLaunchKernelGGL(sort_segsum_kernel<bf16>, dim3((unsigned)nwg), block, 0, s, c.offsets, c.chunk_off, c.item_key, V,
-                       chunk, (int)max_items, nslab, c.pairs, static_cast<const bf16*>(rows), d, c.part, out,
+                       chunk, nslab, c.pairs, static_cast<const bf16*>(rows), d, c.part, out,
                        accumulate);
   RTE_TRY(check_launch("segment_reduce_sum"));
   const int64_t n4 = (int64_t)V * (d / 4);

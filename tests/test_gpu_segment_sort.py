@@ -20,6 +20,7 @@ DEV = "cuda"
     (1 << 19, 32768, 128, 128),      # short sort blocks, the largest key count
     ((1 << 19) + 4097, 1000, 264, 128),  # long sort blocks, a last block of one pair
     (5000, 1025, 2048, 1),           # widest rows, few pairs
+    (5000, 32768, 264, 1),           # far fewer pairs than keys
 ])
 def test_sums_against_float64(P, V, d, div, f32):
     from rte_amd.kernels import hip_ops as H
@@ -49,3 +50,16 @@ def test_sums_against_float64(P, V, d, div, f32):
     acc = torch.ones_like(got)
     H.segment_reduce_rows(kd, V, rd, w=wd, row_div=div, out=acc, accumulate=True)
     assert bool(((acc.cpu().double() - want - 1.0).abs() <= bound + 2.0 ** -23 * (1.0 + want.abs())).all())
+
+
+def test_no_key_in_range():
+    from rte_amd.kernels import hip_ops as H
+
+    keys = torch.full((5000,), -1, device=DEV)
+    keys[::2] = 2000
+    rows = torch.randn(5000, 520, device=DEV)
+    print("segment_reduce without a valid key", flush=True)
+    assert not bool(H.segment_reduce_rows(keys, 2000, rows).any())
+    acc = torch.ones(2000, 520, device=DEV)
+    H.segment_reduce_rows(keys, 2000, rows, out=acc, accumulate=True)
+    assert bool((acc == 1).all())

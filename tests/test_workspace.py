@@ -1,4 +1,5 @@
-"""The cached scratch buffers of hip_ops (CPU: the buffer logic, with a stand-in for the stream)."""
+"""The cached scratch buffers of hip_ops (CPU: the buffer logic, with a stand-in for the stream) and the
+bytes that operators ask for."""
 
 from __future__ import annotations
 
@@ -45,3 +46,11 @@ def test_threads_on_one_stream_have_their_own():
     t.join()
     assert other[0] == other[1] != mine
     assert H.workspace(4096, CPU)[0] == mine
+
+
+def test_segment_sums_ask_for_no_more_partials_than_pairs():
+    ask = _lib.load().rte_segment_reduce_workspace_bytes
+    pairs, cols = 5000, 2048
+    few_keys, many_keys = ask(pairs, 1025, cols), ask(pairs, 32768, cols)
+    sort = 4 * 32768 * (pairs // 1024 + 1 + 3) + 16 * pairs  # histograms, totals, offsets; items and pairs
+    assert few_keys < many_keys <= 4 * pairs * cols + sort + 4096
