@@ -1,12 +1,11 @@
 // Token -> cluster routing, deterministic packing and fixed-order combine.
 //
-//  route_topk  : one wave64 per token; C <= 128: each logit ranked against the row
-//                (readlane broadcast), else k rounds of a wave arg-max over the C
-//                router logits (value descending, index ascending on ties,
-//                NaN above everything as torch.topk does), then softmax over
-//                the k selected logits.  Many tokens (T >= 16384, C <= 128): one lane
-//                per token instead, rows staged through LDS and a sorted top-k kept in
-//                registers by insertion (same order, same softmax summation tree).
+//  route_topk  : the k best of the C router logits (value descending, index ascending on
+//                ties, NaN above everything as torch.topk does), then softmax over them.
+//                Few short rows: one wave64 per token, each logit ranked against the row
+//                (readlane broadcast); else 8 to 64 lanes per token with sorted runs of
+//                64-bit keys in registers, merged over xor partners.  Every form gives the
+//                same ids and the same bits of the weights.
 //  pack        : stable counting sort of the T*k (token, cluster) pairs by
 //                cluster.  Slots inside a cluster follow ascending pair index,
 //                i.e. ascending token, like the nonzero()-based index build of
@@ -28,22 +27,29 @@ __device__ __forceinline__ bool better(float a, int ia, float b, int ib) {
 
 constexpr int kMaxC = 1024;
 
-// Small pools (C <= 64): the rank of element c is the number of elements better than it, counted
-// against every logit of the row broadcast with readlane (no LDS round trips on the critical path);
-// the k best land in LDS at their rank, then lanes j < k take the softmax over them (xor tree).
-template <bool kNaN>
-__device__ __forceinline__ int rank_row(float v, int lane, int C) {
-  int rank = 0;
-  for (int l = 0; l < C; ++l) {
-    const float vj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-    if (kNaN)
-      rank += better(vj, l, v, lane) ? 1 : 0;
-    else
-      rank += (vj > v || (vj == v && l < lane)) ? 1 : 0;
+// Few rows over small pools (C <= 64 PER): the rank of element c is the number of elements better than
+// it, counted against every logit of the row broadcast with readlane (no LDS round trips on the critical
+// path); the k best land in LDS at their rank, then lanes j < k take the softmax over them (xor tree).
+template <int PER, bool kNaN>
+__device__ __forceinline__ void rank_row(const float (&v)[PER], int lane, int C, int (&rank)[PER]) {
+#pragma unroll
+  for (int i = 0; i < PER; ++i) rank[i] = 0;
+#pragma unroll
+  for (int q = 0; q < PER; ++q) {
+    const int n = C - 64 * q < 64 ? C - 64 * q : 64;
+    for (int l = 0; l < n; ++l) {
+      const float vj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[q]), l));
+      const int j = 64 * q + l;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int c = lane + 64 * i;
+        rank[i] += (kNaN ? better(vj, j, v[i], c) : (vj > v[i] || (vj == v[i] && j < c))) ? 1 : 0;
+      }
+    }
   }
-  return rank;
 }
 
+template <int PER>
 __global__ void __launch_bounds__(256) route_topk_rank_kernel(const float* __restrict__ logits, int T, int C, int k,
                                                               int32_t* __restrict__ ids,
                                                               float* __restrict__ weights) {
@@ -53,12 +59,24 @@ __global__ void __launch_bounds__(256) route_topk_rank_kernel(const float* __res
   const int t = blockIdx.x * 4 + wave;
   const bool live = t < T;  // no early exit: every wave reaches the barrier below
   const float* row = logits + (int64_t)(live ? t : 0) * C;
-  const float v = (live && lane < C) ? row[lane] : 0.0f;
-  const int rank = __ballot(v != v) != 0 ? rank_row<true>(v, lane, C) : rank_row<false>(v, lane, C);
-  if (lane < C && rank < k) {
-    sel_v[wave][rank] = v;
-    sel_i[wave][rank] = lane;
+  float v[PER];
+  int rank[PER];
+  bool nan = false;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    v[i] = (live && lane + 64 * i < C) ? row[lane + 64 * i] : 0.0f;
+    nan |= v[i] != v[i];
   }
+  if (__ballot(nan) != 0)
+    rank_row<PER, true>(v, lane, C, rank);
+  else
+    rank_row<PER, false>(v, lane, C, rank);
+#pragma unroll
+  for (int i = 0; i < PER; ++i)
+    if (lane + 64 * i < C && rank[i] < k) {
+      sel_v[wave][rank[i]] = v[i];
+      sel_i[wave][rank[i]] = lane + 64 * i;
+    }
   __syncthreads();
   if (!live) return;
   const float my_v = lane < k ? sel_v[wave][lane] : 0.0f;
@@ -609,26 +627,26 @@ __device__ __forceinline__ void rt_merge(uint64_t (&a)[K], const uint64_t (&b)[K
       }
 }
 
-// Eight lanes per token: each sorts its share of the row (K keys at a time, merged into a running
-// list of K), then the eight lists merge over xor partners, so every lane ends with the row's K best
+// O lanes per token: each sorts its share of the row (K keys at a time, merged into a running
+// list of K), then the O lists merge over xor partners, so every lane ends with the row's K best
 // in order.  Bound by its compare-exchanges, which need no LDS and no rounds over the wave: C 256,
-// k 16, T 16384 took 157 us as 16 rounds of a wave arg-max.  The softmax sums with the xor tree of
-// topk_softmax_store.
-template <int K>
-__global__ void __launch_bounds__(256) route_topk_oct_kernel(const float* __restrict__ logits, int T, int C, int k,
+// k 16, T 16384 took 157 us as 16 rounds of a wave arg-max, and 17.9 in octets.  The softmax sums with
+// the xor tree of topk_softmax_store.
+template <int K, int O>
+__global__ void __launch_bounds__(256) route_topk_lanes_kernel(const float* __restrict__ logits, int T, int C, int k,
                                                              int32_t* __restrict__ ids,
                                                              float* __restrict__ weights) {
-  const int o = threadIdx.x & 7;
-  const int64_t t = (int64_t)blockIdx.x * 32 + (threadIdx.x >> 3);
+  const int o = threadIdx.x & (O - 1);
+  const int64_t t = (int64_t)blockIdx.x * (256 / O) + threadIdx.x / O;
   const float* row = logits + (t < T ? t : T - 1) * (int64_t)C;
-  const int quads = (C + 31) / 32;  // groups of four logits per lane
+  const int quads = (C + 4 * O - 1) / (4 * O);  // groups of four logits per lane
   const bool vec = (C & 3) == 0 && ((uintptr_t)logits & 15) == 0;
   uint64_t best[K];
   for (int q0 = 0; q0 < quads; q0 += K / 4) {
     uint64_t key[K];
 #pragma unroll
     for (int q = 0; q < K / 4; ++q) {
-      const int c = ((q0 + q) * 8 + o) * 4;
+      const int c = ((q0 + q) * O + o) * 4;
       float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
       if (vec && c < C) {
         const float4 x = *reinterpret_cast<const float4*>(row + c);
@@ -650,7 +668,7 @@ __global__ void __launch_bounds__(256) route_topk_oct_kernel(const float* __rest
     }
   }
 #pragma unroll
-  for (int off = 1; off <= 4; off <<= 1) {
+  for (int off = 1; off < O; off <<= 1) {
     uint64_t other[K];
 #pragma unroll
     for (int i = 0; i < K; ++i) other[i] = rt_shfl_xor(best[i], off);
@@ -664,7 +682,7 @@ __global__ void __launch_bounds__(256) route_topk_oct_kernel(const float* __rest
     tv[j] = rt_key_val(best[j]);
     ti[j] = rt_key_idx(best[j]);
   }
-  topk_softmax_store<K>(tv, ti, k, ids + t * k, weights + t * k, o, 8);
+  topk_softmax_store<K>(tv, ti, k, ids + t * k, weights + t * k, o, O);
 }
 
 template <int CB, int K>
@@ -903,25 +921,53 @@ __global__ void __launch_bounds__(256) pack_place_kernel(const int32_t* __restri
 
 }  // namespace
 
+template <int O>
+static int launch_topk(const float* logits, int T, int C, int k, int32_t* ids, float* weights, hipStream_t s) {
+  const dim3 grid((unsigned)(((int64_t)T * O + 255) / 256));
+  if (k <= 4)
+    hipLaunchKernelGGL((route_topk_lanes_kernel<4, O>), grid, dim3(256), 0, s, logits, T, C, k, ids, weights);
+  else if (k <= 8)
+    hipLaunchKernelGGL((route_topk_lanes_kernel<8, O>), grid, dim3(256), 0, s, logits, T, C, k, ids, weights);
+  else
+    hipLaunchKernelGGL((route_topk_lanes_kernel<16, O>), grid, dim3(256), 0, s, logits, T, C, k, ids, weights);
+  return check_launch("route_topk");
+}
+
 int route_topk(const float* logits, int T, int C, int k, int32_t* ids, float* weights, hipStream_t s) {
   RTE_REQUIRE(T >= 0 && C >= 1 && C <= kMaxC, "route_topk: C must be in [1, 1024]");
   RTE_REQUIRE(k >= 1 && k <= 16 && k <= C, "route_topk: k must be in [1, min(16, C)]");
   if (T == 0) return 0;
-  // Few short rows: one wave per row counts ranks with less latency (C 64, k 16: T 1024 5.3 us
-  // against 11.2, T 8192 10.0 against 11.6, T 16384 20 against 13.5; k 8: T 1024 5.4 against 6.1, T
-  // 8192 10.0 against 6.3); everything else in octets (C 256, k 16, T 16384: 17.9 us).
-  if (C <= 64 && T <= (k > 8 ? 8192 : 2048)) {
-    hipLaunchKernelGGL(route_topk_rank_kernel, dim3((T + 3) / 4), dim3(256), 0, s, logits, T, C, k, ids, weights);
+  // A wave per row counting ranks has the least latency over short rows, and costs a wave per row and a
+  // step per logit: k <= 4 up to 32 logits (C 8: T 4096 3.7 us against 3.9, T 8192 4.5 and 3.9; C 64: T 1
+  // 5.0 and 3.7), k <= 8 up to 64 (C 32: T 4096 5.1 and 6.0, T 8192 6.8 and 6.1; C 65: T 1 5.6 and 5.9), k
+  // <= 16 up to 128 (C 64: T 8192 10.0 and 11.1, T 16384 16.1 and 12.1; C 128: T 1024 9.6 and 10.8, T
+  // 4096 13.4 and 11.0).
+  const int64_t work = (int64_t)T * C;
+  const bool rank = k > 8   ? (C <= 64 ? work <= 1 << 19 : C <= 128 && work <= 3 << 17)
+                    : k > 4 ? C <= 64 && work <= 1 << 17
+                            : C <= 32 && work <= 1 << 15;
+  if (rank) {
+    const dim3 grid((unsigned)((T + 3) / 4));
+    if (C <= 64)
+      hipLaunchKernelGGL(route_topk_rank_kernel<1>, grid, dim3(256), 0, s, logits, T, C, k, ids, weights);
+    else
+      hipLaunchKernelGGL(route_topk_rank_kernel<2>, grid, dim3(256), 0, s, logits, T, C, k, ids, weights);
     return check_launch("route_topk");
   }
-  const dim3 grid((unsigned)((T + 31) / 32));
-  if (k <= 4)
-    hipLaunchKernelGGL(route_topk_oct_kernel<4>, grid, dim3(256), 0, s, logits, T, C, k, ids, weights);
-  else if (k <= 8)
-    hipLaunchKernelGGL(route_topk_oct_kernel<8>, grid, dim3(256), 0, s, logits, T, C, k, ids, weights);
-  else
-    hipLaunchKernelGGL(route_topk_oct_kernel<16>, grid, dim3(256), 0, s, logits, T, C, k, ids, weights);
-  return check_launch("route_topk");
+  // Lanes per row: eight give the most rows per second; over long rows, as many as leave a lane 8 logits
+  // (16 for k > 8) while the chip has room for the waves.  In us, 8 lanes / this rule: C 256, k 4, T 1024
+  // 7.5 / 4.7, T 8192 7.8 / 7.8; C 1000, k 1, T 1 19.5 / 5.2, T 4096 20.4 / 9.2, T 8192 26.7 / 13.4; C 1000,
+  // k 16, T 1 31.9 / 11.8, T 8192 40.5 / 30.5 (16 lanes 29.1); C 128, k 8, T 2048 7.2 / 6.3.
+  int lanes = 8;
+  const int share = k > 8 ? 16 : 8;
+  const int64_t room = 256 * (int64_t)(C > 128 ? C : 128);
+  while (lanes < 64 && lanes * share < C && 2 * lanes * (int64_t)T <= room) lanes *= 2;
+  switch (lanes) {
+    case 8: return launch_topk<8>(logits, T, C, k, ids, weights, s);
+    case 16: return launch_topk<16>(logits, T, C, k, ids, weights, s);
+    case 32: return launch_topk<32>(logits, T, C, k, ids, weights, s);
+    default: return launch_topk<64>(logits, T, C, k, ids, weights, s);
+  }
 }
 
 // 256-pair sub-chunks per pack block: one up to 64 Ki pairs, growing to 16 for large P

@@ -28,9 +28,12 @@ def _order(lg, k):
     return key.sort(dim=1, descending=True, stable=True).indices[:, :k].int()
 
 
-@pytest.mark.parametrize("C,k", [(1, 1), (3, 2), (31, 4), (64, 16), (65, 5), (100, 8), (129, 1), (256, 16), (257, 9),
-                                 (1000, 16), (1024, 3)])
-@pytest.mark.parametrize("T", [1, 37, 2050, 16400])
+# widths on both sides of one and two logits per lane and of the lanes-per-row limits, counts on both sides
+# of each of them: C 1000 takes 64, 32, 16 and 8 lanes a row over these T
+@pytest.mark.parametrize("C,k", [(1, 1), (3, 2), (31, 4), (32, 1), (33, 3), (64, 16), (65, 5), (65, 16), (100, 8),
+                                 (128, 12), (129, 1), (129, 16), (256, 16), (257, 9), (512, 8), (1000, 1), (1000, 16),
+                                 (1024, 3)])
+@pytest.mark.parametrize("T", [1, 37, 2050, 5000, 12000, 16400])
 def test_order_and_agreement(C, k, T):
     from rte_amd.kernels import hip_ops as H
 
@@ -49,7 +52,8 @@ def test_order_and_agreement(C, k, T):
                                                                                          equal_nan=True)
 
 
-@pytest.mark.parametrize("T,C,k", [(1, 1, 1), (5, 7, 3), (130, 256, 16), (33, 1025, 16), (9, 4098, 4)])
+@pytest.mark.parametrize("T,C,k", [(1, 1, 1), (5, 7, 3), (35, 63, 5), (70, 64, 16), (18, 65, 16),
+                                   (130, 256, 16), (33, 1025, 16), (9, 4098, 4)])
 def test_route_bwd_rows(T, C, k):
     from rte_amd import _lib
 
