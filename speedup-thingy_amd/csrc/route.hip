@@ -495,24 +495,25 @@ __global__ void __launch_bounds__(256) combine_kernel(const bf16* __restrict__ r
   store8<OutT>(out + (int64_t)t * d + c, acc);
 }
 
-constexpr int kRouteBwdCols = 1024;  // columns of a row held in LDS at a time
-
 // Routing-weight gradient: weights are softmax over the k selected logits, so
 // dlogit_j = w_j * (dw_j - sum_i w_i dw_i); everything else in the row is 0.
-// One wave per token row: lane j holds selection j, the sum runs in j order, and the row leaves
-// whole through LDS (the last j that selected a cluster writes it).  Bound by the row writes; with a
-// thread per logit, each rereading the token's k selections, T 16384, C 256, k 16 took 42 us.
+// G lanes per token row: lane j holds selection j, the sum runs in j order, and the row leaves
+// whole through LDS, COLS columns at a time (the last j that selected a cluster writes it).  Bound by the
+// row writes, for short rows by the waves: T 16384, C 256, k 16 took 35 us with a thread per logit, each
+// rereading the token's k selections, and 12.6 with a wave per row; T 65536, C 32, k 16 20 us with a thread
+// per logit, 36 with a wave per row and 12.1 with 16 lanes.
+template <int G, int COLS>
 __global__ void __launch_bounds__(256) route_bwd_kernel(const int32_t* __restrict__ ids,
                                                         const float* __restrict__ w,
                                                         const float* __restrict__ dw_slot,
                                                         const int32_t* __restrict__ slot_of_pair, int T,
                                                         int C, int k, bf16* __restrict__ dlogits,
                                                         float* __restrict__ dlogits_f32) {
-  __shared__ __align__(16) float row_lds[4][kRouteBwdCols];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t t = (int64_t)blockIdx.x * 4 + wave;
-  float* row = row_lds[wave];
-  if (t >= T) return;  // rows are private to their wave: no workgroup barrier below
+  __shared__ __align__(16) float row_lds[256 / G][COLS];
+  const int lane = threadIdx.x & (G - 1);
+  const int64_t t = (int64_t)blockIdx.x * (256 / G) + threadIdx.x / G;
+  float* row = row_lds[threadIdx.x / G];
+  if (t >= T) return;  // rows are private to their lanes of a wave: no workgroup barrier below
   int id = -1;
   float wv = 0.0f, dv = 0.0f;
   if (lane < k) {
@@ -524,32 +525,32 @@ __global__ void __launch_bounds__(256) route_bwd_kernel(const int32_t* __restric
   float s = 0.0f;
   bool last = lane < k;
   for (int j = 0; j < k; ++j) {
-    s += __shfl(wv, j, 64) * __shfl(dv, j, 64);
-    if (__shfl(id, j, 64) == id && j > lane) last = false;
+    s += __shfl(wv, j, G) * __shfl(dv, j, G);
+    if (__shfl(id, j, G) == id && j > lane) last = false;
   }
   auto fence = [] {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
-  for (int c0 = 0; c0 < C; c0 += kRouteBwdCols) {
-    const int n = C - c0 < kRouteBwdCols ? C - c0 : kRouteBwdCols;
+  for (int c0 = 0; c0 < C; c0 += COLS) {
+    const int n = C - c0 < COLS ? C - c0 : COLS;
     fence();  // the previous columns have left
-    for (int c = lane; c < n; c += 64) row[c] = 0.0f;
+    for (int c = lane; c < n; c += G) row[c] = 0.0f;
     fence();
     if (last && id >= c0 && id < c0 + n) row[id - c0] = wv * (dv - s);
     fence();
     if (dlogits) {
       bf16* d = dlogits + t * C + c0;
       if ((C & 1) == 0 && ((uintptr_t)dlogits & 3) == 0) {
-        for (int c = 2 * lane; c < n; c += 128)
+        for (int c = 2 * lane; c < n; c += 2 * G)
           *reinterpret_cast<uint32_t*>(d + c) = pack_bf2(row[c], row[c + 1]);
       } else {
-        for (int c = lane; c < n; c += 64) d[c] = f2bf(row[c]);
+        for (int c = lane; c < n; c += G) d[c] = f2bf(row[c]);
       }
     }
     if (dlogits_f32)
-      for (int c = lane; c < n; c += 64) dlogits_f32[t * C + c0 + c] = row[c];
+      for (int c = lane; c < n; c += G) dlogits_f32[t * C + c0 + c] = row[c];
   }
 }
 
@@ -1078,8 +1079,14 @@ int route_bwd(const int32_t* ids, const float* w, const float* dw_slot, const in
               int C, int k, bf16* dlogits, float* dlogits_f32, hipStream_t s) {
   RTE_REQUIRE(k >= 1 && k <= 16, "route_bwd: k must be in [1, 16]");
   if (T == 0) return 0;
-  hipLaunchKernelGGL(route_bwd_kernel, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, s, ids, w, dw_slot, slot_of_pair,
-                     T, C, k, dlogits, dlogits_f32);
+  // up to 64 columns 16 lanes hold a row's selections and its stores (C 65, T 65536, k 16: 37.6 us a wave a
+  // row; C 64 13.0 us)
+  if (C <= 64)
+    hipLaunchKernelGGL((route_bwd_kernel<16, 64>), dim3((unsigned)((T + 15) / 16)), dim3(256), 0, s, ids, w, dw_slot,
+                       slot_of_pair, T, C, k, dlogits, dlogits_f32);
+  else
+    hipLaunchKernelGGL((route_bwd_kernel<64, 1024>), dim3((unsigned)((T + 3) / 4)), dim3(256), 0, s, ids, w, dw_slot,
+                       slot_of_pair, T, C, k, dlogits, dlogits_f32);
   return check_launch("route_bwd");
 }
 
