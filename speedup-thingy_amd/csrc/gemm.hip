@@ -1208,8 +1208,19 @@ uint32_t tile_operand(const Operand& o, int64_t rows, int64_t cols) {
   return bytes < ((int64_t)1 << 31) ? (uint32_t)bytes : 0;
 }
 
+// Both operands k-contiguous and K < 256: two to four LDS stages of work, so the loop of the general
+// kernel, which starts on less, is the better one unless the output fills the chip's tiles once or twice
+// over (bf16, tile / general, us: 128 x 1024 x 128 6.6 / 6.0, 8192 x 1024 9.9 / 11.6, 16384 x 1024 15.6 /
+// 15.9, 32768 x 1024 27.2 / 24.7, 32768 x 2048 51 / 42) or is long in fp32 (8192 x 2048 19.2 / 19.2, 16384 x
+// 4096 61 / 66); a residual is always its (1024 x 512 10.7 / 8.0, 32768 x 1024 87 / 68).  K 192 the same.
+bool short_k_tiles(const GemmArgs& p) {
+  const int64_t out = (int64_t)p.M * p.N;
+  return !p.epi.resid && out >= 6 << 20 && (p.epi.c_f32 || out < 24 << 20);
+}
+
 bool tile_ok(GemmArgs& p, int epi_kind) {
   if (p.mode != MODE_DENSE || p.a_koff2 || p.K < kTileMinK || (p.a_t && !p.b_t) || p.splits_forced) return false;
+  if (epi_kind == EPI_STORE && !p.a_t && !p.b_t && p.K < 256 && !short_k_tiles(p)) return false;
   // narrow outputs and few rows over a long reduction: the narrow tiles below, split further
   if (p.N <= 64 || (epi_kind == EPI_STORE && p.M <= 64 && (p.a_t || p.K > kTileRowK))) return false;
   if (!(p.a_t && p.b_t) && p.K % 64 != 0) return false;

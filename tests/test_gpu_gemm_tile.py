@@ -34,9 +34,12 @@ def _mat(rows, cols, g):
 
 
 @pytest.mark.parametrize("lay,M,N,K", [
-    ("nn", 65, 72, 128),        # one k tile per stage, ragged tile edges
+    ("nn", 65, 72, 128),        # the general kernel
+    ("nn", 3079, 2104, 128),    # one k tile per stage, ragged tile edges
     ("nn", 7, 520, 512),        # few rows, short reduction: unsplit
-    ("nn", 129, 136, 192),      # three k tiles in two stages
+    ("nn", 129, 136, 192),      # three k tiles: short k and few outputs, the general kernel
+    ("nn", 3080, 2104, 192),    # the same k over enough outputs: three k tiles in two stages
+    ("nn", 130, 136, 320),      # five k tiles in two stages
     ("nn", 300, 200, 576),
     ("nn", 4096, 4160, 320),    # 256 x 256 tiles with ragged columns, odd tile count
     ("nt", 257, 264, 448),
