@@ -572,34 +572,38 @@ int layouts(const GemmArgs& p, hipStream_t stream, int vec) {
 }
 
 
-// Tile and split choice: the estimated time of each (tile, splits) pair, in us.  Measured on the
-// card (M x N x K from 128 x 512 x 512 to 16384 x 8192 x 16384, all layouts): a 256x256 tile alone
-// on its CU takes 0.0268 us per k (1.25 PFLOP/s over the chip); a 128x128 tile 0.0155 with two on
-// its CU, 0.0104 alone and 0.0085 with most of the chip idle; a round of workgroups costs about 4.5
-// us besides (first loads, output).  Split partials are written and read once at about 5 TB/s, and
-// the reduce launch costs about 6 us.  The estimate is mostly within 15% of the measured times, so
-// it picks the large tile where the grid fills the chip (16384 x 3072 x 1024: 104 us against 118),
-// the small one where it does not (8192 x 512 x 4096: 46 against 81), and splits long reductions
-// into one chip's worth of workgroups (3072 x 1024 x 16384: 111 us at 4 splits; the same product
-// unsplit on 128x128 tiles: 263).
+// Tile and split choice: the estimated time of each (tile, splits) pair, in us.  A 256x256 tile alone on
+// its CU takes 0.0235 us per k; a 128x128 tile 0.0144 with two on its CU, 0.0107 alone and 0.0088 with most
+// of the chip idle (both operands layout T, half as much k per stage: 0.0275, 0.0179, 0.0111 and 0.0099); a
+// round of workgroups 4 us (256) or 2.7 us besides (first loads, output); the launch that adds the partials
+// 3.85, 0.07 for each of them, and their bytes at 1.78 TB/s.  Fitted to 10611 measured (layouts, M, N, K,
+// tile, splits), M and N 65 to 32768, K 256 to 32768: the pick of 1246 shapes takes 0.6% more than their
+// best pair on average and 19% at most (8192 x 128 x 2048: 24.1 us, 20.2 in 3 splits).  The estimate before
+// set that launch at 6 us, counted bytes alone, split from 256 k and went 29% wrong (weight gradients of
+// 200 x 512 x 1024: 12.7 us unsplit, 10.1 in 8; 6000 x 3072 x 256 31 us in large tiles, 24 in small ones;
+// 512 x 128 x 8192 16.0 us in 32 splits, 13.7 in 16).  Large tiles where the grid fills the chip (16384 x
+// 3072 x 1024: 104 us against 118), small ones where it does not (8192 x 512 x 4096: 46 against 81).
 struct TilePick {
   int tile, splits;
   double us;
 };
 
-TilePick pick_tile(int M, int N, int K, int lo, int hi) {
+TilePick pick_tile(int M, int N, int K, bool a_t, int lo, int hi) {
   TilePick best{128, 1, 1e30};
   for (int tile : {256, 128}) {
     const int64_t tiles = (int64_t)((M + tile - 1) / tile) * ((N + tile - 1) / tile);
     const int64_t slots = tile == 256 ? 256 : 512;
     for (int s = lo; s <= hi; ++s) {
       const int kc = ((K + s - 1) / s + 63) / 64 * 64;
-      if (s > 1 && (kc < kTileSplitK || (K + kc - 1) / kc != s || K - (s - 1) * kc < kTileMinK)) continue;
+      if (s > 1 && (kc < kTileMinK || (K + kc - 1) / kc != s || K - (s - 1) * kc < kTileMinK)) continue;
       if (tiles * s > 2 * slots && s > lo) break;  // two rounds of splits never pay
-      const double part = 4.0 * M * N * s;
       const int64_t wgs = tiles * s, rounds = (wgs + slots - 1) / slots;
-      const double per_k = tile == 256 ? 0.0268 : (wgs <= 64 ? 0.0085 : (wgs <= 256 ? 0.0104 : 0.0155));
-      const double us = rounds * (per_k * (s > 1 ? kc : K) + 4.5) + (s > 1 ? 2.0 * part / 5e6 + 6.0 : 0.0);
+      const double per_k = tile == 256  ? (a_t ? 0.0275 : 0.0235)
+                           : wgs <= 64  ? (a_t ? 0.0099 : 0.0088)
+                           : wgs <= 256 ? (a_t ? 0.0111 : 0.0107)
+                                        : (a_t ? 0.0179 : 0.0144);
+      const double round = per_k * (s > 1 ? kc : K) + (tile == 256 ? 4.0 : 2.7);
+      const double us = rounds * round + (s > 1 ? 3.85 + s * (0.07 + 4.0 * M * N / 1.78e6) : 0.0);
       if (us < best.us) best = {tile, s, us};
     }
   }
@@ -617,8 +621,8 @@ int row_bucket(int M) {
 // Splits of a product with room for its partials, by the shape alone: the same call gives the same
 // bits whatever ran before it, and so do a sample's rows beside others of their bucket.
 int tile_splits(int M, int N, int K, bool a_t) {
-  if (a_t) return pick_tile(M, N, K, 1, kTileMaxSplits).splits;
-  return K > kTileRowK ? pick_tile(row_bucket(M), N, K, 1, kTileMaxSplits).splits : 1;
+  if (a_t) return pick_tile(M, N, K, true, 1, kTileMaxSplits).splits;
+  return K > kTileRowK ? pick_tile(row_bucket(M), N, K, false, 1, kTileMaxSplits).splits : 1;
 }
 
 template <int EPI>
@@ -766,7 +770,7 @@ int gemm_tile_group_launch(const GemmArgs& p, int epi_kind, hipStream_t stream, 
 }
 
 size_t gemm_tile_split_bytes(int M, int N, int K) {
-  if (M <= 0 || N <= 0 || K < kTileSplitK + kTileMinK) return 0;
+  if (M <= 0 || N <= 0 || K < 2 * kTileMinK) return 0;
   const int wgrad = tile_splits(M, N, K, true), rows = tile_splits(M, N, K, false);
   const int most = wgrad > rows ? wgrad : rows;
   return most > 1 ? (size_t)most * M * N * sizeof(float) : 0;
@@ -777,7 +781,7 @@ int gemm_tile_launch(const GemmArgs& p0, int epi_kind, hipStream_t stream, int v
   GemmArgs p = p0;
   p.splits = epi_kind == EPI_STORE && ws ? tile_splits(p.M, p.N, p.K, p.a_t) : 1;
   if ((size_t)p.splits * p.M * p.N * sizeof(float) > ws_bytes) p.splits = 1;
-  const int tile = pick_tile(p.M, p.N, p.K, p.splits, p.splits).tile;
+  const int tile = pick_tile(p.M, p.N, p.K, p.a_t, p.splits, p.splits).tile;
   if (p.splits > 1) {
     p.k_chunk = ((p.K + p.splits - 1) / p.splits + 63) / 64 * 64;
     p.splitk_ws = static_cast<float*>(ws);

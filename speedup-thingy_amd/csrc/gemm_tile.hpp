@@ -7,7 +7,6 @@ namespace rte {
 
 constexpr int kTileMinK = 128;      // shortest k range of a workgroup: one tile per LDS stage
 constexpr int kTileMaxSplits = 32;
-constexpr int kTileSplitK = 256;    // shortest k range of a split reduction
 // Products over rows of activations (layout-N A) up to this k are never split, whatever M: a
 // 1024 x 512 x 512 product takes 8.8 us in one launch, 12.8 in four splits and their sum; 128 x 512
 // x 512 8.7 and 8.6.
