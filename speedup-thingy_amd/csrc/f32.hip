@@ -6,8 +6,8 @@
 //    strides: the attention's (sample, head) pairs read straight out of the packed QKV rows), and
 //    grouped products over device-side group offsets: GROUP_M (each group a row range with its own
 //    weight block: routed / banked pools, per-key macro products) and GROUP_K (each group a
-//    reduction range writing its own output block: their weight gradients, one workgroup per
-//    output tile summing its group's rows in order, so results repeat bitwise).  Rows of A and B
+//    reduction range writing its own output block: their weight gradients, summed in row order or,
+//    with a workspace, in chunks whose partials are added in order, so results repeat bitwise).  Rows of A and B
 //    may be gathered through index arrays and scaled per row; rows of C may be scattered.
 //  * causal softmax over score rows (scaled, optional per-(batch) output scale), forward and backward
 //  * SwiGLU over [up | gate] rows, forward and backward
@@ -20,8 +20,8 @@
 // memory, with one barrier per step.  These products are bound by the latency of their k steps and
 // by too few workgroups, not by the matrix cores, so long reductions are cut into k ranges whose
 // fp32 partials a second kernel adds in order: a 32 x 256 x 8192 weight gradient took 4 workgroups
-// 512 serial steps before.  fp32 routed pool layer (T 8192, d 256, 32 x 32, top-4) forward +
-// backward: 1333 -> 540 us (kernel time 1361 -> 327).
+// 512 serial steps before.  fp32 routed pool layer (T 8192, d 256, 32 x 32, top-4) forward + backward:
+// 1335 us with 16-k steps of one buffer and unsplit reductions, 440 now.
 #include "common.hpp"
 
 namespace rte {

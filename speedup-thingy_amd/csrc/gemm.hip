@@ -19,9 +19,6 @@
 #include "gemm_dev.hpp"
 #include "gemm_tile.hpp"
 
-#include <stdio.h>
-#include <stdlib.h>
-
 #include <type_traits>
 
 namespace rte {
@@ -891,10 +888,13 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(GemmArgs p, EpiFlags
 }
 
 // Chunk of a GROUP_K group.  Few output tiles over all groups (fewer than 4 workgroups per CU): about
-// half the mean group size, at least 256 rows, so a long reduction is shared by a few workgroups (the
-// fp32 partials cost less than the serial k steps: 64 groups of 1024 rows, 64 x 512 outputs).  With
-// enough tiles the partials only cost: chunks of two to four mean groups still cut a dominant group (256
-// groups of 1024 rows, 128 x 1024 outputs: the partials' sum alone took 102 us).
+// half the mean group size, at least 256 rows, so a long reduction is shared by a few workgroups.  With
+// enough tiles the partials only cost: chunks of two to four mean groups still cut a dominant group.  Whole
+// backward of the grouped SwiGLU in us, short chunks / long ones, by the tiles of its weight gradients: 128
+// tiles, 32768 rows (d 1024, 16 groups of 64) 108 / 222 and (d 512, 16 of 128) 134 / 256; 512 (d 1024, 64
+// groups), 16384 rows 103 / 78; 1024 (d 1024, 128 groups), 4096 rows 81.0 / 80.7, 32768 182 / 138; 2048 (256
+// groups), 32768 191 / 186.  The line is where long chunks never lose; from 256 tiles on they gain at most
+// sizes.
 int groupk_chunk(int M, int N, int K, int G) {
   const int64_t mean = ((int64_t)K + G - 1) / (G > 0 ? G : 1);
   const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * G;
@@ -961,12 +961,8 @@ int launch_cfg(const GemmArgs& p0, hipStream_t stream, void* ws, size_t ws_bytes
     // at least 128 k per split
     const int tiles = (int)(grid.x * grid.y);
     p.splits = 1;
-    static const int target = [] {  // RTE_SPLIT_WG: workgroup target of the split, for diagnostics
-      const char* v = getenv("RTE_SPLIT_WG");
-      return v && *v && atoi(v) >= 64 ? atoi(v) : 512;
-    }();
     if (EPI == EPI_STORE && ws && tiles < 256 && p.K >= 256) {
-      int splits = (target + tiles - 1) / tiles;
+      int splits = (512 + tiles - 1) / tiles;
       const int max_by_k = p.K / 128;
       if (splits > max_by_k) splits = max_by_k;
       if (splits > kMaxSplits) splits = kMaxSplits;
@@ -1230,13 +1226,15 @@ bool tile_ok(GemmArgs& p, int epi_kind) {
   return p.a_bytes && p.b_bytes;
 }
 
-// Grouped products on the tile kernels: whole 64-k stages of known extent (GROUP_M), or reductions
-// over layout-T rows with at most one gathered operand, in chunks (GROUP_K).
 bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15) == 0; }
 
-// Grouped rows through a weight held in LDS: plain bf16 stores of K 64 or 128.  From 4096 rows on: 64 groups
-// of 512 columns take 7.9 / 8.6 us (K 64 / 128) at 2048 rows where the tiles took 7.0 / 9.0, and 8.0 / 9.1
-// against 8.2 / 10.4 at 4096.
+// Grouped rows through a weight held in LDS: plain bf16 stores of K 64 or 128 (a slab of 256 columns takes
+// 32 KB of LDS per 64 k; from K 192 on it would leave one workgroup per CU).  From 4096 rows on: the whole
+// forward / backward of G groups of 64 neurons (K 64 / 128) in us, tiles first: 4096 rows of 512, G 64 22.1,
+// 21.0 / 51.8, 48.4; of 1024, G 256 39.2, 32.7 / 138, 131; of 256, G 64 17.3, 18.2 / 45.6, 44.9; 16384 rows of
+// 512, G 64 29.4, 25.4 / 73.3, 67.3; of 2048, G 64 65.7, 52.1 / 151, 135.  2048 rows of 256, G 64 14.6, 15.6 /
+// 41.0, 42.9; of 512, G 8 19.2, 20.1 / 52.0, 50.8; wide rows of many groups gain below the line too (1024
+// rows of 1024, G 256 36.5, 30.5 / 134, 127).
 bool rows_ok(const GemmArgs& p) {
   const Epilogue& e = p.epi;
   if ((p.K != 64 && p.K != 128) || p.M < 4096 || p.N < 128 || p.N % 8 != 0) return false;
@@ -1246,6 +1244,8 @@ bool rows_ok(const GemmArgs& p) {
          e.alpha == 1.0f && e.beta == 0.0f && e.ldc % 8 == 0 && aligned16(e.c);
 }
 
+// Grouped products on the tile kernels: whole 64-k stages of known extent (GROUP_M), or reductions
+// over layout-T rows with at most one gathered operand, in chunks (GROUP_K).
 bool tile_group_ok(GemmArgs& p, int epi_kind, void* ws, size_t ws_bytes) {
   const int64_t lim = (int64_t)1 << 31;
   for (const Operand* o : {&p.a, &p.b})
@@ -1256,6 +1256,8 @@ bool tile_group_ok(GemmArgs& p, int epi_kind, void* ws, size_t ws_bytes) {
   if (p.mode == MODE_GROUP_M) {
     if (p.K % 64 != 0 || p.K < kTileMinK || p.a_t || p.a.ilv || p.b.rows || p.a_koff2) return false;
     if (epi_kind == EPI_SWIGLU_FWD) return !p.b_t;
+    // a row's <z, dZ> has to lie in one 64-column output patch: 64 neurons (32 fill half a patch, 96 and
+    // 128 take two: the general kernel)
     return epi_kind == EPI_SWIGLU_BWD && p.b_t && p.N > 32 && p.N <= 64 && !p.b.ilv && !p.b.growstride;
   }
   if (p.mode != MODE_GROUP_K || epi_kind != EPI_STORE || !p.a_t || !p.b_t || p.K <= 0) return false;
@@ -1291,7 +1293,6 @@ int launch_tiles(const GemmArgs& p, int epi_kind, hipStream_t stream, int vec, v
 }
 
 bool pow2_or_zero(int v) { return v == 0 || (v > 0 && (v & (v - 1)) == 0); }
-
 
 }  // namespace
 

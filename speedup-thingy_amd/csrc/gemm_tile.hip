@@ -1,9 +1,12 @@
-// Dense bf16 MFMA GEMM with a register-pipelined main loop (gfx950), fp32 accumulation.
+// bf16 MFMA products with a register-pipelined main loop (gfx950), fp32 accumulation: dense ones, the
+// grouped SwiGLU products (GROUP_M) and the grouped weight gradients (GROUP_K); at the end of the file the
+// products of grouped rows with a short-k weight (gemm_rows_kernel).
 //
 // One workgroup owns a BM x BN output tile; each of its WM x WN waves holds a (BM / WM) x
 // (BN / WN) block in v_mfma_f32_32x32x16_bf16 accumulators.  K advances in tiles of BK through ST
-// LDS stages filled by global_load_lds_dwordx4 (no registers), and the MFMA operands of the next
-// 16-k step are read from LDS while the current step's products run, across tile boundaries too:
+// LDS stages filled through buffer descriptors (buffer_load_dwordx4 ... lds, no registers; loads past
+// an operand's end come back as zeros), and the MFMA operands of the next 16-k step are read from LDS
+// while the current step's products run, across tile boundaries too:
 //
 //   step (kt, last): wait until tile kt + 1 has landed; barrier; refill tile kt's stage with tile
 //                    kt + ST; read the operands of (kt + 1, 0); products of (kt, last)

@@ -1,4 +1,4 @@
-// Dense GEMM on the register-pipelined tile kernels (gemm_tile.hip).
+// Dense and grouped GEMM on the register-pipelined tile kernels (gemm_tile.hip).
 #pragma once
 
 #include "gemm.hpp"

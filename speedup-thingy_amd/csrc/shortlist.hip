@@ -17,7 +17,8 @@
 // fwd     : logits[t, j] = hidden[t] . W[shortlist[t, j]]; 8 lanes per vocab row, 8 rows
 //           per wave pass; lse[t] = logsumexp_j logits[t, j]; loss[t] = lse[t] - logits[t, 0].
 // bwd     : g[t, j] = dloss[t] (softmax_j - [j == 0]) + dlogits_ext[t, j]
-//           dhidden[t] = sum_j g[t, j] W[shortlist[t, j]]             (ascending j)
+//           dhidden[t] = sum_j g[t, j] W[shortlist[t, j]]: four sums over j mod 4, each
+//           in ascending j, added as (0 + 1) + (2 + 3)
 //           dW[v]      = sum over pairs (t, j) with shortlist[t, j] = v of g[t, j] hidden[t]
 //           The pairs are counting-sorted by vocab row (stable: ascending pair index),
 //           each row's run is summed in chunks by one wave per column slab, and chunk
