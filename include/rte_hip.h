@@ -251,7 +251,9 @@ int rte_svd_ffn_fwd(const void* x, int T, int d, int F, int r, const void* us_ug
                     const void* v_dn, const void* us_dn, const float* resid, void* a_ug, void* ug, void* z,
                     void* b, void* y, int y_f32, void* stream);
 /* bwd from dy bf16 [T, d]: scratch db [T, r], dug [T, 2F], da_ug [T, 2r] (bf16); dx [T, d] bf16;
- * weight grads f32 (overwritten) dus_ug [d, 2r], dv_ug [2F, r], dv_dn [F, r], dus_dn [d, r]. */
+ * weight grads f32 (overwritten) dus_ug [d, 2r], dv_ug [2F, r], dv_dn [F, r], dus_dn [d, r].
+ * workspace: split-K partials of the weight gradients, max of rte_gemm_workspace_bytes(d, r, T),
+ * (F, r, T) and (d, 2r, T) bytes (fewer bytes: fewer splits or none). */
 int rte_svd_ffn_bwd(const void* dy, const void* x, int T, int d, int F, int r, const void* us_ug,
                     const void* v_ug, const void* v_dn, const void* us_dn, const void* a_ug, const void* ug,
                     const void* z, const void* b, void* db, void* dug, void* da_ug, void* dx, float* dus_ug,
