@@ -1214,6 +1214,13 @@ bool short_k_tiles(const GemmArgs& p) {
   return !p.epi.resid && out >= 6 << 20 && (p.epi.c_f32 || out < 24 << 20);
 }
 
+// QKV of short k on the general kernel, which starts on less (same k order and bits).  Tile / general in us
+// by rows: K 128 64 8.6 / 7.5, 2048 8.9 / 7.0, 32768 21.1 / 16.2; K 256 16 6.3 / 8.2, 128 9.2 / 7.7, 4096 10.5 /
+// 10.0, 32768 33.6 / 33.4; K 512 64 10.6 / 11.9, 128 10.6 / 9.9, 1024 11.2 / 10.8, 2048 12.1 / 12.8.
+bool short_k_qkv(const GemmArgs& p) {
+  return p.K <= 256 ? p.M >= 64 : p.K <= 512 && p.M >= 128 && p.M <= 1024;
+}
+
 bool tile_ok(GemmArgs& p, int epi_kind) {
   if (p.mode != MODE_DENSE || p.a_koff2 || p.K < kTileMinK || (p.a_t && !p.b_t) || p.splits_forced) return false;
   if (epi_kind == EPI_STORE && !p.a_t && !p.b_t && p.K < 256 && !short_k_tiles(p)) return false;
@@ -1435,7 +1442,7 @@ int gemm_launch(const GemmArgs& p, int epi_kind, hipStream_t stream, void* ws, s
         ps.splits_forced = 1;
         return gemm_launch(ps, EPI_STORE, stream, ws, ws_bytes);
       }
-      if (tiles) return launch_tiles(q, epi_kind, stream, 1, nullptr, 0);
+      if (tiles && !short_k_qkv(p)) return launch_tiles(q, epi_kind, stream, 1, nullptr, 0);
       if (dl_ok(p)) return launch_dl<EPI_ROPE_QKV>(p, stream, ws, ws_bytes, 1);
       return launch_cfg<128, 128, 64, 2, 2, false, false, EPI_ROPE_QKV>(p, stream, ws, ws_bytes, 1);
     default:

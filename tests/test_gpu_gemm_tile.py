@@ -135,6 +135,35 @@ def test_splits_come_from_the_shape(lay, M, N, K):
     assert all(torch.equal(o, outs[0]) for o in outs[1:])
 
 
+@pytest.mark.parametrize("d,hd,batches", [
+    (128, 32, (1, 3, 40)), (256, 64, (1, 2, 17)),  # 33 rows on tiles, more on the general kernel
+    (512, 64, (1, 4, 16, 40)),                     # tiles, general, general, tiles
+])
+def test_qkv_rope_by_rows(d, hd, batches):
+    """QKV + RoPE of short k against float64, and a sample's rows the same bits in every batch."""
+    from rte_amd import _lib
+
+    g = torch.Generator().manual_seed(d)
+    S, H = 33, d // hd
+    x, w = _mat(max(batches) * S, d, g), _mat(3 * d, d, g)
+    ang = torch.rand(S, hd // 2, generator=g).repeat_interleave(2, dim=1) * 6.0
+    cos, sin = ang.cos().contiguous(), ang.sin().contiguous()
+    xd, wd, cd, sd = (t.to(DEV) for t in (x, w, cos, sin))
+    firsts = []
+    for B in batches:
+        out = torch.empty(3, B, H, S, hd, device=DEV, dtype=torch.bfloat16)
+        need = _lib.load().rte_gemm_workspace_bytes(B * S, 3 * d, d)
+        ws = torch.empty(max(need, 16), dtype=torch.uint8, device=DEV)
+        _lib.call("rte_qkv_rope_fwd", xd.data_ptr(), wd.data_ptr(), cd.data_ptr(), sd.data_ptr(), B, S, H, hd,
+                  out[0].data_ptr(), out[1].data_ptr(), out[2].data_ptr(), ws.data_ptr(), need, _lib.stream_ptr())
+        firsts.append(out[:, 0])
+        y = (x[:B * S].double() @ w.double().t()).view(B, S, 3, H, hd).permute(2, 0, 3, 1, 4)
+        turned = torch.stack([-y[..., 1::2], y[..., 0::2]], dim=-1).flatten(-2)
+        ref = torch.cat([y[:2] * cos.double() + turned[:2] * sin.double(), y[2:]])
+        assert _rel(out, ref) <= 2**-9
+    assert all(torch.equal(f, firsts[0]) for f in firsts[1:])
+
+
 @pytest.mark.parametrize("T,d,F", [(5, 128, 32), (70, 192, 96), (300, 256, 1056), (2048, 512, 2048)])
 def test_dense_swiglu(T, d, F):
     from rte_amd.kernels import hip_ops as H
