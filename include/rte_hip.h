@@ -203,8 +203,8 @@ int rte_dense_swiglu_bwd(const void* dout, const void* x, int T, int d, int F, c
 /* ---- fused QKV projection + interleaved RoPE (rte/layers.py:53-75, rte/kernels/reference.py:20-37) ----
  * x [B*S, d] bf16, wqkv [3d, d] bf16 (nn.Linear(d, 3d).weight), cos/sin [S, hd] f32.
  * q, k, v written as contiguous [B, H, S, hd] bf16.  workspace (optional, see
- * rte_gemm_workspace_bytes(B*S, 3d, d)): with few output tiles (short batches) the reduction is
- * split, the partials added in split order and rotated by the split-K reduce. */
+ * rte_gemm_workspace_bytes(B*S, 3d, d)): with few output tiles (short batches) a reduction
+ * over more than 512 k is split, the partials added in split order and rotated by the split-K reduce. */
 int rte_qkv_rope_fwd(const void* x, const void* wqkv, const float* cos_t, const float* sin_t, int B, int S,
                      int H, int hd, void* q, void* k, void* v, void* workspace, size_t workspace_bytes,
                      void* stream);
